@@ -100,6 +100,41 @@ def test_decode_matches_oracle(ctx, dd, frames):
     model.free()
 
 
+@pytest.mark.parametrize("frames", [20, 36, 72])
+def test_long_decode_tiles(ctx, frames):
+    """The residual units and the head take larger tiles from 18, 35 and 69 frames on
+    (32, 64/128 and 256 channels). The decoder is causal with under 20 frames of
+    history, so a long decode starts like the oracle's decode of its first 4 frames and
+    ends like a decode of its last 20 (small tiles but for the 32 channels)."""
+    print(f"vae long decode frames {frames}", flush=True)
+    cfg, model, eng, lat, o = engine_case(ctx, 2048, frames, 0x5EED0530)
+    wave = eng.decode_latents(lat)[1]
+    assert rel_l2(wave[:4 * 1920], o.decode(lat[:4 * 64])) < 1e-3
+    tail = eng.decode_latents(lat[-20 * 64:])[1]
+    assert rel_l2(wave[-1920:], tail[-1920:]) < 1e-5
+    eng.close()
+    model.free()
+
+
+def test_decode_large_snake_arguments(ctx):
+    """Snake arguments past the reduced-range sine (|a x| >= 32768): with alphas of
+    60000 the term sin(a x)^2 / a is below 2e-5, so the wave has to match the oracle
+    whatever the sine of so large an argument rounds to."""
+    cfg = synth.audiovae_config(decoder_dim=256)
+    m = synth.build_audiovae(cfg, seed=0x5EED0540)
+    for t in m.tensors:
+        if t.name.endswith("alpha"):
+            m.data[t.offset:t.offset + t.nbytes].view(np.float16)[::3] = 60000.0
+    model = Model(ctx, m.data, m.tensors)
+    eng = AudioVaeEngine(ctx, model, cfg, strict_geometry=False)
+    lat = 4.0 * synth.normal_f32(8 * 64, 0x5EED0541)
+    want = voxref.AudioVae(m.data, {t.name: t for t in m.tensors}, cfg).decode(lat)
+    wave = eng.decode_latents(lat)[1]
+    assert np.isfinite(wave).all() and rel_l2(wave, want) < 1e-3
+    eng.close()
+    model.free()
+
+
 def test_decode_errors(ctx):
     cfg, model, eng, lat, o = engine_case(ctx, 256, 4, 0x5EED0520)
     for bad, code in ((lat[:63], "VX_ERR_SHAPE"), (lat[:128], "VX_ERR_SHAPE"),

@@ -6,12 +6,13 @@
 //   model.0   depthwise k=7 causal conv                  k_vae_dwconv_fm
 //   model.1   1x1 conv latent -> decoder_dim             k_vae_linear_fm (K = latent)
 //   6 stages  scale/bias + snake + ConvTranspose1d(k=2s, stride s):
-//               [pre(x[j]) | pre(x[j-1])] rows           k_vae_convt_input_fm
-//               one GEMM, N = s * Cout, K = 2 Cin        k_gemm (repacked weights)
+//               P = pre(x) behind a zero row             k_vae_pre_fm, or the last unit before
+//               one GEMM over rows [P[j-1] | P[j]],
+//               N = s * Cout, K = 2 Cin                  k_gemm (repacked weights)
 //             3 residual units (dilation 1, 3, 9):
-//               snake -> depthwise k=7 dilated -> snake  k_vae_dwconv_fm
-//               x += 1x1 conv + bias                     k_gemm residual (or k_vae_linear_fm)
-//               (32 and 64 channels: both in one pass, k_vae_resunit_fm)
+//               32 to 256 channels: one pass             k_vae_unit
+//               else snake -> depthwise k=7 -> snake     k_vae_dwconv_fm
+//               and x += 1x1 conv + bias                 k_gemm residual (or k_vae_linear_fm)
 //   head      snake -> conv k=7 to one channel -> tanh   k_vae_head_fm
 // Row j of the transposed convolution's output phases r = 0..s-1 is output time
 // s j + r, so the GEMM's [L][s Cout] output is the frame-major [s L][Cout] output.
@@ -32,15 +33,20 @@ constexpr uint32_t kSrBuckets = 4;   // DECODER_SR_BUCKETS
 
 struct Res {
     const __half *a1 = nullptr, *dw_w = nullptr, *dw_b = nullptr, *a2 = nullptr, *pw_w = nullptr, *pw_b = nullptr;
+    float *p = nullptr;        // k_vae_unit's parameters and weight, where the width has it
+    __half *w = nullptr;
     uint32_t dilation = 1;
 };
 struct Stage {
     const __half *scale = nullptr, *bias = nullptr, *alpha = nullptr;   // scale/bias rows of the bucket
+    float *pre = nullptr;      // the same as f32 [4][Cin] (launch_vae_repack_pre)
     __half *ct_w = nullptr;    // [s Cout][2 Cin]
     float *ct_b = nullptr;     // [s Cout]
     uint32_t stride = 1, cin = 0, cout = 0;
     Res res[3];
 };
+
+inline uint64_t up256(uint64_t n) { return (n + 255u) / 256u * 256u; }
 
 inline float *F(vx_buf *b) { return static_cast<float *>(b->ptr); }
 
@@ -53,7 +59,7 @@ struct vx_audiovae {
     const __half *m0_w = nullptr, *m0_b = nullptr, *m1_w = nullptr, *m1_b = nullptr;
     const __half *head_alpha = nullptr, *head_w = nullptr, *head_b = nullptr;
     Stage st[kStages];
-    vx_buf *arena = nullptr;               // repacked transposed-conv weights and biases
+    vx_buf *arena = nullptr;               // repacked weights and parameters
     vx_buf *cur = nullptr, *tmp = nullptr, *x2 = nullptr, *io = nullptr, *wave = nullptr;
     uint64_t act_cap = 0, tmp_cap = 0, x2_cap = 0, io_cap = 0, wave_cap = 0;
 };
@@ -186,8 +192,12 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
         return fail(VX_ERR_UNSUPPORTED, "AudioVAE decoder activation exceeds the 32-bit index range");
     VX_CHECK(grow(ctx, &e->cur, &e->act_cap, act));
     VX_CHECK(grow(ctx, &e->tmp, &e->tmp_cap, act));
-    VX_CHECK(grow(ctx, &e->x2, &e->x2_cap, x2_max));
-    float *cur = F(e->cur), *tmp = F(e->tmp);
+    // P of every stage starts behind decoder_dim floats of zeros (its row -1).
+    const uint64_t x2_cap = e->x2_cap;
+    VX_CHECK(grow(ctx, &e->x2, &e->x2_cap, c.decoder_dim + x2_max / 2u));
+    if (e->x2_cap != x2_cap) VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(F(e->x2)), 0u, c.decoder_dim));
+    float *cur = F(e->cur), *tmp = F(e->tmp), *const P = F(e->x2) + c.decoder_dim;
+    bool have_pre = false;   // P holds this stage's input already
     uint32_t len = frames, ch = c.latent_dim;
     {
         ProfSpan sp(ctx, "audiovae.stem");
@@ -209,38 +219,29 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
         const Stage &S = e->st[i];
         {
             ProfSpan sp(ctx, "audiovae.upsample");
-            VaeConvtInArgs a;
-            a.x = cur;
-            a.x2 = F(e->x2);
-            a.scale = S.scale;
-            a.bias = S.bias;
-            a.alpha = S.alpha;
-            a.channels = ch;
-            a.length = len;
-            VX_CHECK(launch_vae_convt_input_fm(s, a));
-            VX_CHECK(linear(ctx, F(e->x2), 2u * ch, S.ct_w, nullptr, S.ct_b, tmp, S.stride * S.cout, len,
+            if (!have_pre) VX_CHECK(launch_vae_pre_fm(s, cur, P, S.pre, ch, len));
+            VX_CHECK(linear(ctx, P - ch, ch, S.ct_w, nullptr, S.ct_b, tmp, S.stride * S.cout, len,
                             S.stride * S.cout, 2u * ch, false));
         }
         std::swap(cur, tmp);
         len *= S.stride;
         ch = S.cout;
+        have_pre = false;
         for (const Res &R : S.res) {
             ProfSpan sp(ctx, "audiovae.residual");
-            VaeResUnitArgs u;
-            u.x = cur;
-            u.y = tmp;
-            u.a1 = R.a1;
-            u.dw = R.dw_w;
-            u.db = R.dw_b;
-            u.a2 = R.a2;
-            u.pw = R.pw_w;
-            u.pb = R.pw_b;
-            u.channels = ch;
-            u.length = len;
-            u.dilation = R.dilation;
-            if (vae_resunit_eligible(u)) {
-                VX_CHECK(launch_vae_resunit_fm(s, u));
-                std::swap(cur, tmp);
+            if (R.p) {
+                VaeUnitArgs u;
+                u.x = cur;
+                u.p = R.p;
+                u.w = R.w;
+                u.channels = ch;
+                u.length = len;
+                u.dilation = R.dilation;
+                have_pre = &R == &S.res[2] && i + 1 < kStages;
+                u.pre = have_pre ? e->st[i + 1].pre : nullptr;
+                u.y = have_pre ? P : tmp;
+                VX_CHECK(launch_vae_unit(s, u));
+                if (!have_pre) std::swap(cur, tmp);
                 continue;
             }
             VaeDwArgs d;
@@ -337,7 +338,8 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
     uint32_t din = c.decoder_dim;
     for (uint32_t i = 0; i < kStages; ++i) {
         const uint32_t s = c.decoder_rates[i], dout = din / 2u;
-        arena += ((uint64_t)s * dout * 2u * din * 2u + 255u) / 256u * 256u + ((uint64_t)s * dout * 4u + 255u) / 256u * 256u;
+        arena += up256((uint64_t)s * dout * 2u * din * 2u) + up256((uint64_t)s * dout * 4u) + up256(din * 16u);
+        if (vae_unit_channels(dout)) arena += 3u * (up256(dout * 52u) + up256((uint64_t)dout * dout * 2u));
         din = dout;
     }
     if ((st = vx_alloc(ctx, arena, &e->arena))) return bail(st);
@@ -367,10 +369,14 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
             (st = conv(model, p + ".block.1", din, dout, 2u * s, 1, true, &ctw, &ctb)))
             return bail(st);
         S.ct_w = reinterpret_cast<__half *>(cur);
-        cur += ((uint64_t)s * dout * 2u * din * 2u + 255u) / 256u * 256u;
+        cur += up256((uint64_t)s * dout * 2u * din * 2u);
         S.ct_b = reinterpret_cast<float *>(cur);
-        cur += ((uint64_t)s * dout * 4u + 255u) / 256u * 256u;
-        if ((st = launch_vae_repack_convt(ctx->stream, ctw, ctb, din, dout, s, S.ct_w, S.ct_b))) return bail(st);
+        cur += up256((uint64_t)s * dout * 4u);
+        S.pre = reinterpret_cast<float *>(cur);
+        cur += up256(din * 16u);
+        if ((st = launch_vae_repack_convt(ctx->stream, ctw, ctb, din, dout, s, S.ct_w, S.ct_b)) ||
+            (st = launch_vae_repack_pre(ctx->stream, S.scale, S.bias, S.alpha, din, S.pre)))
+            return bail(st);
         static const uint32_t dil[3] = {1, 3, 9};
         for (uint32_t r = 0; r < 3; ++r) {
             Res &R = S.res[r];
@@ -380,6 +386,13 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
                 (st = conv(model, q + ".1", dout, dout, 7, dout, false, &R.dw_w, &R.dw_b)) ||
                 (st = alpha(model, q + ".2.alpha", dout, &R.a2)) ||
                 (st = conv(model, q + ".3", dout, dout, 1, 1, false, &R.pw_w, &R.pw_b)))
+                return bail(st);
+            if (!vae_unit_channels(dout)) continue;
+            R.p = reinterpret_cast<float *>(cur);
+            cur += up256(dout * 52u);
+            R.w = reinterpret_cast<__half *>(cur);
+            cur += up256((uint64_t)dout * dout * 2u);
+            if ((st = launch_vae_repack_unit(ctx->stream, R.a1, R.dw_w, R.dw_b, R.a2, R.pw_w, R.pw_b, dout, R.p, R.w)))
                 return bail(st);
         }
         din = dout;

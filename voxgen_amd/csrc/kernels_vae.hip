@@ -8,7 +8,7 @@
 //    and the transposed convolutions are GEMMs on MFMA (k_gemm) and the
 //    elementwise work (scale/bias, snake) is fused into the passes around them.
 // Snake: x + sin(a x)^2 / (a + 1e-9) (vae_snake.comp:13-16).
-#include "vx_internal.h"
+#include "vae_dev.h"
 
 namespace vx {
 namespace {
@@ -24,12 +24,21 @@ __device__ __forceinline__ float snake(float x, float a) {
     const float s = sinf(a * x);
     return x + (s * s) / (a + 1e-9f);
 }
-// The decode engine's snake with the channel's 1 / (a + 1e-9) computed once.
-__device__ __forceinline__ float snake_inv(float a) { return 1.0f / (a + 1e-9f); }
-// (The native __sinf measured no faster here: 0.72 against 0.69 ms per decode.)
-__device__ __forceinline__ float snake_fm(float x, float a, float inv) {
-    const float s = sinf(a * x);
-    return fmaf(s * s, inv, x);
+// The decode engine's snake with the channel's 1 / (a + 1e-9) computed once:
+// x + sin(ax)^2 inv, ax = a x inside sin_sq's range.
+__device__ __forceinline__ float snake_fm(float x, float ax, float inv) { return fmaf(sin_sq(ax), inv, x); }
+__device__ __forceinline__ float snake_any(float x, float ax, float inv) { return fmaf(sin_sq_any(ax), inv, x); }
+
+// Lane exchanges inside a row of 16 lanes (gfx9 DPP controls).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+// Sum over each 8 consecutive lanes: quad swaps, then the half-row mirror.
+__device__ __forceinline__ float sum8(float v) {
+    v += dpp<0xb1>(v);   // quad_perm [1,0,3,2]
+    v += dpp<0x4e>(v);   // quad_perm [2,3,0,1]
+    return v + dpp<0x141>(v);   // row_half_mirror
 }
 
 // ------------------------------------------------------------ channel-major
@@ -152,122 +161,102 @@ __global__ __launch_bounds__(256) void k_vae_dwconv_tiled_fm(VaeDwArgs a, uint32
     float wk[KMAX];
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) wk[k] = cval && (uint32_t)k < a.kernel ? hf(a.w[c * a.kernel + k]) : 0.f;
+    float big = 0.f;
 #pragma unroll
     for (uint32_t i = 0; i < NS; ++i) {
         const uint32_t idx = tid + 256u * i;
-        if (idx < n_st) xs[idx] = a.alpha_in ? snake_fm(xv[i], ain, iin) : xv[i];
+        big = fmaxf(big, fabsf(ain * xv[i]));
+        if (idx < n_st) xs[idx] = a.alpha_in ? snake_fm(xv[i], ain * xv[i], iin) : xv[i];
+    }
+    if (a.alpha_in && any_large(big)) {
+#pragma unroll 1
+        for (uint32_t idx = tid; idx < n_st; idx += 256u) {
+            const int ti = (int)(t0 + (idx >> cb_shift)) - (int)halo;
+            if (!cval || ti < 0 || (uint32_t)ti >= a.length) continue;
+            const float v = a.x[(size_t)ti * C + c];
+            xs[idx] = snake_any(v, ain * v, iin);
+        }
     }
     __syncthreads();
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; ++i) {   // TB * CB = 2048 outputs, 8 per thread
-        const uint32_t r = (tid + 256u * i) >> cb_shift, t = t0 + r;
-        if (t >= a.length || !cval) continue;
+    auto conv = [&](uint32_t r) {
         float sum = bias;
 #pragma unroll
         for (int k = 0; k < KMAX; ++k)
             if ((uint32_t)k < a.kernel) sum += xs[((r + k * a.dilation) << cb_shift) + cc] * wk[k];
-        if (a.alpha_out) sum = snake_fm(sum, aout, iout);
-        a.y[(size_t)t * C + c] = sum;
+        return sum;
+    };
+    big = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i) {   // TB * CB = 2048 outputs, 8 per thread
+        const uint32_t r = (tid + 256u * i) >> cb_shift, t = t0 + r;
+        if (t >= a.length || !cval) continue;
+        const float sum = conv(r);
+        big = fmaxf(big, fabsf(aout * sum));
+        a.y[(size_t)t * C + c] = a.alpha_out ? snake_fm(sum, aout * sum, iout) : sum;
+    }
+    if (a.alpha_out && any_large(big)) {
+#pragma unroll 1
+        for (uint32_t i = 0; i < 8u; ++i) {
+            const uint32_t r = (tid + 256u * i) >> cb_shift, t = t0 + r;
+            if (t >= a.length || !cval) continue;
+            const float sum = conv(r);
+            a.y[(size_t)t * C + c] = snake_any(sum, aout * sum, iout);
+        }
     }
 }
 
-// A residual unit of a narrow stage (C = 32 or 64 channels) in one pass: the
-// workgroup stages snake_a1(x) for TB = 4096 / C rows and their causal halo
-// (6 d rows) in LDS, computes the depthwise conv and snake_a2 into a second LDS
-// tile, then the 1x1 conv with each thread's weight row in registers (the tile's
-// row read as float4 broadcasts) plus bias and the residual x. Two launches and a
-// round trip of the intermediate through HBM become one; every staging load is
-// issued before the first is used. (At 128 channels the same pass, 93 KB of LDS
-// and 128 FMAs per output on one workgroup per CU, took 79.5 us against 27.3 for
-// the depthwise kernel plus the MFMA GEMM.)
-template <int C>
-__global__ __launch_bounds__(256) void k_vae_resunit_fm(VaeResUnitArgs a) {
-    static_assert(C == 32 || C == 64, "narrow stages only");
-    constexpr uint32_t TB = 4096u / C, kMaxHalo = 54u, K = 7u;
-    constexpr uint32_t NS = ((TB + kMaxHalo) * C + 255u) / 256u;
-    constexpr uint32_t G = 256u / C;   // row groups of the thread block
-    __shared__ __align__(16) float xs[(TB + kMaxHalo) * C];
-    __shared__ __align__(16) float hs[TB * C];
-    const uint32_t tid = threadIdx.x, t0 = blockIdx.x * TB, halo = 6u * a.dilation;
-    const uint32_t n_st = (TB + halo) * C;
-    const uint32_t c = tid % C;   // n_st, C are multiples of 256 / C, so idx % C == c
-    float xv[NS];
-#pragma unroll
-    for (uint32_t i = 0; i < NS; ++i) {
-        const uint32_t idx = tid + 256u * i;
-        const int ti = (int)(t0 + idx / C) - (int)halo;
-        xv[i] = idx < n_st && ti >= 0 && (uint32_t)ti < a.length ? a.x[(size_t)ti * C + c] : 0.f;
+// The input of a stage's transposed convolution, P = snake_pa(x * ps + pt) per
+// channel (pre: f32 [4][C]: ps, pt, pa, 1 / (pa + 1e-9)). P is kept with a zero row
+// ahead of row 0: the GEMM row of output time j is [P[j-1] | P[j]], which is
+// contiguous there, so the rows overlap and nothing is copied twice.
+template <int V>
+__global__ __launch_bounds__(256) void k_vae_pre_fm(const float *x, float *y, const float *pre, uint32_t C,
+                                                    uint64_t n) {
+    const uint64_t i = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * V;
+    if (i >= n) return;
+    const uint32_t c = (uint32_t)(i % C);
+    float v[V], s[V], big = 0.f;
+    if constexpr (V == 4) {
+        const float4 q = *reinterpret_cast<const float4 *>(x + i);
+        v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+    } else {
+        v[0] = x[i];
     }
-    const float a1 = hf(a.a1[c]), a2 = hf(a.a2[c]), db = hf(a.db[c]);
-    const float i1 = snake_inv(a1), i2 = snake_inv(a2);
 #pragma unroll
-    for (uint32_t i = 0; i < NS; ++i) {
-        const uint32_t idx = tid + 256u * i;
-        if (idx < n_st) xs[idx] = snake_fm(xv[i], a1, i1);   // snake(0) = 0: the padding stays zero
+    for (int j = 0; j < V; ++j) {
+        v[j] = fmaf(v[j], pre[c + j], pre[C + c + j]);
+        s[j] = pre[2u * C + c + j] * v[j];
+        big = fmaxf(big, fabsf(s[j]));
     }
-    float wk[K];
-#pragma unroll
-    for (uint32_t k = 0; k < K; ++k) wk[k] = hf(a.dw[c * K + k]);
-    float pw[C];
-#pragma unroll
-    for (uint32_t j = 0; j < C; j += 8) {
-        const uint4 u = *reinterpret_cast<const uint4 *>(a.pw + (size_t)c * C + j);
-        const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const __half2 h = __builtin_bit_cast(__half2, uw[e]);
-            pw[j + 2 * e] = __low2float(h);
-            pw[j + 2 * e + 1] = __high2float(h);
+    if (any_large(big)) {
+#pragma unroll 1
+        for (int j = 0; j < V; ++j) {
+            const float w = fmaf(x[i + j], pre[c + j], pre[C + c + j]);
+            y[i + j] = snake_any(w, pre[2u * C + c + j] * w, pre[3u * C + c + j]);
         }
+        return;
     }
-    const float pb = hf(a.pb[c]);
-    __syncthreads();
-    for (uint32_t r = tid / C; r < TB; r += G) {
-        float sum = db;
 #pragma unroll
-        for (uint32_t k = 0; k < K; ++k) sum += xs[(r + k * a.dilation) * C + c] * wk[k];
-        hs[r * C + c] = snake_fm(sum, a2, i2);
-    }
-    __syncthreads();
-    for (uint32_t r = tid / C; r < TB; r += G) {
-        const uint32_t t = t0 + r;
-        if (t >= a.length) break;
-        const float4 *h4 = reinterpret_cast<const float4 *>(hs + r * C);
-        float s0 = pb, s1 = 0.f;
-#pragma unroll
-        for (uint32_t j = 0; j < C / 4; ++j) {
-            const float4 v = h4[j];
-            s0 = fmaf(v.x, pw[4 * j], s0);
-            s1 = fmaf(v.y, pw[4 * j + 1], s1);
-            s0 = fmaf(v.z, pw[4 * j + 2], s0);
-            s1 = fmaf(v.w, pw[4 * j + 3], s1);
-        }
-        a.y[(size_t)t * C + c] = a.x[(size_t)t * C + c] + (s0 + s1);
-    }
+    for (int j = 0; j < V; ++j) v[j] = snake_fm(v[j], s[j], pre[3u * C + c + j]);
+    if constexpr (V == 4)
+        *reinterpret_cast<float4 *>(y + i) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+        y[i] = v[0];
 }
 
-// Input of a stride-s transposed convolution as a GEMM: row j of X2 is
-// [pre(x[j]) | pre(x[j-1])] (zeros for j = 0), pre = snake(alpha)(x * scale + bias)
-// with the per-channel scale/bias of the sample-rate bucket.
-__global__ __launch_bounds__(256) void k_vae_convt_input_fm(VaeConvtInArgs a) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    const uint32_t C = a.channels;
-    if (i >= (uint64_t)a.length * 2u * C) return;
-    const uint32_t j = (uint32_t)(i / (2u * C)), r = (uint32_t)(i - (uint64_t)j * 2u * C);
-    const uint32_t tap = r >= C ? 1u : 0u, c = r - tap * C;
-    float v = 0.f;
-    if (j >= tap) {
-        const float x = a.x[(size_t)(j - tap) * C + c];
-        const float pre = a.scale ? x * hf(a.scale[c]) + hf(a.bias[c]) : x;
-        const float al = hf(a.alpha[c]);
-        v = snake_fm(pre, al, snake_inv(al));
-    }
-    a.x2[i] = v;
+__global__ __launch_bounds__(256) void k_vae_repack_pre(const __half *scale, const __half *bias, const __half *alpha,
+                                                        uint32_t C, float *pre) {
+    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+    if (c >= C) return;
+    pre[c] = hf(scale[c]);
+    pre[C + c] = hf(bias[c]);
+    pre[2u * C + c] = hf(alpha[c]);
+    pre[3u * C + c] = snake_inv(hf(alpha[c]));
 }
 
 // Repack of a ConvTranspose1d weight [Cin][Cout][2s] (kernel 2s, stride s) for
-// the GEMM form: W'[(r Cout + oc)][tap Cin + ic] = W[ic][oc][r + tap s], and the
-// bias tiled over the s phases, b'[r Cout + oc] = b[oc].
+// the GEMM form: W'[(r Cout + oc)][(1 - tap) Cin + ic] = W[ic][oc][r + tap s] (tap 1
+// multiplies the earlier row, which comes first), and the bias tiled over the s phases, b'[r Cout + oc] = b[oc].
 __global__ __launch_bounds__(256) void k_vae_repack_convt(const __half *w, const __half *b, uint32_t cin,
                                                           uint32_t cout, uint32_t s, __half *wp, float *bp) {
     const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
@@ -275,7 +264,7 @@ __global__ __launch_bounds__(256) void k_vae_repack_convt(const __half *w, const
     if (i < n) {
         const uint32_t row = (uint32_t)(i / (2u * cin)), col = (uint32_t)(i - (uint64_t)row * 2u * cin);
         const uint32_t r = row / cout, oc = row - r * cout, tap = col / cin, ic = col - tap * cin;
-        wp[i] = w[((size_t)ic * cout + oc) * (2u * s) + r + tap * s];
+        wp[i] = w[((size_t)ic * cout + oc) * (2u * s) + r + (1u - tap) * s];
     }
     if (i < (uint64_t)s * cout) bp[i] = hf(b[i % cout]);
 }
@@ -368,41 +357,95 @@ __global__ __launch_bounds__(256) void k_vae_head_fm(VaeHeadArgs a) {
     a.y[t] = tanhf(sum);
 }
 
-// The head tiled over 256 output rows: snake(x) of the rows and the left halo
-// staged once in LDS (row stride C + 1), C <= 48, with the conv weights in LDS.
-// For the decoder's 32 output channels (NC = 32) every staging load is issued
-// before the first is used; NC = 0 takes any C with a plain staging loop.
-template <uint32_t NC>
+// The head for the decoder's 32 output channels, tiled over 32 * NO output rows:
+// snake(x) of the rows and the left halo staged once in LDS, every load issued before
+// the first is used. Eight lanes of four channels each compute NO consecutive
+// outputs from NO + 6 rows (a 16-byte read a row for 28 products an output) and meet
+// by DPP. (One thread per output, reading every channel and tap from LDS, was bound
+// by those reads: 63.2 us at 483840 samples.)
+template <int NO>
+__global__ __launch_bounds__(256) void k_vae_head32_fm(VaeHeadArgs a) {
+    constexpr uint32_t TB = 32u * NO, NR = TB + 6u, NS = (NR * 8u + 255u) / 256u;
+    __shared__ __align__(16) float xs[NR * 32u];
+    const uint32_t tid = threadIdx.x, g = tid & 7u, t0 = blockIdx.x * TB;
+    float4 xv[NS];
+#pragma unroll
+    for (uint32_t i = 0; i < NS; ++i) {
+        const uint32_t r = (tid >> 3) + 32u * i;
+        const int t = (int)(t0 + r) - 6;
+        xv[i] = r < NR && t >= 0 && (uint32_t)t < a.length
+                    ? *reinterpret_cast<const float4 *>(a.x + (size_t)t * 32u + 4u * g)
+                    : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float al[4], inv[4], w[7][4], big = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        al[e] = hf(a.alpha[4u * g + e]);
+        inv[e] = snake_inv(al[e]);
+#pragma unroll
+        for (int k = 0; k < 7; ++k) w[k][e] = hf(a.w[(4u * g + e) * 7u + k]);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < NS; ++i) {
+        const uint32_t r = (tid >> 3) + 32u * i;
+        const float v[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float s = al[e] * v[e];
+            big = fmaxf(big, fabsf(s));
+            o[e] = snake_fm(v[e], s, inv[e]);   // snake(0) = 0: the padding stays zero
+        }
+        if (r < NR) *reinterpret_cast<float4 *>(xs + r * 32u + 4u * g) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+    if (any_large(big)) {
+#pragma unroll 1
+        for (uint32_t i = 0; i < 4u * NS; ++i) {
+            const uint32_t r = (tid >> 3) + 32u * (i >> 2), c = 4u * g + (i & 3u);
+            const int t = (int)(t0 + r) - 6;
+            if (r >= NR || t < 0 || (uint32_t)t >= a.length) continue;
+            const float v = a.x[(size_t)t * 32u + c], av = hf(a.alpha[c]);
+            xs[r * 32u + c] = snake_any(v, av * v, snake_inv(av));
+        }
+    }
+    __syncthreads();
+    const uint32_t o0 = (tid >> 3) * NO;
+    float acc[NO] = {};
+#pragma unroll
+    for (int r = 0; r < NO + 6; ++r) {
+        const float4 q = *reinterpret_cast<const float4 *>(xs + (o0 + r) * 32u + 4u * g);
+#pragma unroll
+        for (int o = 0; o < NO; ++o) {
+            const int k = r - o;
+            if (k < 0 || k > 6) continue;
+            acc[o] = fmaf(q.x, w[k][0], acc[o]);
+            acc[o] = fmaf(q.y, w[k][1], acc[o]);
+            acc[o] = fmaf(q.z, w[k][2], acc[o]);
+            acc[o] = fmaf(q.w, w[k][3], acc[o]);
+        }
+    }
+    float mine = 0.f;
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+        const float v = sum8(acc[o]);
+        mine = g == (uint32_t)o ? v : mine;
+    }
+    const uint32_t t = t0 + o0 + g;
+    if (g < (uint32_t)NO && t < a.length) a.y[t] = tanhf(mine + hf(a.b[0]));
+}
+
+// Other channel counts up to 48: one thread an output row, snake(x) of 256 rows and
+// the left halo staged in LDS (row stride C + 1) with the conv weights.
 __global__ __launch_bounds__(256) void k_vae_head_tiled_fm(VaeHeadArgs a) {
     __shared__ float xs[(256 + 6) * 49];
     __shared__ float ws[48 * 7];
-    const uint32_t C = NC ? NC : a.channels, S = C + 1u, t0 = blockIdx.x * 256u, halo = a.left_pad;
+    const uint32_t C = a.channels, S = C + 1u, t0 = blockIdx.x * 256u, halo = a.left_pad;
     const uint32_t n_st = (256u + halo) * C, tid = threadIdx.x;
     for (uint32_t i = tid; i < C * a.kernel; i += 256u) ws[i] = hf(a.w[i]);
-    if constexpr (NC != 0) {
-        constexpr uint32_t NS = ((256u + 6u) * NC + 255u) / 256u;
-        float xv[NS];
-#pragma unroll
-        for (uint32_t i = 0; i < NS; ++i) {
-            const uint32_t idx = tid + 256u * i, r = idx / NC, c = idx % NC;
-            const int ti = (int)(t0 + r) - (int)halo;
-            xv[i] = idx < n_st && ti >= 0 && (uint32_t)ti < a.length ? a.x[(size_t)ti * NC + c] : 0.f;
-        }
-        const uint32_t c = tid % NC;   // NC divides 256: each thread keeps one channel
-        const float al = hf(a.alpha[c]), inv = snake_inv(al);
-#pragma unroll
-        for (uint32_t i = 0; i < NS; ++i) {
-            const uint32_t idx = tid + 256u * i;
-            if (idx < n_st) xs[(idx / NC) * S + c] = snake_fm(xv[i], al, inv);   // snake(0) = 0
-        }
-    } else {
-        for (uint32_t idx = tid; idx < n_st; idx += 256u) {
-            const uint32_t r = idx / C, c = idx - r * C;
-            const int ti = (int)(t0 + r) - (int)halo;
-            const float al = hf(a.alpha[c]);
-            xs[r * S + c] = ti >= 0 && (uint32_t)ti < a.length ? snake_fm(a.x[(size_t)ti * C + c], al, snake_inv(al))
-                                                               : 0.f;
-        }
+    for (uint32_t idx = tid; idx < n_st; idx += 256u) {
+        const uint32_t r = idx / C, c = idx - r * C;
+        const int ti = (int)(t0 + r) - (int)halo;
+        xs[r * S + c] = ti >= 0 && (uint32_t)ti < a.length ? snake(a.x[(size_t)ti * C + c], hf(a.alpha[c])) : 0.f;
     }
     __syncthreads();
     const uint32_t t = t0 + tid;
@@ -478,32 +521,21 @@ int launch_vae_dwconv_fm(hipStream_t s, const VaeDwArgs &a) {
     return VX_OK;
 }
 
-bool vae_resunit_eligible(const VaeResUnitArgs &a) {
-    const bool aligned = ((reinterpret_cast<uintptr_t>(a.pw) | reinterpret_cast<uintptr_t>(a.x) |
-                           reinterpret_cast<uintptr_t>(a.y)) & 15u) == 0;
-    return (a.channels == 32u || a.channels == 64u) && a.dilation >= 1u &&
-           6u * a.dilation <= 54u && aligned && a.x != a.y;
-}
-
-int launch_vae_resunit_fm(hipStream_t s, const VaeResUnitArgs &a) {
-    if (!a.length) return VX_OK;
-    if (!vae_resunit_eligible(a)) return fail(VX_ERR_UNSUPPORTED, "vae residual unit: %u channels, dilation %u",
-                                              a.channels, a.dilation);
-    const uint32_t tb = 4096u / a.channels;
-    const uint32_t grid = (a.length + tb - 1u) / tb;
-    if (a.channels == 32u)
-        k_vae_resunit_fm<32><<<grid, 256, 0, s>>>(a);
+int launch_vae_pre_fm(hipStream_t s, const float *x, float *y, const float *pre, uint32_t channels, uint32_t length) {
+    const uint64_t n = (uint64_t)length * channels;
+    if (!n) return VX_OK;
+    if (channels % 4u == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0)
+        k_vae_pre_fm<4><<<grid1(n / 4u), 256, 0, s>>>(x, y, pre, channels, n);
     else
-        k_vae_resunit_fm<64><<<grid, 256, 0, s>>>(a);
-    VX_LAUNCHED("k_vae_resunit_fm");
+        k_vae_pre_fm<1><<<grid1(n), 256, 0, s>>>(x, y, pre, channels, n);
+    VX_LAUNCHED("k_vae_pre_fm");
     return VX_OK;
 }
 
-int launch_vae_convt_input_fm(hipStream_t s, const VaeConvtInArgs &a) {
-    const uint64_t n = (uint64_t)a.length * 2u * a.channels;
-    if (!n) return VX_OK;
-    k_vae_convt_input_fm<<<grid1(n), 256, 0, s>>>(a);
-    VX_LAUNCHED("k_vae_convt_input_fm");
+int launch_vae_repack_pre(hipStream_t s, const __half *scale, const __half *bias, const __half *alpha,
+                          uint32_t channels, float *pre) {
+    k_vae_repack_pre<<<grid1(channels), 256, 0, s>>>(scale, bias, alpha, channels, pre);
+    VX_LAUNCHED("k_vae_repack_pre");
     return VX_OK;
 }
 
@@ -538,11 +570,17 @@ int launch_vae_linear_fm(hipStream_t s, const VaeLinearArgs &a) {
 
 int launch_vae_head_fm(hipStream_t s, const VaeHeadArgs &a) {
     if (!a.length) return VX_OK;
-    if (a.channels <= 48u && a.left_pad <= 6u && a.kernel == a.left_pad + 1u) {
-        if (a.channels == 32u)
-            k_vae_head_tiled_fm<32><<<grid1(a.length), 256, 0, s>>>(a);
+    if (a.channels == 32u && a.left_pad == 6u && a.kernel == 7u && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0) {
+        // 256 rows a workgroup once that gives every CU one, else 64.
+        if (a.length >= 256u * 256u)
+            k_vae_head32_fm<8><<<(a.length + 255u) / 256u, 256, 0, s>>>(a);
         else
-            k_vae_head_tiled_fm<0><<<grid1(a.length), 256, 0, s>>>(a);
+            k_vae_head32_fm<2><<<(a.length + 63u) / 64u, 256, 0, s>>>(a);
+        VX_LAUNCHED("k_vae_head32_fm");
+        return VX_OK;
+    }
+    if (a.channels <= 48u && a.left_pad <= 6u && a.kernel == a.left_pad + 1u) {
+        k_vae_head_tiled_fm<<<grid1(a.length), 256, 0, s>>>(a);
         VX_LAUNCHED("k_vae_head_tiled_fm");
         return VX_OK;
     }

@@ -608,25 +608,26 @@ struct VaeDwArgs {                  // depthwise conv over frame-major rows
     uint32_t channels = 0, length = 0, kernel = 7, dilation = 1, left_pad = 0;
 };
 int launch_vae_dwconv_fm(hipStream_t s, const VaeDwArgs &a);
-// A decoder residual unit in one pass for 32 or 64 channels:
-//   y[t][n] = x[t][n] + pb[n] + sum_c pw[n][c] snake_a2(db[c] + sum_k dw[c][k] snake_a1(x[t + k d - 6d][c]))
-// (the depthwise conv, kernel 7, causal, and the 1x1 conv). y must not alias x.
-struct VaeResUnitArgs {
+// A decoder residual unit in one pass (32, 64, 128 or 256 channels), parameters and
+// 1x1 weight as launch_vae_repack_unit lays them out; pre (nullable, f32 [4][C] as
+// launch_vae_repack_pre) also applies the next stage's input transform. y must not
+// alias x.
+struct VaeUnitArgs {
     const float *x = nullptr;
     float *y = nullptr;
-    const __half *a1 = nullptr, *dw = nullptr, *db = nullptr, *a2 = nullptr, *pw = nullptr, *pb = nullptr;
+    const float *p = nullptr;
+    const __half *w = nullptr;
+    const float *pre = nullptr;
     uint32_t channels = 0, length = 0, dilation = 1;
 };
-bool vae_resunit_eligible(const VaeResUnitArgs &a);
-int launch_vae_resunit_fm(hipStream_t s, const VaeResUnitArgs &a);
-struct VaeConvtInArgs {             // [pre(x[j]) | pre(x[j-1])] rows for the transposed-conv GEMM
-    const float *x = nullptr;
-    float *x2 = nullptr;
-    const __half *scale = nullptr, *bias = nullptr;     // nullable: the sample-rate bucket's rows
-    const __half *alpha = nullptr;
-    uint32_t channels = 0, length = 0;
-};
-int launch_vae_convt_input_fm(hipStream_t s, const VaeConvtInArgs &a);
+bool vae_unit_channels(uint32_t channels);
+int launch_vae_unit(hipStream_t s, const VaeUnitArgs &a);
+int launch_vae_repack_unit(hipStream_t s, const __half *a1, const __half *dw, const __half *db, const __half *a2,
+                           const __half *pw, const __half *pb, uint32_t channels, float *p, __half *w);
+// y = snake_pa(x * ps + pt) per channel, pre as launch_vae_repack_pre lays it out.
+int launch_vae_pre_fm(hipStream_t s, const float *x, float *y, const float *pre, uint32_t channels, uint32_t length);
+int launch_vae_repack_pre(hipStream_t s, const __half *scale, const __half *bias, const __half *alpha,
+                          uint32_t channels, float *pre);
 int launch_vae_repack_convt(hipStream_t s, const __half *w, const __half *b, uint32_t cin, uint32_t cout,
                             uint32_t stride, __half *wp, float *bp);
 struct VaeLinearArgs {              // y[t][n] (+)= b[n] + x[t] . W[n], short K
