@@ -172,6 +172,34 @@ def test_batched_prefill_f16_weights(ctx):
     model.free()
 
 
+@pytest.mark.parametrize("n", [128, 129, 300, 500])
+def test_batched_prefill_f16_tiles(ctx, n):
+    """F16 weights from one whole 128-token tile up: 128 and 129 rows (one and two
+    tiles, split K), 300 (stream-K gate/up, both hand-off orders bit-identical) and 500
+    (whole tiles and K halves)."""
+    print(f"batched f16 prefill n={n}", flush=True)
+    cfg = synth.baselm_config(layers=1, vocab=512, context_length=32768, active_context=512)
+    m = synth.build_baselm(cfg, seed=0x5EED0120, weight_type="f16")
+    model = Model(ctx, m.data, m.tensors)
+    toks = [int(t) for t in synth.uniform_u32(n, 0x5EED0121 + n, cfg["vocab_size"])]
+    o = oracle_of(m, cfg)
+    for p, t in enumerate(toks):
+        o.decode_token(t, p)
+    got = []
+    for sched in ("auto", "streamk_tail_first") if n == 300 else ("auto",):
+        eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False, prefill_schedule=sched)
+        eng.prefill_tokens_batched(toks)
+        got.append(eng.output())
+        assert rel_l2(got[-1], o.norm) < 1e-3
+        for name, ref in (("kv_k", o.kv_k), ("kv_v", o.kv_v)):
+            rows = kv_rows(eng, name, 1, 512)
+            assert rel_l2(f16(rows[0, :n]), f16(ref.reshape(512, 256)[:n])) < 1e-3, name
+            assert np.all(rows[:, n:] == 0)
+        eng.close()
+    assert np.array_equal(got[0], got[-1])
+    model.free()
+
+
 def test_batched_prefill_errors(ctx, small):
     cfg, m, model = small
     eng = BaseLmEngine(ctx, model, dict(cfg, active_context_length=64), exec_mode="graph", strict_geometry=False)

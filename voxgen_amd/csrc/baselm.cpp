@@ -530,49 +530,12 @@ PrefillStack make_stack(vx_baselm *e) {
     return p;
 }
 
-// Split-K factor that brings a projection to about one workgroup per CU.
-// Repack every layer's Q8_0 projections into the prefill-GEMM layout (once;
-// about 53 MB per layer at the VoxCPM2 geometry). Left empty, so that prefill
-// uses the general GEMM, when a projection is not Q8_0.
 int ensure_prefill_weights(vx_baselm *e) {
     if (e->pw_tried) return VX_OK;
     e->pw_tried = true;
     const vx_baselm_config &c = e->cfg;
-    const uint32_t nH = c.embedding_length, nF = c.feed_forward_length, nKV = c.kv_dim;
-    for (const Layer &L : e->layers) {
-        const WRef *m[7] = {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down};
-        for (const WRef *w : m)
-            if (w->dtype != VX_DTYPE_Q8_0 || !w->raw) return VX_OK;
-    }
-    if (nH % 32u || nF % 32u) return VX_OK;
-    const uint64_t per_layer = prefill_matrix_bytes(nH, nH) + 2u * prefill_matrix_bytes(nKV, nH) +
-                               prefill_matrix_bytes(nH, nH) + prefill_matrix_bytes(2u * nF, nH) +
-                               prefill_matrix_bytes(nH, nF) + 6u * 256u;
-    VX_CHECK(alloc(e->ctx, per_layer * c.block_count, &e->pw_arena));
-    uint8_t *cur = static_cast<uint8_t *>(e->pw_arena->ptr);
-    hipStream_t s = e->ctx->stream;
-    auto place = [&](PrefillMatrix &pm, const WRef &w0, const WRef *w1, uint32_t rows, uint32_t K) {
-        const uint32_t rows_out = w1 ? 2u * rows : rows;
-        pm.rows_pad = (rows_out + 127u) / 128u * 128u;
-        pm.q = reinterpret_cast<int8_t *>(cur);
-        pm.d = reinterpret_cast<float *>(cur + (uint64_t)pm.rows_pad * K);
-        cur += (prefill_matrix_bytes(rows_out, K) + 255u) / 256u * 256u;
-        return launch_repack_prefill(s, w0.raw, w0.raw_offset, w1 ? w1->raw_offset : 0u, rows, K, w1 ? 1 : 0, pm.q,
-                                     pm.d);
-    };
-    e->pw.resize(c.block_count);
-    for (uint32_t l = 0; l < c.block_count; ++l) {
-        const Layer &L = e->layers[l];
-        StackPrefillWeights &P = e->pw[l];
-        int st = VX_OK;
-        if ((st = place(P.q, L.q, nullptr, nH, nH)) || (st = place(P.k, L.k, nullptr, nKV, nH)) ||
-            (st = place(P.v, L.v, nullptr, nKV, nH)) || (st = place(P.o, L.o, nullptr, nH, nH)) ||
-            (st = place(P.gu, L.gate, &L.up, nF, nH)) || (st = place(P.down, L.down, nullptr, nH, nF))) {
-            e->pw.clear();
-            return st;
-        }
-    }
-    return VX_OK;
+    return prefill_stack_weights(e->ctx, e->layers.data(), c.block_count, c.embedding_length, c.feed_forward_length,
+                                 c.kv_dim, &e->pw, &e->pw_arena);
 }
 
 // One chunk of T tokens at positions pos0..pos0+T-1, token ids at tok (device).

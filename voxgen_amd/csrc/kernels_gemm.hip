@@ -1,7 +1,18 @@
-// Prefill projection GEMM for Q8_0 weights on gfx950, token-batched (T >= 128):
-//   C[t][n] = sum_k X[t][k] * W[n][k],   X as hi/lo f16 planes, W = d * q (Q8_0).
+// Prefill projection GEMM on gfx950, token-batched (T >= 128):
+//   C[t][n] = sum_k X[t][k] * W[n][k],   X as hi/lo f16 planes, W = d * q (Q8_0) or f16.
 //
-// Same arithmetic as k_gemm (kernels_seq.hip): the int8 quants enter the MFMA as
+// F16 weights run the same tiles, ring, schedules and epilogues (k_gemm_pf<WT_F16>):
+// a stage holds an 8 KB piece of f16 weights instead of 4 KB of quants and the scales,
+// and the products accumulate in place, with no widening and no scale step. Against
+// k_gemm's 64-token tiles (operands through registers, two barriers a stage, 4-byte
+// atomic epilogues), four F16 layers of the VoxCPM2 geometry took on MI355X at
+// T = 130 / 256 / 384 / 512: 475 / 546 / 773 / 840 -> 441 / 501 / 613 / 691 us. A lone
+// workgroup's block costs 436 ns: the DMA of its 24 KB alone 347 (29 bytes a cycle
+// whatever the ring depth, 3 to 6 slots, and whether the source is one cached block),
+// its products and LDS reads alone 310; the rest of a launch is about 10 us of
+// prologue, epilogue and boundary.
+//
+// Q8_0: same arithmetic as k_gemm (kernels_seq.hip): the int8 quants enter the MFMA as
 // exact f16, each 32-column block's partial product is scaled by its f32 block
 // scale afterwards (acc += d[n][b] * sum_{k in b} q*x, matvec.comp:32-44), and X
 // enters as hi + lo planes through two MFMAs. The kernel is organised around
@@ -54,13 +65,16 @@ typedef float acc16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 128;                       // tokens per workgroup tile
 constexpr int kBN = 128;                       // weight rows per workgroup tile
-constexpr int kStages = 3;                     // LDS ring slots (61.5 KB: two workgroups per CU)
+constexpr int kStages = 3;                     // LDS ring slots (61.5 or 72 KB: two workgroups per CU)
 constexpr int kXBytes = kBM * 32 * 2;          // one plane of a stage: f16 [token][32]
-constexpr int kWBytes = kBN * 32;              // int8 quants [row][32]
-constexpr int kDBytes = kBN * 4;               // f32 scales [row]
-constexpr int kXOff = 0, kWOff = 2 * kXBytes, kDOff = kWOff + kWBytes;
-constexpr int kStageBytes = kDOff + kDBytes;   // 20992
 constexpr int kOpsPerStage = 6;                // DMA instructions per wave per stage
+template <int WK>
+struct Slot {                                  // one stage in the ring
+    static constexpr int kWBytes = WK == WT_Q8 ? kBN * 32 : kBN * 64;   // int8 quants or f16 weights [row][32]
+    static constexpr int kDBytes = WK == WT_Q8 ? kBN * 4 : 0;           // f32 scales [row]
+    static constexpr int kXOff = 0, kWOff = 2 * kXBytes, kDOff = kWOff + kWBytes;
+    static constexpr int kBytes = kDOff + kDBytes;                      // 20992 or 24576: two workgroups per CU
+};
 
 // Chunk permutations of the stored layouts: X rows of 64 bytes in 16-byte
 // chunks (tiled_plane_index), quant rows of 32 bytes in 8-byte chunks
@@ -132,60 +146,179 @@ __device__ __forceinline__ const uint8_t *uniform_ptr(const void *p) {
 }
 
 // Stage b (32-column block) of the tile: wave w copies X pieces 4w .. 4w + 3
-// (1 KB each, plane = piece / 8), quant piece w (1 KB), and one 256 B half of
-// the scales (waves 2 and 3 repeat what waves 0 and 1 copy). Bases are the
-// wave's pieces at block 0; lane i adds 16 i (4 i for the scales).
+// (1 KB each, plane = piece / 8) and, of Q8_0 weights, quant piece w (1 KB) and one
+// 256 B half of the scales (waves 2 and 3 repeat what waves 0 and 1 copy), of F16
+// weights pieces 2w and 2w + 1. Bases are the wave's pieces at block 0; lane i adds
+// 16 i (4 i for the scales).
 struct Src {
     const uint8_t *x[4];   // X plane piece
-    const uint8_t *w;      // quants + 1024 * wave
+    const uint8_t *w;      // the wave's weight piece(s)
     const uint8_t *d;      // scales + 256 * (wave & 1)
 };
 
-__device__ __forceinline__ void issue_stage(const Src &src, uint32_t blk, uint32_t slot, uint32_t wave,
-                                            uint32_t lane) {
+// Byte offset of block blk in the X planes: tiled planes, or (XB) block-major ones,
+// whose first x_shift blocks are read one row earlier.
+template <bool XB>
+__device__ __forceinline__ int64_t x_offset(const GemmArgs &a, uint32_t blk) {
+    if constexpr (!XB) return (int64_t)blk * kXBytes;
+    return blk < a.x_shift ? (int64_t)(blk * a.x_block) - 64 : (int64_t)((blk - a.x_shift) * a.x_block);
+}
+
+template <int WK, bool XB>
+__device__ __forceinline__ void issue_stage(const GemmArgs &a, const Src &src, uint32_t blk, uint32_t slot,
+                                            uint32_t wave, uint32_t lane) {
+    typedef Slot<WK> S;
+    const int64_t xo = x_offset<XB>(a, blk);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint32_t u = 4u * wave + (uint32_t)j;
-        dma16(src.x[j] + (size_t)blk * kXBytes, 16u * lane, slot + kXOff + (u >> 3) * kXBytes + (u & 7u) * 1024u);
+        dma16(src.x[j] + xo, 16u * lane, slot + S::kXOff + (u >> 3) * kXBytes + (u & 7u) * 1024u);
     }
-    dma16(src.w + (size_t)blk * kWBytes, 16u * lane, slot + kWOff + wave * 1024u);
-    dma4(src.d + (size_t)blk * kDBytes, 4u * lane, slot + kDOff + (wave & 1u) * 256u);
+    const uint8_t *w = src.w + (size_t)blk * S::kWBytes;
+    if constexpr (WK == WT_Q8) {
+        dma16(w, 16u * lane, slot + S::kWOff + wave * 1024u);
+        dma4(src.d + (size_t)blk * S::kDBytes, 4u * lane, slot + S::kDOff + (wave & 1u) * 256u);
+    } else {
+        dma16(w, 16u * lane, slot + S::kWOff + wave * 2048u);
+        dma16(w + 1024, 16u * lane, slot + S::kWOff + wave * 2048u + 1024u);
+    }
 }
 
 // The LDS ring of the block loop; the epilogues stage their results in it too.
+template <int WK>
 __device__ __forceinline__ uint8_t *gemm_ring() {
-    __shared__ __attribute__((aligned(16))) uint8_t ring[kStages * kStageBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t ring[kStages * Slot<WK>::kBytes];
     return ring;
 }
 
-// Blocks kb0 .. kb0 + nkb - 1 (nkb >= 1) of tile (tn, tm) of segment sg into acc
-// (overwritten). Every DMA of the wave has landed when this returns; the ring is
-// reused only after a barrier (other waves may still read their last block).
-template <int EPI>
-__device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg, uint32_t tn, uint32_t tm,
-                                            uint32_t kb0, uint32_t nkb, acc16 (&acc)[2][2]) {
-    uint8_t *const ring = gemm_ring();
-    const uint32_t ring_lds = lds_addr(ring);
+// DMA sources of tile (tn, tm) at block 0 (wave-uniform bases).
+template <int WK, int EPI, bool XB>
+__device__ __forceinline__ Src tile_src(const GemmArgs &a, const GemmSeg &sg, uint32_t tn, uint32_t tm, uint32_t wave) {
+    typedef Slot<WK> S;
     const uint32_t nblk = a.K / 32u;
+    const uint32_t lt = EPI == GEPI_SWIGLU ? tn : tn - sg.tile0;   // tile within the matrix
+    Src src;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t u = 4u * wave + (uint32_t)j;
+        const uint8_t *plane = reinterpret_cast<const uint8_t *>((u >> 3) ? a.xl : a.xh);
+        src.x[j] = uniform_ptr(plane + (size_t)tm * (XB ? 1u : nblk) * kXBytes + (u & 7u) * 1024u);
+    }
+    src.w = uniform_ptr(reinterpret_cast<const uint8_t *>(sg.pq) + ((size_t)lt * nblk) * S::kWBytes +
+                        (WK == WT_Q8 ? 1024u : 2048u) * wave);
+    src.d = nullptr;
+    if constexpr (WK == WT_Q8)
+        src.d = uniform_ptr(reinterpret_cast<const uint8_t *>(sg.pd) + ((size_t)lt * nblk) * S::kDBytes +
+                            256u * (wave & 1u));
+    return src;
+}
+
+// Blocks kb0 .. kb0 + nkb - 1 (nkb >= 1) of tile (tn, tm) of segment sg into acc
+// (overwritten), F16 weights. Every DMA of the wave has landed when this returns; the
+// ring is reused only after a barrier (other waves may still read their last block).
+template <int EPI, bool XB>
+__device__ __forceinline__ void tile_blocks_f16(const GemmArgs &a, const GemmSeg &sg, uint32_t tn, uint32_t tm,
+                                                uint32_t kb0, uint32_t nkb, acc16 (&acc)[2][2]) {
+    typedef Slot<WT_F16> S;
+    uint8_t *const ring = gemm_ring<WT_F16>();
+    const uint32_t ring_lds = lds_addr(ring);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, hs = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave & 1u, wn = wave >> 1;
+    const Src src = tile_src<WT_F16, EPI, XB>(a, sg, tn, tm, wave);
+    // Fragment addresses inside a slot (k-step e, 16 columns; this lane chunk 2e + hs).
+    // Rows read one earlier carry the permutation of that row.
+    uint32_t xa[XB ? 2 : 1][2][2], wa[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t t = 64u * wm + 32u * (uint32_t)i + l32, n = 64u * wn + 32u * (uint32_t)i + l32;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t c = 2u * (uint32_t)e + hs;
+            xa[0][i][e] = S::kXOff + t * 64u + ((c ^ xperm(t)) * 16u);
+            if constexpr (XB) xa[1][i][e] = S::kXOff + t * 64u + ((c ^ xperm(t - 1u)) * 16u);
+            wa[i][e] = S::kWOff + n * 64u + ((c ^ xperm(n)) * 16u);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < kStages; ++s)
+        issue_stage<WT_F16, XB>(a, src, kb0 + ((uint32_t)s < nkb ? (uint32_t)s : nkb - 1u),
+                                ring_lds + (uint32_t)s * S::kBytes, wave, lane);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = acc16{};
+    // The fragments of block i + 1 are read while block i is multiplied (two register
+    // sets), so LDS reads and matrix work overlap inside one wave: with a lone
+    // workgroup per CU the four waves meet at every barrier, and reading first and
+    // multiplying after left each side idle while the other ran (1400 cycles a block
+    // for 512 of MFMA). A slot is free for block i + 3 once every wave has read block
+    // i's fragments, that is after the barrier that opens block i's products.
+    struct Frags {
+        h8 ah[2][2], al[2][2], bf[2][2];   // [e][tile]
+    };
+    auto read = [&](uint32_t it, uint32_t slot, Frags &f) {
+        const uint8_t *const base = ring + slot * (uint32_t)S::kBytes;
+        const bool shifted = XB && kb0 + it < a.x_shift;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t x = XB && shifted ? xa[XB ? 1 : 0][i][e] : xa[0][i][e];
+                f.bf[e][i] = *reinterpret_cast<const h8 *>(base + wa[i][e]);
+                f.ah[e][i] = *reinterpret_cast<const h8 *>(base + x);
+                f.al[e][i] = *reinterpret_cast<const h8 *>(base + x + kXBytes);
+            }
+    };
+    uint32_t slot = 0;   // ring slot of block `it`
+    auto step = [&](uint32_t it, const Frags &cur, Frags &next) {
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vm<kOpsPerStage * (kStages - 2), true>();   // block it + 1 has landed, cur is read
+        __builtin_amdgcn_s_barrier();
+        const uint32_t nxt = it + kStages;
+        issue_stage<WT_F16, XB>(a, src, kb0 + (nxt < nkb ? nxt : nkb - 1u), ring_lds + slot * (uint32_t)S::kBytes, wave,
+                                lane);
+        slot = slot + 1u == kStages ? 0u : slot + 1u;
+        __builtin_amdgcn_sched_barrier(0);
+        read(it + 1u, slot, next);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {   // no two dependent MFMAs adjacent
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) acc[mt][nt] = mfma(cur.ah[e][mt], cur.bf[e][nt], acc[mt][nt]);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) acc[mt][nt] = mfma(cur.al[e][mt], cur.bf[e][nt], acc[mt][nt]);
+        }
+    };
+    Frags f0, f1;
+    wait_vm<kOpsPerStage * (kStages - 1)>();   // block 0 has landed
+    __builtin_amdgcn_s_barrier();
+    read(0, 0, f0);
+    uint32_t it = 0;
+    for (; it + 2u <= nkb; it += 2u) {
+        step(it, f0, f1);
+        step(it + 1u, f1, f0);
+    }
+    if (it < nkb) step(it, f0, f1);
+    wait_vm<0>();
+}
+
+// The same for Q8_0 weights.
+template <int EPI>
+__device__ __forceinline__ void tile_blocks_q8(const GemmArgs &a, const GemmSeg &sg, uint32_t tn, uint32_t tm,
+                                               uint32_t kb0, uint32_t nkb, acc16 (&acc)[2][2]) {
+    typedef Slot<WT_Q8> S;
+    constexpr int kXOff = S::kXOff, kWOff = S::kWOff, kDOff = S::kDOff, kStageBytes = S::kBytes;
+    uint8_t *const ring = gemm_ring<WT_Q8>();
+    const uint32_t ring_lds = lds_addr(ring);
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, hs = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave & 1u, wn = wave >> 1;
-
-    // ---- DMA sources of this tile at block 0 (wave-uniform bases)
-    Src src;
-    {
-        const uint32_t lt = EPI == GEPI_SWIGLU ? tn : tn - sg.tile0;   // tile within the matrix
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t u = 4u * wave + (uint32_t)j;
-            const uint8_t *plane = reinterpret_cast<const uint8_t *>((u >> 3) ? a.xl : a.xh);
-            src.x[j] = uniform_ptr(plane + ((size_t)tm * nblk) * kXBytes + (u & 7u) * 1024u);
-        }
-        src.w = uniform_ptr(reinterpret_cast<const uint8_t *>(sg.pq) + ((size_t)lt * nblk) * kWBytes + 1024u * wave);
-        src.d = uniform_ptr(reinterpret_cast<const uint8_t *>(sg.pd) + ((size_t)lt * nblk) * kDBytes +
-                            256u * (wave & 1u));
-    }
+    const Src src = tile_src<WT_Q8, EPI, false>(a, sg, tn, tm, wave);
 
     // ---- fragment addresses inside a stage slot: k-step e covers columns
     // 16e .. 16e + 15 of the block; this lane takes 8 of them, chunk 2e + hs.
@@ -209,8 +342,8 @@ __device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg
     // number of DMA instructions per stage, which the vmcnt waits count on)
 #pragma unroll
     for (int s = 0; s < kStages - 1; ++s)
-        issue_stage(src, kb0 + ((uint32_t)s < nkb ? (uint32_t)s : nkb - 1u), ring_lds + (uint32_t)s * kStageBytes, wave,
-                    lane);
+        issue_stage<WT_Q8, false>(a, src, kb0 + ((uint32_t)s < nkb ? (uint32_t)s : nkb - 1u),
+                                  ring_lds + (uint32_t)s * kStageBytes, wave, lane);
 
     acc16 p[2][2];
 #pragma unroll
@@ -235,8 +368,8 @@ __device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg
         wait_vm<kOpsPerStage * (kStages - 2), true>();
         __builtin_amdgcn_s_barrier();
         const uint32_t nxt = it + kStages - 1u;
-        issue_stage(src, kb0 + (nxt < nkb ? nxt : nkb - 1u), ring_lds + ((SL + kStages - 1u) % kStages) * kStageBytes,
-                    wave, lane);
+        issue_stage<WT_Q8, false>(a, src, kb0 + (nxt < nkb ? nxt : nkb - 1u),
+                                  ring_lds + ((SL + kStages - 1u) % kStages) * kStageBytes, wave, lane);
         const uint8_t *slot = ring + SL * kStageBytes;
         uint2 q[2][2];
         h8 ah[2][2], al[2][2], bf[2][2];   // [e][nt], [e][mt], [e][mt], [e][nt]
@@ -312,6 +445,15 @@ __device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg
     wait_vm<0>();
 }
 
+template <int WK, int EPI, bool XB = false>
+__device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg, uint32_t tn, uint32_t tm,
+                                            uint32_t kb0, uint32_t nkb, acc16 (&acc)[2][2]) {
+    if constexpr (WK == WT_Q8)
+        tile_blocks_q8<EPI>(a, sg, tn, tm, kb0, nkb, acc);
+    else
+        tile_blocks_f16<EPI, XB>(a, sg, tn, tm, kb0, nkb, acc);
+}
+
 // Accumulator layout: lane (l32, hs) of wave (wm, wn) holds, for tile (mt, nt),
 // tile row rho = 64wn + 32nt + l32 and tokens m0 + 64wm + 32mt + 8(r/4) + 4hs + r%4.
 // SwiGLU tiles interleave 32 gate rows (nt = 0) with the same 32 up rows (nt = 1),
@@ -321,11 +463,12 @@ __device__ __forceinline__ void tile_blocks(const GemmArgs &a, const GemmSeg &sg
 // contiguous 8 KB block per plane in that layout, built in LDS and copied out
 // whole with 16-byte stores. Token rows past T (the last tile's padding) get
 // zeros. Every thread of the workgroup calls it (barriers inside).
+template <int WK>
 __device__ __forceinline__ void swiglu_planes(const GemmArgs &a, uint32_t tn, uint32_t m0, const acc16 (&acc)[2][2]) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, hs = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave & 1u, wn = wave >> 1;
-    _Float16 *const st = reinterpret_cast<_Float16 *>(gemm_ring());   // [plane][group][128][32]
+    _Float16 *const st = reinterpret_cast<_Float16 *>(gemm_ring<WK>());   // [plane][group][128][32]
     __syncthreads();   // ring idle: every wave has drained its DMA and read its last block
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -382,8 +525,8 @@ __device__ __forceinline__ void swiglu_scalar(const GemmArgs &a, uint32_t tn, ui
     }
 }
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void k_gemm_q8p(GemmArgs a) {
+template <int WK, int EPI, bool XB>
+__global__ __launch_bounds__(256, 2) void k_gemm_pf(GemmArgs a) {
     // XCD-major order: workgroup b runs on XCD b % 8; consecutive ids of one XCD
     // cover the token tiles of the same weight rows.
     const uint32_t b = blockIdx.x;
@@ -403,11 +546,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p(GemmArgs a) {
     if (kb1 == kb0) return;   // nothing to add (ksplit is clamped to the block count)
 
     acc16 acc[2][2];
-    tile_blocks<EPI>(a, sg, tn, tm, kb0, kb1 - kb0, acc);
+    tile_blocks<WK, EPI, XB>(a, sg, tn, tm, kb0, kb1 - kb0, acc);
 
     if constexpr (EPI == GEPI_SWIGLU) {
         if (a.o_tiled && a.oh && !a.seg[0].out)
-            swiglu_planes(a, tn, m0, acc);
+            swiglu_planes<WK>(a, tn, m0, acc);
         else
             swiglu_scalar(a, tn, m0, acc);
     } else {
@@ -416,17 +559,35 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p(GemmArgs a) {
         const uint32_t wm = wave & 1u, wn = wave >> 1;
         float *const out0 = sg.out;
         const uint32_t ldo0 = sg.ldo, rows0 = sg.rows;
+        if constexpr (WK == WT_F16) {   // the bias enters with the first split
+            if (sg.bias && ks == 0) {
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    const uint32_t row = tile_row<EPI>(tn, sg.tile0, 64u * wn + 32u * (uint32_t)nt + l32);
+                    if (row >= rows0) continue;
+                    const float bias = sg.bias_dtype == 0 ? static_cast<const float *>(sg.bias)[row]
+                                                          : (float)static_cast<const _Float16 *>(sg.bias)[row];
+#pragma unroll
+                    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) acc[mt][nt][r] += bias;
+                }
+            }
+        }
         // Plain stores (a whole product, or one split's partial slab) go through
         // LDS (the ring is free once every wave has drained its DMA) in two passes
         // of 64 tokens and leave as 16-byte stores, 512 contiguous bytes per token
         // row, instead of 4-byte stores scattered over every lane's 64 results.
-        const bool plain =
-            EPI == GEPI_STORE ? (a.ksplit == 1u || a.split_store != 0u) : (a.ws != nullptr && a.ksplit > 1u);
+        // An F16 residual product without a split is added to its output the same way
+        // (Q8_0 ones that large do not occur in a 512-row chunk).
+        const bool add = WK == WT_F16 && EPI == GEPI_RESIDUAL && a.ksplit == 1u;
+        const bool plain = EPI == GEPI_STORE ? (a.ksplit == 1u || a.split_store != 0u) : (add || a.ws != nullptr);
         if (plain && a.wide) {
             float *const base = EPI == GEPI_STORE ? out0 + (a.ksplit > 1u ? ks * a.ws_stride : 0u)
+                                : add             ? out0
                                                   : a.ws + ks * a.ws_stride;
             const float f = EPI == GEPI_STORE ? a.alpha : a.scale;
-            float *const st = reinterpret_cast<float *>(gemm_ring());
+            float *const st = reinterpret_cast<float *>(gemm_ring<WK>());
             constexpr uint32_t kLd = kBN + 8;   // staging row: the two half-waves' tokens 32 banks apart
             const uint32_t row_base = tile_row<EPI>(tn, sg.tile0, 0);
 #pragma unroll
@@ -447,9 +608,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p(GemmArgs a) {
                 for (uint32_t i = tid; i < 64u * (kBN / 4u); i += 256u) {
                     const uint32_t tl = i / (kBN / 4u), c4 = i % (kBN / 4u);
                     const uint32_t tok = m0 + 64u * pass + tl, row = row_base + 4u * c4;
-                    if (tok < a.T && row < rows0)
-                        *reinterpret_cast<float4 *>(base + (size_t)tok * ldo0 + row) =
-                            *reinterpret_cast<const float4 *>(st + tl * kLd + 4u * c4);
+                    if (tok < a.T && row < rows0) {
+                        float4 v = *reinterpret_cast<const float4 *>(st + tl * kLd + 4u * c4);
+                        float4 *const dst = reinterpret_cast<float4 *>(base + (size_t)tok * ldo0 + row);
+                        if (add) {
+                            const float4 o = *dst;
+                            v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
+                        }
+                        *dst = v;
+                    }
                 }
             }
             return;
@@ -549,11 +716,11 @@ __device__ __forceinline__ void sk_add(const float *slot, acc16 (&acc)[2][2]) {
 // counter. Nothing waits on another workgroup, and fp32 addition of the two parts
 // commutes, so the result does not depend on which finishes. TAIL_FIRST computes
 // the tail first, so the store-and-count path runs every time (same result bits).
-template <bool TAIL_FIRST>
-__global__ __launch_bounds__(256, 2) void k_gemm_q8p_sk(GemmArgs a) {
+template <int WK, bool TAIL_FIRST>
+__global__ __launch_bounds__(256, 2) void k_gemm_pf_sk(GemmArgs a) {
     __shared__ uint32_t flag;
     const uint32_t b = blockIdx.x;
-    const uint32_t id = (b & 7u) * (gridDim.x >> 3) + (b >> 3);   // XCD-major, as k_gemm_q8p
+    const uint32_t id = (b & 7u) * (gridDim.x >> 3) + (b >> 3);   // XCD-major, as k_gemm_pf
     const uint32_t nblk = a.K / 32u;
     const uint32_t total = a.ntn * a.ntm * nblk;
     const uint32_t g0 = min(id * a.sk_per, total), g1 = min(g0 + a.sk_per, total);
@@ -568,11 +735,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p_sk(GemmArgs a) {
         if (!first) __syncthreads();   // the previous piece's ring and staging reads are done
         first = false;
         const uint32_t tn = tile / a.ntm, tm = tile - tn * a.ntm;
-        tile_blocks<GEPI_SWIGLU>(a, a.seg[0], tn, tm, kb, n, acc);
+        tile_blocks<WK, GEPI_SWIGLU>(a, a.seg[0], tn, tm, kb, n, acc);
     };
     auto finish = [&](uint32_t tile, const acc16 (&acc)[2][2]) {
         const uint32_t tn = tile / a.ntm;
-        swiglu_planes(a, tn, (tile - tn * a.ntm) * kBM, acc);
+        swiglu_planes<WK>(a, tn, (tile - tn * a.ntm) * kBM, acc);
     };
     auto head = [&]() {   // the head of tile t_last; its tail starts range id + 1
         acc16 acc[2][2];
@@ -632,7 +799,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p_sk(GemmArgs a) {
 // whole tiles. The halves of a tile (on one XCD) store their parts, count on the
 // tile's counter, and the second to count adds the other part and runs the
 // epilogue, then clears the counter; nothing waits, and the sum commutes.
-__global__ __launch_bounds__(256, 2) void k_gemm_q8p_half(GemmArgs a) {
+template <int WK>
+__global__ __launch_bounds__(256, 2) void k_gemm_pf_half(GemmArgs a) {
     __shared__ uint32_t flag;
     const uint32_t b = blockIdx.x, G = a.sk_grid, nblk = a.K / 32u;
     const uint32_t tid = threadIdx.x;
@@ -651,7 +819,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p_half(GemmArgs a) {
     }
     const uint32_t tn = tile / a.ntm, tm = tile - tn * a.ntm;
     acc16 acc[2][2];
-    tile_blocks<GEPI_SWIGLU>(a, a.seg[0], tn, tm, kb0, nkb, acc);
+    tile_blocks<WK, GEPI_SWIGLU>(a, a.seg[0], tn, tm, kb0, nkb, acc);
     if (half) {
         uint32_t *const cnt = a.sk_cnt + (hid >> 1);
         sk_store(a.sk_ws + (size_t)hid * kSkTileFloats, acc);
@@ -661,7 +829,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q8p_half(GemmArgs a) {
         sk_add(a.sk_ws + (size_t)(hid ^ 1u) * kSkTileFloats, acc);
         if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    swiglu_planes(a, tn, tm * kBM, acc);
+    swiglu_planes<WK>(a, tn, tm * kBM, acc);
 }
 
 // One thread per 32-byte quant row piece (tile, block b, row n) of the output.
@@ -697,21 +865,48 @@ __global__ __launch_bounds__(256) void k_repack_prefill(const uint8_t *raw, uint
         live ? (float)__builtin_bit_cast(_Float16, (unsigned short)(b[0] | (b[1] << 8))) : 0.f;
 }
 
-}  // namespace
-
-uint32_t gemm_q8p_tile_tokens() { return kBM; }
-
-bool gemm_q8p_eligible(const GemmArgs &a) {
-    if (a.wk != WT_Q8 || a.xf32 || !a.x_tiled || a.T == 0 || a.K % 32u) return false;
-    const uint32_t nseg = a.epi == GEPI_SWIGLU ? 1u : a.nseg;
-    for (uint32_t i = 0; i < nseg; ++i)
-        if (!a.seg[i].pq || !a.seg[i].pd || a.seg[i].bias) return false;   // no bias epilogue here
-    return true;
+// F16: one thread per 16-byte chunk (tile, block, row n, chunk) of the output; rows of
+// w0 (and w1, 32 by 32, when given) are row-major [rows][K].
+__global__ __launch_bounds__(256) void k_repack_prefill_f16(const __half *w0, const __half *w1, uint32_t rows,
+                                                            uint32_t K, uint64_t total, uint4 *out) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= total) return;
+    const uint32_t nb = K / 32u, n = (uint32_t)(i >> 2) & 127u;
+    const uint32_t blk = (uint32_t)((i >> 9) % nb), tile = (uint32_t)((i >> 9) / nb), r_out = 128u * tile + n;
+    const __half *w = w1 && ((r_out >> 5) & 1u) ? w1 : w0;
+    const uint32_t row = w1 ? 32u * (r_out >> 6) + (r_out & 31u) : r_out, c = ((uint32_t)i & 3u) ^ xperm(n);
+    out[i] = row < rows ? *reinterpret_cast<const uint4 *>(w + (size_t)row * K + 32u * blk + 8u * c)
+                        : make_uint4(0u, 0u, 0u, 0u);
 }
 
-uint64_t prefill_matrix_bytes(uint32_t rows_out, uint32_t K) {
+}  // namespace
+
+uint32_t gemm_pf_tile_tokens() { return kBM; }
+
+bool gemm_pf_eligible(const GemmArgs &a) {
+    if (a.xf32 || !a.x_tiled || a.T == 0 || a.K % 32u) return false;
+    const uint32_t nseg = a.epi == GEPI_SWIGLU ? 1u : a.nseg;
+    for (uint32_t i = 0; i < nseg; ++i) {
+        if (!a.seg[i].pq) return false;
+        if (a.wk == WT_Q8 && (!a.seg[i].pd || a.seg[i].bias)) return false;   // no bias epilogue for Q8_0
+    }
+    return a.wk == WT_Q8 ? a.x_block == 0u : a.wk == WT_F16;
+}
+
+uint64_t prefill_matrix_bytes(uint32_t wt, uint32_t rows_out, uint32_t K) {
     const uint64_t rp = (rows_out + 127u) / 128u * 128u;
-    return rp * K + rp * (K / 32u) * 4u;
+    return wt == WT_F16 ? rp * K * 2u : rp * K + rp * (K / 32u) * 4u;
+}
+
+int launch_repack_prefill_f16(hipStream_t s, const __half *w0, const __half *w1, uint32_t rows, uint32_t K, void *out) {
+    if (K % 32u || !w0 || !out || ((uintptr_t)w0 | (uintptr_t)w1) & 15u)
+        return fail(VX_ERR_INVALID_ARG, "prefill repack: K %% 32, buffers and their alignment");
+    if (w1 && rows % 32u) return fail(VX_ERR_INVALID_ARG, "prefill repack: interleaved rows %% 32");
+    const uint64_t rp = ((w1 ? 2u * rows : rows) + 127u) / 128u * 128u, total = rp * (K / 8u);
+    k_repack_prefill_f16<<<(unsigned)((total + 255u) / 256u), 256, 0, s>>>(w0, w1, rows, K, total,
+                                                                           static_cast<uint4 *>(out));
+    VX_LAUNCHED("k_repack_prefill_f16");
+    return VX_OK;
 }
 
 int launch_repack_prefill(hipStream_t s, const uint8_t *raw, uint32_t off0, uint32_t off1, uint32_t rows,
@@ -729,7 +924,7 @@ int launch_repack_prefill(hipStream_t s, const uint8_t *raw, uint32_t off0, uint
 
 // Called by launch_gemm with validated arguments; sets the tiling fields.
 // For GEPI_SWIGLU, seg[0].pq/pd hold the interleaved gate/up matrix.
-int launch_gemm_q8p(hipStream_t s, GemmArgs a) {
+int launch_gemm_pf(hipStream_t s, GemmArgs a) {
     uint32_t tiles = 0;
     if (a.epi == GEPI_SWIGLU) {
         tiles = (a.seg[0].rows + 63u) / 64u;
@@ -759,11 +954,17 @@ int launch_gemm_q8p(hipStream_t s, GemmArgs a) {
         // 1.25 tiles per CU, where the second-tile imbalance is worth removing
         // (from 1.5 up, two resident workgroups per CU do better).
         a.sk_per = (uint32_t)((tiles_all * nblk + a.sk_grid - 1u) / a.sk_grid);
-        if (a.sk_tail_first)
-            k_gemm_q8p_sk<true><<<a.sk_grid, 256, 0, s>>>(a);
-        else
-            k_gemm_q8p_sk<false><<<a.sk_grid, 256, 0, s>>>(a);
-        VX_LAUNCHED("k_gemm_q8p_sk");
+        if (a.wk == WT_F16) {
+            if (a.sk_tail_first)
+                k_gemm_pf_sk<WT_F16, true><<<a.sk_grid, 256, 0, s>>>(a);
+            else
+                k_gemm_pf_sk<WT_F16, false><<<a.sk_grid, 256, 0, s>>>(a);
+        } else if (a.sk_tail_first) {
+            k_gemm_pf_sk<WT_Q8, true><<<a.sk_grid, 256, 0, s>>>(a);
+        } else {
+            k_gemm_pf_sk<WT_Q8, false><<<a.sk_grid, 256, 0, s>>>(a);
+        }
+        VX_LAUNCHED("k_gemm_pf_sk");
         return VX_OK;
     }
     if (a.epi == GEPI_SWIGLU && a.sk_ws && a.sk_cnt && a.sk_grid >= 8u && a.sk_grid % 8u == 0u && a.o_tiled &&
@@ -774,8 +975,11 @@ int launch_gemm_q8p(hipStream_t s, GemmArgs a) {
         // most one per CU beside its whole tile; a part slot per half, a counter per
         // split tile.
         const uint32_t halves = 2u * (uint32_t)(tiles_all - a.sk_grid);
-        k_gemm_q8p_half<<<a.sk_grid + halves, 256, 0, s>>>(a);
-        VX_LAUNCHED("k_gemm_q8p_half");
+        if (a.wk == WT_F16)
+            k_gemm_pf_half<WT_F16><<<a.sk_grid + halves, 256, 0, s>>>(a);
+        else
+            k_gemm_pf_half<WT_Q8><<<a.sk_grid + halves, 256, 0, s>>>(a);
+        VX_LAUNCHED("k_gemm_pf_half");
         return VX_OK;
     }
     // 16-byte epilogue stores need every output row start and slab 16-byte aligned.
@@ -783,14 +987,22 @@ int launch_gemm_q8p(hipStream_t s, GemmArgs a) {
     if (a.epi != GEPI_SWIGLU)
         for (uint32_t i = 0; i < a.nseg; ++i)
             if (a.seg[i].rows % 4u || a.seg[i].ldo % 4u || reinterpret_cast<uintptr_t>(a.seg[i].out) % 16u) a.wide = 0;
-    switch (a.epi) {
-        case GEPI_STORE: k_gemm_q8p<GEPI_STORE><<<(unsigned)grid, 256, 0, s>>>(a); break;
-        case GEPI_RESIDUAL: k_gemm_q8p<GEPI_RESIDUAL><<<(unsigned)grid, 256, 0, s>>>(a); break;
-        case GEPI_SWIGLU: k_gemm_q8p<GEPI_SWIGLU><<<(unsigned)grid, 256, 0, s>>>(a); break;
-        default: return fail(VX_ERR_UNSUPPORTED, "gemm: epilogue %u", a.epi);
+#define VX_PF_CASE(WKV, EP, XB)                                               \
+    if (a.wk == WKV && a.epi == EP && (a.x_block != 0u) == XB) {              \
+        k_gemm_pf<WKV, EP, XB><<<(unsigned)grid, 256, 0, s>>>(a);             \
+        VX_LAUNCHED("k_gemm_pf");                                             \
+        return VX_OK;                                                         \
     }
-    VX_LAUNCHED("k_gemm_q8p");
-    return VX_OK;
+    VX_PF_CASE(WT_Q8, GEPI_STORE, false)
+    VX_PF_CASE(WT_Q8, GEPI_RESIDUAL, false)
+    VX_PF_CASE(WT_Q8, GEPI_SWIGLU, false)
+    VX_PF_CASE(WT_F16, GEPI_STORE, false)
+    VX_PF_CASE(WT_F16, GEPI_RESIDUAL, false)
+    VX_PF_CASE(WT_F16, GEPI_SWIGLU, false)
+    VX_PF_CASE(WT_F16, GEPI_STORE, true)
+    VX_PF_CASE(WT_F16, GEPI_RESIDUAL, true)
+#undef VX_PF_CASE
+    return fail(VX_ERR_UNSUPPORTED, "gemm: epilogue %u", a.epi);
 }
 
 }  // namespace vx

@@ -1421,7 +1421,7 @@ __global__ __launch_bounds__(256) void k_dense_attn_fused(DenseAttnArgs a) {
 }  // namespace
 
 // ------------------------------------------------------------------ launchers
-uint32_t gemm_tile_tokens(const GemmArgs &a) { return gemm_q8p_eligible(a) ? gemm_q8p_tile_tokens() : (uint32_t)GM; }
+uint32_t gemm_tile_tokens(const GemmArgs &a) { return gemm_pf_eligible(a) ? gemm_pf_tile_tokens() : (uint32_t)GM; }
 
 int launch_gemm(hipStream_t s, const GemmArgs &in) {
     GemmArgs a = in;
@@ -1460,7 +1460,7 @@ int launch_gemm(hipStream_t s, const GemmArgs &in) {
         if (a.wk == WT_Q8 ? (!g.qs || !g.d) : !g.w)
             return fail(VX_ERR_INVALID_ARG, "gemm: segment %u weight pointers missing", i);
     }
-    if (gemm_q8p_eligible(a)) return launch_gemm_q8p(s, a);
+    if (gemm_pf_eligible(a)) return launch_gemm_pf(s, a);
     if (gemm_skinny_eligible(a)) return launch_gemm_skinny(s, a);
     if (a.frag)
         return fail(VX_ERR_UNSUPPORTED, "gemm: fragment-layout operands need the short-batch kernel (F16, T <= 128, "

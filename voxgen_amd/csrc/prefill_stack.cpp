@@ -76,6 +76,53 @@ int prefill_stack_check(const PrefillStack &p) {
     return VX_OK;
 }
 
+int prefill_stack_weights(vx_ctx *ctx, const StackLayer *layers, uint32_t n_layers, uint32_t nH, uint32_t nF,
+                          uint32_t nKV, std::vector<StackPrefillWeights> *pw, vx_buf **arena) {
+    pw->clear();
+    if (!n_layers || nH % 32u || nF % 32u) return VX_OK;
+    const uint32_t wt = layers[0].q.wt;
+    for (uint32_t l = 0; l < n_layers; ++l) {
+        const StackLayer &L = layers[l];
+        for (const WRef *w : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
+            if (w->wt != wt || (wt == WT_Q8 ? w->dtype != VX_DTYPE_Q8_0 || !w->raw
+                                            : wt != WT_F16 || !w->ptr || ((uintptr_t)w->ptr & 15u)))
+                return VX_OK;
+    }
+    const uint64_t per_layer = prefill_matrix_bytes(wt, nH, nH) + 2u * prefill_matrix_bytes(wt, nKV, nH) +
+                               prefill_matrix_bytes(wt, nH, nH) + prefill_matrix_bytes(wt, 2u * nF, nH) +
+                               prefill_matrix_bytes(wt, nH, nF) + 6u * 256u;
+    const int st_alloc = vx_alloc(ctx, per_layer * n_layers, arena);
+    if (st_alloc == VX_ERR_OOM && wt == WT_F16) return VX_OK;   // the general GEMM reads the model's own rows
+    VX_CHECK(st_alloc);
+    uint8_t *cur = static_cast<uint8_t *>((*arena)->ptr);
+    hipStream_t s = ctx->stream;
+    auto place = [&](PrefillMatrix &pm, const WRef &w0, const WRef *w1, uint32_t rows, uint32_t K) {
+        const uint32_t rows_out = w1 ? 2u * rows : rows;
+        pm.rows_pad = (rows_out + 127u) / 128u * 128u;
+        pm.q = reinterpret_cast<int8_t *>(cur);
+        pm.d = wt == WT_Q8 ? reinterpret_cast<float *>(cur + (uint64_t)pm.rows_pad * K) : nullptr;
+        cur += (prefill_matrix_bytes(wt, rows_out, K) + 255u) / 256u * 256u;
+        return wt == WT_Q8 ? launch_repack_prefill(s, w0.raw, w0.raw_offset, w1 ? w1->raw_offset : 0u, rows, K,
+                                                   w1 ? 1 : 0, pm.q, pm.d)
+                           : launch_repack_prefill_f16(s, static_cast<const __half *>(w0.ptr),
+                                                       w1 ? static_cast<const __half *>(w1->ptr) : nullptr, rows, K,
+                                                       pm.q);
+    };
+    pw->resize(n_layers);
+    for (uint32_t l = 0; l < n_layers; ++l) {
+        const StackLayer &L = layers[l];
+        StackPrefillWeights &P = (*pw)[l];
+        int st = VX_OK;
+        if ((st = place(P.q, L.q, nullptr, nH, nH)) || (st = place(P.k, L.k, nullptr, nKV, nH)) ||
+            (st = place(P.v, L.v, nullptr, nKV, nH)) || (st = place(P.o, L.o, nullptr, nH, nH)) ||
+            (st = place(P.gu, L.gate, &L.up, nF, nH)) || (st = place(P.down, L.down, nullptr, nH, nF))) {
+            pw->clear();
+            return st;
+        }
+    }
+    return VX_OK;
+}
+
 int prefill_stack_alloc(vx_ctx *ctx, uint32_t cap, uint32_t nH, uint32_t nF, uint32_t nKV, StackWork *w) {
     if (w->cap) return VX_OK;
     const uint64_t H = nH, F = nF, KV = nKV, T = cap;
@@ -125,8 +172,8 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
     if (T == 0 || T > w.cap) return fail(VX_ERR_INVALID_ARG, "prefill chunk of %u rows (capacity %u)", T, w.cap);
     // The deep-pipelined GEMM takes the prefill-layout weights and tiled planes,
     // from one full 128-token tile up.
-    const bool tiled = p.pw != nullptr && T >= gemm_q8p_tile_tokens();
-    const uint32_t tt = tiled ? gemm_q8p_tile_tokens() : 64u;
+    const bool tiled = p.pw != nullptr && T >= gemm_pf_tile_tokens();
+    const uint32_t tt = tiled ? gemm_pf_tile_tokens() : 64u;
     const uint32_t ks_qkv = pick_split(p.ctx, tt, (nH + 127u) / 128u + 2u * ((nKV + 127u) / 128u), T, nH);
     const uint32_t ks_o = pick_split(p.ctx, tt, (nH + 127u) / 128u, T, nH);
     const uint32_t ks_down = pick_split(p.ctx, tt, (nH + 127u) / 128u, T, nF);

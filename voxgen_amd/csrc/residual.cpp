@@ -75,6 +75,8 @@ struct vx_residual {
     // activations, the fusion input [cap][2H] (right half kept zero) and the
     // BaseLM output rows of a cross-engine chunk [cap][H].
     StackWork pf;
+    std::vector<StackPrefillWeights> pw;   // the layers' prefill-layout weights ...
+    vx_buf *pw_arena = nullptr;            // ... and their memory
     vx_buf *fuse_x = nullptr, *rows = nullptr;
 };
 
@@ -160,6 +162,9 @@ void free_all(vx_residual *e) {
         if (g.g) vx_graph_free(e->ctx, g.g);
     e->graphs.clear();
     prefill_stack_free(e->ctx, &e->pf);
+    e->pw.clear();
+    if (e->pw_arena) vx_free(e->ctx, e->pw_arena);
+    e->pw_arena = nullptr;
     for (vx_buf **b : {&e->fuse_x, &e->rows})
         if (*b) {
             vx_free(e->ctx, *b);
@@ -577,6 +582,9 @@ int ensure_prefill_work(vx_residual *e) {
     if (e->pf.cap) return VX_OK;
     const vx_acoustic_config &c = e->cfg;
     const uint32_t cap = std::min<uint32_t>(kPrefillChunk, c.active_context_length);
+    if (!e->pw_arena)
+        VX_CHECK(prefill_stack_weights(e->ctx, e->layers.data(), c.residual_block_count, c.embedding_length,
+                                       c.feed_forward_length, c.kv_dim, &e->pw, &e->pw_arena));
     VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
     VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.fusion_input_dim * 4u, &e->fuse_x));
     VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.embedding_length * 4u, &e->rows));
@@ -599,6 +607,7 @@ PrefillStack make_stack(vx_residual *e) {
     p.eps = c.rms_epsilon;
     p.residual_scale = c.residual_scale;
     p.layers = e->layers.data();
+    p.pw = e->pw.empty() ? nullptr : e->pw.data();
     p.rope = false;
     p.kc = H(e->kv_k);
     p.vc = H(e->kv_v);

@@ -360,8 +360,8 @@ enum GemmEpilogue : uint32_t {
 struct GemmSeg {                    // one weight matrix covering part of N
     const int8_t *qs = nullptr;     // Q8_0: repacked quants (WRef::ptr) ...
     const __half *d = nullptr;      // ... and scales (WRef::d)
-    const int8_t *pq = nullptr;     // Q8_0 in the prefill-GEMM layout (PrefillMatrix), nullable ...
-    const float *pd = nullptr;      // ... and its f32 scales
+    const int8_t *pq = nullptr;     // Q8_0 or F16 in the prefill-GEMM layout (PrefillMatrix), nullable ...
+    const float *pd = nullptr;      // ... and the f32 scales of Q8_0
     const __half *w = nullptr;      // F16: [rows][K]
     uint32_t rows = 0;
     uint32_t tile0 = 0;             // set by launch_gemm
@@ -386,6 +386,11 @@ struct GemmArgs {
     uint32_t ksplit = 1;
     uint32_t ntn = 0, ntm = 0;                  // set by launch_gemm
     uint32_t x_tiled = 0;           // 1: xh/xl are in the tiled plane layout (tiled_plane_index)
+    // F16 weights in the prefill layout only: with x_block set (bytes between 32-column
+    // blocks) the planes are block-major, [block][row][32] with the rows' chunks permuted
+    // as in the tiled layout, and rows past T of the last 128-row tile may be read; the
+    // first x_shift blocks of K are read one row earlier (row -1 is the row before xh).
+    uint32_t x_block = 0, x_shift = 0;
     uint32_t o_tiled = 0;           // 1: GEPI_SWIGLU writes oh/ol in the tiled plane layout
     // GEPI_RESIDUAL with ksplit > 1 on the prefill-layout kernel: when set, split
     // s stores scale * (its partial product) to ws + s * ws_stride ([T][ldo]) with
@@ -475,19 +480,22 @@ __host__ __device__ __forceinline__ size_t tiled_plane_index(uint32_t t, uint32_
 // With interleave, rows come from two matrices (gate, up) as 32 of the first,
 // the same 32 of the second, and so on, the row order of a SwiGLU tile.
 // Padding rows hold q = 0 (byte 0x80) with scale 0.
+// F16 weights (q as bytes, no d): pieces [rows_pad/128][K/32][128][32] f16, the 16-byte
+// chunks of a row permuted as in tiled_plane_index; padding rows are zero.
 struct PrefillMatrix {
     int8_t *q = nullptr;
     float *d = nullptr;
     uint32_t rows_pad = 0;
 };
-uint64_t prefill_matrix_bytes(uint32_t rows_out, uint32_t K);   // q + d, rows padded to 128
+uint64_t prefill_matrix_bytes(uint32_t wt, uint32_t rows_out, uint32_t K);   // q (+ d), rows padded to 128
 int launch_repack_prefill(hipStream_t s, const uint8_t *raw, uint32_t off0, uint32_t off1, uint32_t rows,
                           uint32_t K, int interleave, int8_t *q, float *d);
-// The deep-pipelined Q8_0 x hi/lo-plane GEMM (kernels_gemm.hip), which
+int launch_repack_prefill_f16(hipStream_t s, const __half *w0, const __half *w1, uint32_t rows, uint32_t K, void *out);
+// The deep-pipelined Q8_0 or F16 x hi/lo-plane GEMM (kernels_gemm.hip), which
 // launch_gemm picks when the weights have the prefill layout and X is tiled.
-bool gemm_q8p_eligible(const GemmArgs &a);
-uint32_t gemm_q8p_tile_tokens();
-int launch_gemm_q8p(hipStream_t s, GemmArgs a);
+bool gemm_pf_eligible(const GemmArgs &a);
+uint32_t gemm_pf_tile_tokens();
+int launch_gemm_pf(hipStream_t s, GemmArgs a);
 // Tokens per workgroup tile of the kernel launch_gemm picks for these arguments.
 uint32_t gemm_tile_tokens(const GemmArgs &a);
 
@@ -550,7 +558,7 @@ struct StackLayer {
     WRef q, k, v, o, gate, up, down;
     const float *attn_norm = nullptr, *ffn_norm = nullptr;
 };
-struct StackPrefillWeights {        // Q8_0 projections in the prefill-GEMM layout
+struct StackPrefillWeights {        // Q8_0 or F16 projections in the prefill-GEMM layout
     PrefillMatrix q, k, v, o, gu, down;
 };
 struct StackWork {                  // activations of one chunk of rows (cap rows)
@@ -569,7 +577,7 @@ struct PrefillStack {
     uint32_t nH = 0, nF = 0, nKV = 0, q_heads = 0, kv_heads = 0, head_dim = 0, context = 0, n_layers = 0;
     float eps = 0.f, residual_scale = 1.f;
     const StackLayer *layers = nullptr;
-    const StackPrefillWeights *pw = nullptr;   // nullable: per-layer prefill-layout Q8_0 weights
+    const StackPrefillWeights *pw = nullptr;   // nullable: per-layer prefill-layout weights
     bool rope = true;
     const float *rope_factors = nullptr;
     float theta = 10000.f, rope_scaling = 1.f;
@@ -578,6 +586,12 @@ struct PrefillStack {
     uint32_t schedule = VX_PREFILL_AUTO;       // gate/up GEMM schedule (VX_PREFILL_*)
 };
 int prefill_stack_check(const PrefillStack &p);
+// Repacks every layer's projections into the prefill-GEMM layout (53 MB a layer of
+// Q8_0, 94 MB of F16 at the VoxCPM2 geometry). Leaves *pw empty, so that prefill uses
+// the general GEMM, where the projections are not all Q8_0 or all F16, a width does
+// not fit, or the device has no room for the F16 copy.
+int prefill_stack_weights(vx_ctx *ctx, const StackLayer *layers, uint32_t n_layers, uint32_t nH, uint32_t nF,
+                          uint32_t nKV, std::vector<StackPrefillWeights> *pw, vx_buf **arena);
 int prefill_stack_alloc(vx_ctx *ctx, uint32_t cap, uint32_t nH, uint32_t nF, uint32_t nKV, StackWork *w);
 void prefill_stack_free(vx_ctx *ctx, StackWork *w);
 // The layers over rows 0..T-1 of work->h at positions pos0..pos0+T-1 (K/V rows
