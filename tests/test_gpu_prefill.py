@@ -200,6 +200,33 @@ def test_batched_prefill_f16_tiles(ctx, n):
     model.free()
 
 
+@pytest.mark.parametrize("weights", ["q8_0", "f16"])
+def test_batched_prefill_short_chunks(ctx, weights):
+    """Chunks below one 128-token tile at both sides of the 16-row fragment edges, one
+    after another in one cache: 16 and 17 rows, 1, 33, 64, 112 and 127."""
+    cfg = synth.baselm_config(layers=1, vocab=512, context_length=32768, active_context=512)
+    m = synth.build_baselm(cfg, seed=0x5EED0130, weight_type=weights)
+    model = Model(ctx, m.data, m.tensors)
+    sizes = [16, 17, 1, 33, 64, 112, 127]
+    toks = [int(t) for t in synth.uniform_u32(sum(sizes), 0x5EED0131, cfg["vocab_size"])]
+    o = oracle_of(m, cfg)
+    eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False)
+    done = 0
+    for n in sizes:
+        print(f"short chunk {weights} n={n} at {done}", flush=True)
+        eng.prefill_tokens_batched(toks[done:done + n])
+        for p in range(done, done + n):
+            o.decode_token(toks[p], p)
+        done += n
+        assert rel_l2(eng.output(), o.norm) < 1e-3
+    for name, ref in (("kv_k", o.kv_k), ("kv_v", o.kv_v)):
+        rows = kv_rows(eng, name, 1, 512)
+        assert rel_l2(f16(rows[0, :done]), f16(ref.reshape(512, 256)[:done])) < 1e-3, name
+        assert np.all(rows[:, done:] == 0)
+    eng.close()
+    model.free()
+
+
 def test_batched_prefill_errors(ctx, small):
     cfg, m, model = small
     eng = BaseLmEngine(ctx, model, dict(cfg, active_context_length=64), exec_mode="graph", strict_geometry=False)

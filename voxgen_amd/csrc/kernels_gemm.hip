@@ -925,6 +925,7 @@ int launch_repack_prefill(hipStream_t s, const uint8_t *raw, uint32_t off0, uint
 // Called by launch_gemm with validated arguments; sets the tiling fields.
 // For GEPI_SWIGLU, seg[0].pq/pd hold the interleaved gate/up matrix.
 int launch_gemm_pf(hipStream_t s, GemmArgs a) {
+    if (a.T < kBM && gemm_ps_eligible(a)) return launch_gemm_ps(s, a);
     uint32_t tiles = 0;
     if (a.epi == GEPI_SWIGLU) {
         tiles = (a.seg[0].rows + 63u) / 64u;

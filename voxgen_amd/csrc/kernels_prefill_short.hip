@@ -1,0 +1,292 @@
+// Projections of a short prefill chunk on gfx950 (T <= 128 rows, usually a prompt of
+// a few words or the last chunk of a long one): Q8_0 or F16 weights in the prefill
+// layout, X as tiled hi/lo planes, the arithmetic of k_gemm_pf (kernels_gemm.hip):
+//   C[t][n] = sum_b d[n][b] * sum_{k in b} q * (x_hi + x_lo)
+//
+// At so few rows a launch is bound by how fast a CU takes operands in: the weights once
+// (25 MB of Q8_0 for gate/up at the VoxCPM2 geometry, 5 us at the copy rate) and X, from
+// the L2, by every workgroup. So the work is split for bytes in flight:
+//   * a workgroup owns 32 weight rows (two 16-row fragments), or 32 gate rows and their
+//     up rows, and every token; its waves take interleaved 32-column blocks of its K
+//     range, and each keeps DEPTH blocks of operands in flight in registers;
+//   * both stored layouts are read as they are: 16 rows of one 32-column block are 512
+//     contiguous bytes of quants (1 KB of f16), permuted only inside, which is one
+//     operand of v_mfma_f32_16x16x32_f16 with the lane's chunk picked by the
+//     permutation. A Q8_0 block is one MFMA step, so its products start from zero and
+//     enter the sums scaled by the block's f32 scale;
+//   * the partial tiles of the waves meet in LDS; split K leaves slabs that the consumer
+//     sums.
+// Against k_gemm (64-token tiles, at most four splits, atomic sums) four Q8_0 layers
+// took on MI355X at 2 / 16 / 37 / 64 / 127 rows 381 / 409 / 431 / 435 / 448 ->
+// 193 / 207 / 268 / 308 / 429 us, F16 381 / 406 / 431 / 434 / 448 -> 206 / 221 / 281 /
+// 318 / 427. Gate/up at 37 rows: 17 us with 64 rows a workgroup, 22 with 32 (every
+// workgroup reads all of X), 26 with 128 (too few workgroups); eight waves: 18. The
+// split projections are the other way round (their K ranges are short): 9 us with 32
+// rows, 11 with 64; one workgroup per CU beat two (X again) by 10%.
+#include "vx_internal.h"
+
+namespace vx {
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+
+constexpr int NW = 4;             // waves per workgroup
+constexpr uint32_t kPiece = 128;  // weight rows and tokens of a stored tile
+
+__device__ __forceinline__ uint32_t xperm(uint32_t t) { return ((t >> 1) ^ (t >> 3)) & 3u; }
+__device__ __forceinline__ uint32_t wperm(uint32_t n) { return ((n >> 2) ^ (n >> 4)) & 3u; }
+
+// Eight stored quants u = q + 128 -> exact f16 q: 0x6400 | u is 1024 + u.
+__device__ __forceinline__ h8 widen(u2v u) {
+    const h2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+    u4v r;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u[i], 0x04010400u);
+        const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u[i], 0x04030402u);
+        r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, lo) - bias);
+        r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, hi) - bias);
+    }
+    return __builtin_bit_cast(h8, r);
+}
+
+__device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+template <int WK, int MT, int NF>
+struct Ops {
+    u4v xh[MT], xl[MT];
+    u4v w[NF];
+};
+template <int MT, int NF>
+struct Ops<WT_Q8, MT, NF> {
+    u4v xh[MT], xl[MT];
+    u2v w[NF];
+    float d[NF];
+};
+
+// Grid: a.ntn row tiles x a.ksplit K ranges.
+template <int WK, int EPI, int MT>
+__global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
+    constexpr int NF = EPI == GEPI_SWIGLU ? 4 : 2;
+    constexpr uint32_t kRows = 16u * NF;   // weight rows of the workgroup
+    __shared__ f4 red[NW / 2][MT][NF][64];   // partial tiles [wave][token fragment][row fragment][lane]
+    constexpr int DEPTH = MT <= 4 ? 4 : 3;
+    const uint32_t tile = blockIdx.x % a.ntn, ks = blockIdx.x / a.ntn;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r16 = lane & 15u, g = lane >> 4;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t seg = 0;
+    if constexpr (EPI != GEPI_SWIGLU) {
+        while (seg + 1 < a.nseg && tile >= a.seg[seg + 1].tile0) ++seg;
+    }
+    const GemmSeg &sg = a.seg[seg];
+    const uint32_t nblk = a.K >> 5;
+    // A gate/up tile is stored as 32 gate rows (fragments 0 and 1) and their up rows; padding rows of the last tile are stored as zeros.
+    const uint8_t *wr[NF];
+    const float *dr[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        const uint32_t r0 = kRows * (tile - sg.tile0) + 16u * f;
+        const uint32_t n = (r0 & (kPiece - 1u)) + r16;
+        const size_t piece = (size_t)(r0 / kPiece) * nblk;
+        const uint8_t *base = reinterpret_cast<const uint8_t *>(sg.pq);
+        wr[f] = WK == WT_Q8 ? base + piece * (kPiece * 32u) + n * 32u + 8u * (g ^ wperm(n))
+                            : base + piece * (kPiece * 64u) + n * 64u + 16u * (g ^ xperm(n));
+        dr[f] = WK == WT_Q8 ? sg.pd + piece * kPiece + n : nullptr;
+    }
+    const uint8_t *const xh = reinterpret_cast<const uint8_t *>(a.xh), *const xl = reinterpret_cast<const uint8_t *>(a.xl);
+    uint32_t xo[MT];   // rows past T of the 128-row tile are multiplied and never stored
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const uint32_t t = 16u * mt + r16;
+        xo[mt] = t * 64u + 16u * (g ^ xperm(t));
+    }
+    const uint32_t s0 = ks * nblk / a.ksplit, s1 = (ks + 1u) * nblk / a.ksplit;
+    const int n_it = s0 + wv < s1 ? (int)((s1 - s0 - wv + NW - 1u) / NW) : 0;
+
+    f4 acc[MT][NF];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) acc[mt][f] = f4{0.f, 0.f, 0.f, 0.f};
+    Ops<WK, MT, NF> ring[DEPTH];
+    auto load = [&](Ops<WK, MT, NF> &o, int i) {
+        const size_t blk = s0 + wv + NW * (uint32_t)i;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            if constexpr (WK == WT_Q8) {
+                o.w[f] = __builtin_nontemporal_load(reinterpret_cast<const u2v *>(wr[f] + blk * (kPiece * 32u)));
+                o.d[f] = __builtin_nontemporal_load(dr[f] + blk * kPiece);
+            } else {
+                o.w[f] = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(wr[f] + blk * (kPiece * 64u)));
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            o.xh[mt] = *reinterpret_cast<const u4v *>(xh + blk * (kPiece * 64u) + xo[mt]);
+            o.xl[mt] = *reinterpret_cast<const u4v *>(xl + blk * (kPiece * 64u) + xo[mt]);
+        }
+    };
+    auto mma = [&](const Ops<WK, MT, NF> &o) {
+        h8 b[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            if constexpr (WK == WT_Q8)
+                b[f] = widen(o.w[f]);
+            else
+                b[f] = __builtin_bit_cast(h8, o.w[f]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const h8 ah = __builtin_bit_cast(h8, o.xh[mt]), al = __builtin_bit_cast(h8, o.xl[mt]);
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                if constexpr (WK == WT_Q8) {
+                    const f4 p = mfma16(al, b[f], mfma16(ah, b[f], f4{0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[mt][f][r] = fmaf(o.d[f], p[r], acc[mt][f][r]);
+                } else {
+                    acc[mt][f] = mfma16(al, b[f], mfma16(ah, b[f], acc[mt][f]));
+                }
+            }
+        }
+    };
+    // Loads are unconditional (past the wave's last block they repeat it): under a
+    // branch the compiler would wait for everything in flight before each MFMA.
+    if (n_it > 0) {
+#pragma unroll
+        for (int u = 0; u < DEPTH - 1; ++u) load(ring[u], min(u, n_it - 1));
+        for (int it = 0; it < n_it; it += DEPTH) {
+#pragma unroll
+            for (int u = 0; u < DEPTH; ++u) {
+                const int i = it + u;
+                load(ring[(u + DEPTH - 1) % DEPTH], min(i + DEPTH - 1, n_it - 1));
+                if (i < n_it) mma(ring[u]);
+            }
+        }
+    }
+    // Lane (r16, g) holds tokens 4g .. 4g + 3 of its token fragment for weight row r16.
+    if (wv >= NW / 2) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) red[wv - NW / 2][mt][f][lane] = acc[mt][f];
+    }
+    __syncthreads();
+    if (wv < NW / 2) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) red[wv][mt][f][lane] += acc[mt][f];
+    }
+    __syncthreads();
+    auto part = [&](uint32_t tok, uint32_t f, uint32_t n) {
+        const uint32_t ln = n + 16u * ((tok >> 2) & 3u), mt = tok >> 4, r = tok & 3u;
+        float v = red[0][mt][f][ln][r];
+#pragma unroll
+        for (int w = 1; w < NW / 2; ++w) v += red[w][mt][f][ln][r];
+        return v;
+    };
+    if constexpr (EPI == GEPI_SWIGLU) {
+        constexpr uint32_t kPairs = kRows / 2u;
+        for (uint32_t o = tid; o < kPairs * 16u * MT; o += 64u * NW) {
+            const uint32_t nl = o % kPairs, tok = o / kPairs, row = kPairs * tile + nl, f = nl >> 4, n = nl & 15u;
+            if (tok >= a.T || row >= sg.rows) continue;
+            const float gv = part(tok, f, n), uv = part(tok, f + 2u, n);
+            const float v = gv / (1.0f + expf(-gv)) * uv;   // matvec_swiglu.comp:67
+            const size_t po = tiled_plane_index(tok, row, a.ldp);
+            const _Float16 hv = (_Float16)v;
+            a.oh[po] = __builtin_bit_cast(__half, hv);
+            a.ol[po] = __builtin_bit_cast(__half, (_Float16)(v - (float)hv));
+        }
+    } else {
+        const bool slab = a.ksplit > 1u;
+        float *const out = EPI == GEPI_STORE ? sg.out + (slab ? ks * a.ws_stride : 0u)
+                           : slab            ? a.ws + ks * a.ws_stride
+                                             : sg.out;
+        for (uint32_t o = tid; o < kRows * 16u * MT; o += 64u * NW) {
+            const uint32_t nl = o % kRows, tok = o / kRows, row = kRows * (tile - sg.tile0) + nl;
+            if (tok >= a.T || row >= sg.rows) continue;
+            float v = part(tok, nl >> 4, nl & 15u);
+            if constexpr (WK == WT_F16) {
+                if (sg.bias && ks == 0u)
+                    v += sg.bias_dtype == 0 ? static_cast<const float *>(sg.bias)[row]
+                                            : __half2float(static_cast<const __half *>(sg.bias)[row]);
+            }
+            float *const dst = out + (size_t)tok * sg.ldo + row;
+            if constexpr (EPI == GEPI_STORE)
+                *dst = v * a.alpha;
+            else
+                *dst = slab ? v * a.scale : *dst + v * a.scale;
+        }
+    }
+}
+
+template <int WK, int EPI>
+int launch_ps(hipStream_t s, const GemmArgs &a, uint32_t grid) {
+    switch ((a.T + 15u) / 16u) {
+#define VX_PS_CASE(M)                                           \
+    case M:                                                     \
+        k_gemm_ps<WK, EPI, M><<<grid, 64 * NW, 0, s>>>(a);  \
+        break;
+        VX_PS_CASE(1)
+        VX_PS_CASE(2)
+        VX_PS_CASE(3)
+        VX_PS_CASE(4)
+        VX_PS_CASE(5)
+        VX_PS_CASE(6)
+        VX_PS_CASE(7)
+        VX_PS_CASE(8)
+#undef VX_PS_CASE
+        default: return fail(VX_ERR_UNSUPPORTED, "short prefill gemm: %u rows", a.T);
+    }
+    VX_LAUNCHED("k_gemm_ps");
+    return VX_OK;
+}
+
+}  // namespace
+
+bool gemm_ps_eligible(const GemmArgs &a) {
+    if (a.T == 0 || a.T > kPiece || a.x_block) return false;
+    if (a.epi == GEPI_SWIGLU) return a.o_tiled && a.oh && !a.seg[0].out && a.seg[0].rows % 32u == 0u && a.ldp % 32u == 0u;
+    if (a.epi == GEPI_STORE) return a.ksplit <= 1u || a.split_store;
+    return a.ksplit <= 1u || a.ws != nullptr;
+}
+
+// Called by launch_gemm_pf with arguments it has validated; sets the tiling fields.
+int launch_gemm_ps(hipStream_t s, GemmArgs a) {
+    const uint32_t kRows = a.epi == GEPI_SWIGLU ? 64u : 32u;
+    uint32_t tiles = 0;
+    if (a.epi == GEPI_SWIGLU) {
+        tiles = (2u * a.seg[0].rows + kRows - 1u) / kRows;
+    } else {
+        for (uint32_t i = 0; i < a.nseg; ++i) {
+            a.seg[i].tile0 = tiles;
+            tiles += (a.seg[i].rows + kRows - 1u) / kRows;
+        }
+    }
+    if (a.ksplit == 0) a.ksplit = 1;
+    if (a.ksplit > a.K / 32u) a.ksplit = a.K / 32u;
+    a.ntn = tiles;
+    a.ntm = 1;
+    const uint64_t grid = (uint64_t)tiles * a.ksplit;
+    if (grid == 0) return VX_OK;
+    if (grid > 0x7fffffffull) return fail(VX_ERR_UNSUPPORTED, "short prefill gemm: grid too large");
+#define VX_PS_KIND(WKV, EP) \
+    if (a.wk == WKV && a.epi == EP) return launch_ps<WKV, EP>(s, a, (uint32_t)grid);
+    VX_PS_KIND(WT_Q8, GEPI_STORE)
+    VX_PS_KIND(WT_Q8, GEPI_RESIDUAL)
+    VX_PS_KIND(WT_Q8, GEPI_SWIGLU)
+    VX_PS_KIND(WT_F16, GEPI_STORE)
+    VX_PS_KIND(WT_F16, GEPI_RESIDUAL)
+    VX_PS_KIND(WT_F16, GEPI_SWIGLU)
+#undef VX_PS_KIND
+    return fail(VX_ERR_UNSUPPORTED, "gemm: epilogue %u", a.epi);
+}
+
+}  // namespace vx

@@ -38,6 +38,13 @@ uint32_t pick_split(const vx_ctx *ctx, uint32_t tt, uint32_t n_tiles, uint32_t T
     return std::max<uint32_t>(ks, 1u);
 }
 
+// The same below a whole token tile (k_gemm_ps, 32-row tiles): every workgroup reads
+// all of X, so one per CU (two were 10% slower at 37 rows), four blocks or more each.
+uint32_t pick_split_short(const vx_ctx *ctx, uint32_t n_tiles, uint32_t K) {
+    const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
+    return std::max<uint32_t>(1u, std::min({cus / n_tiles, K / 128u, kPrefillMaxSplit}));
+}
+
 GemmSeg gemm_seg(const WRef &w, uint32_t rows, float *out, uint32_t ldo) {
     GemmSeg g;
     if (w.wt == WT_Q8) {
@@ -170,13 +177,16 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
     const StackWork &w = *p.work;
     const uint32_t nH = p.nH, nF = p.nF, nKV = p.nKV;
     if (T == 0 || T > w.cap) return fail(VX_ERR_INVALID_ARG, "prefill chunk of %u rows (capacity %u)", T, w.cap);
-    // The deep-pipelined GEMM takes the prefill-layout weights and tiled planes,
-    // from one full 128-token tile up.
-    const bool tiled = p.pw != nullptr && T >= gemm_pf_tile_tokens();
+    // The prefill-layout weights and tiled planes go to the deep-pipelined GEMM from one
+    // full 128-token tile up and to the short-chunk one below.
+    const bool tiled = p.pw != nullptr;
+    const bool is_short = tiled && T < gemm_pf_tile_tokens();
     const uint32_t tt = tiled ? gemm_pf_tile_tokens() : 64u;
-    const uint32_t ks_qkv = pick_split(p.ctx, tt, (nH + 127u) / 128u + 2u * ((nKV + 127u) / 128u), T, nH);
-    const uint32_t ks_o = pick_split(p.ctx, tt, (nH + 127u) / 128u, T, nH);
-    const uint32_t ks_down = pick_split(p.ctx, tt, (nH + 127u) / 128u, T, nF);
+    auto split = [&](uint32_t rows, uint32_t kv_rows, uint32_t K) {
+        if (is_short) return pick_split_short(p.ctx, (rows + 31u) / 32u + 2u * ((kv_rows + 31u) / 32u), K);
+        return pick_split(p.ctx, tt, (rows + 127u) / 128u + 2u * ((kv_rows + 127u) / 128u), T, K);
+    };
+    const uint32_t ks_qkv = split(nH, nKV, nH), ks_o = split(nH, 0, nH), ks_down = split(nH, 0, nF);
     // Split residual projections on the tiled path leave their partials in
     // the workspace; the next rmsnorm adds them to h (no atomics in the GEMM epilogue).
     const uint64_t ws_stride = (uint64_t)w.cap * nH;

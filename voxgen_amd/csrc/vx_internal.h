@@ -496,6 +496,10 @@ int launch_repack_prefill_f16(hipStream_t s, const __half *w0, const __half *w1,
 bool gemm_pf_eligible(const GemmArgs &a);
 uint32_t gemm_pf_tile_tokens();
 int launch_gemm_pf(hipStream_t s, GemmArgs a);
+// The same operands at T <= 128 rows (kernels_prefill_short.hip), which launch_gemm_pf
+// picks below a whole token tile.
+bool gemm_ps_eligible(const GemmArgs &a);
+int launch_gemm_ps(hipStream_t s, GemmArgs a);
 // Tokens per workgroup tile of the kernel launch_gemm picks for these arguments.
 uint32_t gemm_tile_tokens(const GemmArgs &a);
 
