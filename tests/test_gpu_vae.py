@@ -116,6 +116,27 @@ def test_long_decode_tiles(ctx, frames):
     model.free()
 
 
+@pytest.mark.parametrize("dd,frames", [(512, 12), (1024, 20), (2048, 12), (2048, 44)])
+def test_decode_plane_gemms(ctx, dd, frames):
+    """Up-convolutions and wide residual units over planes at ragged row counts: small
+    tiles (96 rows; 12 rows from the latents), 128 x 128 tiles with a last partial one
+    (2112 rows), two K ranges (352 rows of 1024 channels), the one-pass unit of 512
+    channels from 2048 rows on, and 16-channel stages behind the planes (512). Whole
+    decode up to 20 frames; the first 4 frames of a causal decode beyond."""
+    print(f"vae plane gemms decoder_dim {dd} frames {frames}", flush=True)
+    cfg, model, eng, lat, o = engine_case(ctx, dd, frames, 0x5EED0550 + dd + frames)
+    head = frames if frames <= 20 else 4
+    want = o.decode(lat[:head * 64])
+    for _ in range(2):
+        wave = eng.decode_latents(lat)[1]
+        assert rel_l2(wave[:want.size], want) < 1e-5   # two f16 planes: 22 bits of x
+    if head < frames:   # the last 20 frames have their whole history in a decode of 40
+        tail = eng.decode_latents(lat[-40 * 64:])[1]
+        assert rel_l2(wave[-20 * 1920:], tail[-20 * 1920:]) < 1e-5
+    eng.close()
+    model.free()
+
+
 def test_decode_large_snake_arguments(ctx):
     """Snake arguments past the reduced-range sine (|a x| >= 32768): with alphas of
     60000 the term sin(a x)^2 / a is below 2e-5, so the wave has to match the oracle

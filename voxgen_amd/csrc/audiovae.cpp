@@ -6,13 +6,15 @@
 //   model.0   depthwise k=7 causal conv                  k_vae_dwconv_fm
 //   model.1   1x1 conv latent -> decoder_dim             k_vae_linear_fm (K = latent)
 //   6 stages  scale/bias + snake + ConvTranspose1d(k=2s, stride s):
-//               P = pre(x) behind a zero row             k_vae_pre_fm, or the last unit before
+//               P = pre(x) behind a zero row,           k_vae_pre_planes, or the epilogue of
+//               as hi/lo f16 planes                     the last unit before
 //               one GEMM over rows [P[j-1] | P[j]],
-//               N = s * Cout, K = 2 Cin                  k_gemm (repacked weights)
+//               N = s * Cout, K = 2 Cin                  k_gemm_pf / k_gemm_ps
 //             3 residual units (dilation 1, 3, 9):
-//               32 to 256 channels: one pass             k_vae_unit
-//               else snake -> depthwise k=7 -> snake     k_vae_dwconv_fm
-//               and x += 1x1 conv + bias                 k_gemm residual (or k_vae_linear_fm)
+//               32 to 512 channels: one pass             k_vae_unit
+//               else snake -> depthwise k=7 -> snake     k_vae_dw7_fm / k_vae_dwconv_*
+//               and x += 1x1 conv + bias                 k_gemm_pf / k_gemm_ps
+//             (widths that are no multiple of 32: P in f32, k_vae_linear_fm)
 //   head      snake -> conv k=7 to one channel -> tanh   k_vae_head_fm
 // Row j of the transposed convolution's output phases r = 0..s-1 is output time
 // s j + r, so the GEMM's [L][s Cout] output is the frame-major [s L][Cout] output.
@@ -35,12 +37,14 @@ struct Res {
     const __half *a1 = nullptr, *dw_w = nullptr, *dw_b = nullptr, *a2 = nullptr, *pw_w = nullptr, *pw_b = nullptr;
     float *p = nullptr;        // k_vae_unit's parameters and weight, where the width has it
     __half *w = nullptr;
+    __half *pf = nullptr;      // wider ones: the 1x1 weight in the prefill layout
     uint32_t dilation = 1;
 };
 struct Stage {
     const __half *scale = nullptr, *bias = nullptr, *alpha = nullptr;   // scale/bias rows of the bucket
     float *pre = nullptr;      // the same as f32 [4][Cin] (launch_vae_repack_pre)
-    __half *ct_w = nullptr;    // [s Cout][2 Cin]
+    __half *ct_w = nullptr;    // [s Cout][2 Cin], in the prefill layout when planes
+    bool planes = false;       // P is kept as block-major planes (Cin % 32 == 0)
     float *ct_b = nullptr;     // [s Cout]
     uint32_t stride = 1, cin = 0, cout = 0;
     Res res[3];
@@ -49,6 +53,7 @@ struct Stage {
 inline uint64_t up256(uint64_t n) { return (n + 255u) / 256u * 256u; }
 
 inline float *F(vx_buf *b) { return static_cast<float *>(b->ptr); }
+inline __half *H(vx_buf *b) { return static_cast<__half *>(b->ptr); }
 
 }  // namespace
 
@@ -132,6 +137,68 @@ int grow(vx_ctx *ctx, vx_buf **b, uint64_t *cap, uint64_t floats) {
     return VX_OK;
 }
 
+// Whether a unit with a one-pass kernel runs as a depthwise pass and a GEMM over planes
+// instead: those of 512 channels below 2048 rows, where one pass would be under 64
+// workgroups of eight channel blocks each (frames 48 and 64, 2304 and 3072 rows: 462 and
+// 515 us in two passes, 453 and 494 in one; 100 and 160 frames 698 and 951 against 679
+// and 902; 252 frames equal). 256 channels are faster in one pass from 960 rows up (4
+// frames: 244 against 250 us).
+inline bool wide_run(uint32_t channels, uint32_t len) { return channels > 256u && (channels != 512u || len < 2048u); }
+
+// Units whose 1x1 weight is kept for that GEMM.
+inline bool wide_unit(uint32_t channels) {
+    return channels % 32u == 0u && (!vae_unit_channels(channels) || wide_run(channels, 0u));
+}
+// How plane_linear runs T rows of N outputs: small tiles of the register-streamed kernel
+// up to 64 tiles of 128 x 128, a quarter of the CUs (a limit of 16 or 160: 48 frames 511
+// or 499 us against 480).
+inline bool small_tiles(uint32_t T, uint32_t N) {
+    return T < 128u || (uint64_t)((N + 127u) / 128u) * ((T + 127u) / 128u) <= 64u;
+}
+
+// Bytes between the 32-channel blocks of a stage input's planes: len rows, whole
+// 128-row tiles of the GEMM, behind row -1.
+inline uint64_t plane_block(uint64_t len) { return ((len + 127u) / 128u * 128u + 1u) * 64u; }
+
+// y[t][n] (+)= b[n] + sum_k x[t][k] W[n][k] from hi/lo planes and a weight in the
+// prefill layout: block-major planes (block, shift as GemmArgs) into y, or tiled ones
+// added to y.
+// Small tiles run without a split, which would sum atomically into a cleared output (a
+// launch more); 128 x 128 tiles that leave half the CUs idle over a long K take two (252
+// frames, 2016 rows x 1024: 27 -> 24 us; the first up-convolution 60 -> 48 + 5).
+int plane_linear(vx_ctx *ctx, const __half *xh, const __half *xl, uint32_t block, uint32_t shift, const __half *pf,
+                 const __half *b16, const float *b32, float *y, uint32_t T, uint32_t N, uint32_t K,
+                 const float *pre = nullptr, const VaePlanes &out = VaePlanes()) {
+    GemmArgs g;
+    g.pre = pre;
+    g.oh = out.h;
+    g.ol = out.l;
+    g.o_block = out.block;
+    g.wk = WT_F16;
+    g.epi = block ? GEPI_STORE : GEPI_RESIDUAL;
+    g.seg[0].pq = reinterpret_cast<const int8_t *>(pf);
+    g.seg[0].rows = N;
+    g.seg[0].out = y;
+    g.seg[0].ldo = N;
+    g.seg[0].bias = b32 ? static_cast<const void *>(b32) : static_cast<const void *>(b16);
+    g.seg[0].bias_dtype = b32 ? 0u : 1u;
+    g.K = K;
+    g.T = T;
+    g.xh = xh;
+    g.xl = xl;
+    g.x_tiled = 1;
+    g.x_block = block;
+    g.x_shift = shift;
+    const uint64_t tiles = (uint64_t)((N + 127u) / 128u) * ((T + 127u) / 128u);
+    if (small_tiles(T, N)) return launch_gemm_ps_tiles(ctx->stream, g);
+    const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
+    if (tiles * 2u <= cus && K >= 1024u) {
+        g.ksplit = 2;
+        if (block) VX_CHECK(launch_fill_u32(ctx->stream, reinterpret_cast<uint32_t *>(y), 0u, (uint64_t)T * N));
+    }
+    return launch_gemm_pf(ctx->stream, g);
+}
+
 // y[t][n] (+)= b[n] + sum_k x[t][k] W[n][k]: the MFMA GEMM when K is a multiple
 // of 128, else the short-K kernel. Few tiles: split K with atomic adds into a
 // zeroed (store) or the residual (residual) output.
@@ -190,13 +257,25 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
     // Every stage indexes its activations (and the output length) in 32 bits.
     if (act > 0xffffffffull || x2_max > 0xffffffffull)
         return fail(VX_ERR_UNSUPPORTED, "AudioVAE decoder activation exceeds the 32-bit index range");
-    VX_CHECK(grow(ctx, &e->cur, &e->act_cap, act));
-    VX_CHECK(grow(ctx, &e->tmp, &e->tmp_cap, act));
-    // P of every stage starts behind decoder_dim floats of zeros (its row -1).
-    const uint64_t x2_cap = e->x2_cap;
-    VX_CHECK(grow(ctx, &e->x2, &e->x2_cap, c.decoder_dim + x2_max / 2u));
-    if (e->x2_cap != x2_cap) VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(F(e->x2)), 0u, c.decoder_dim));
+    // The tiled planes of a wide unit are whole 128-row tiles in tmp or cur; the input P of
+    // a stage is two block-major planes, or f32 rows from decoder_dim floats on.
+    uint64_t act_pad = act, x2_floats = c.decoder_dim + x2_max / 2u, l = frames;
+    for (const Stage &S : e->st) {
+        if (S.planes) x2_floats = std::max<uint64_t>(x2_floats, S.cin / 32u * plane_block(l) / 2u);
+        l *= S.stride;
+        if (S.res[0].pf) act_pad = std::max<uint64_t>(act_pad, (l + 127u) / 128u * 128u * S.cout);
+    }
+    VX_CHECK(grow(ctx, &e->cur, &e->act_cap, act_pad));
+    VX_CHECK(grow(ctx, &e->tmp, &e->tmp_cap, act_pad));
+    VX_CHECK(grow(ctx, &e->x2, &e->x2_cap, x2_floats));
     float *cur = F(e->cur), *tmp = F(e->tmp), *const P = F(e->x2) + c.decoder_dim;
+    auto planes_of = [&](const Stage &S, uint32_t rows) {
+        VaePlanes p;
+        p.block = (uint32_t)plane_block(rows);
+        p.h = H(e->x2) + 32;
+        p.l = p.h + (size_t)(S.cin / 32u) * (p.block / 2u);
+        return p;
+    };
     bool have_pre = false;   // P holds this stage's input already
     uint32_t len = frames, ch = c.latent_dim;
     {
@@ -219,9 +298,17 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
         const Stage &S = e->st[i];
         {
             ProfSpan sp(ctx, "audiovae.upsample");
-            if (!have_pre) VX_CHECK(launch_vae_pre_fm(s, cur, P, S.pre, ch, len));
-            VX_CHECK(linear(ctx, P - ch, ch, S.ct_w, nullptr, S.ct_b, tmp, S.stride * S.cout, len,
-                            S.stride * S.cout, 2u * ch, false));
+            if (S.planes) {
+                const VaePlanes p = planes_of(S, len);
+                if (!have_pre) VX_CHECK(launch_vae_pre_planes(s, cur, p, S.pre, ch, len));
+                VX_CHECK(plane_linear(ctx, p.h, p.l, p.block, ch / 32u, S.ct_w, nullptr, S.ct_b, tmp, len,
+                                      S.stride * S.cout, 2u * ch));
+            } else {
+                VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(P - ch), 0u, ch));   // row -1
+                VX_CHECK(launch_vae_pre_fm(s, cur, P, S.pre, ch, len));
+                VX_CHECK(linear(ctx, P - ch, ch, S.ct_w, nullptr, S.ct_b, tmp, S.stride * S.cout, len,
+                                S.stride * S.cout, 2u * ch, false));
+            }
         }
         std::swap(cur, tmp);
         len *= S.stride;
@@ -229,7 +316,9 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
         have_pre = false;
         for (const Res &R : S.res) {
             ProfSpan sp(ctx, "audiovae.residual");
-            if (R.p) {
+            const bool last = &R == &S.res[2] && i + 1 < kStages;
+            const bool wide = R.pf && (!R.p || wide_run(ch, len));
+            if (R.p && !wide) {
                 VaeUnitArgs u;
                 u.x = cur;
                 u.p = R.p;
@@ -237,9 +326,12 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
                 u.channels = ch;
                 u.length = len;
                 u.dilation = R.dilation;
-                have_pre = &R == &S.res[2] && i + 1 < kStages;
-                u.pre = have_pre ? e->st[i + 1].pre : nullptr;
-                u.y = have_pre ? P : tmp;
+                have_pre = last;
+                if (have_pre) {
+                    u.pre = e->st[i + 1].pre;
+                    u.planes = planes_of(e->st[i + 1], len);
+                }
+                u.y = tmp;
                 VX_CHECK(launch_vae_unit(s, u));
                 if (!have_pre) std::swap(cur, tmp);
                 continue;
@@ -247,6 +339,10 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
             VaeDwArgs d;
             d.x = cur;
             d.y = tmp;
+            if (wide) {
+                d.yh = reinterpret_cast<__half *>(tmp);
+                d.yl = d.yh + (size_t)((len + 127u) / 128u * 128u) * ch;
+            }
             d.w = R.dw_w;
             d.b = R.dw_b;
             d.alpha_in = R.a1;
@@ -257,7 +353,14 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
             d.dilation = R.dilation;
             d.left_pad = 6u * R.dilation;
             VX_CHECK(launch_vae_dwconv_fm(s, d));
-            VX_CHECK(linear(ctx, tmp, ch, R.pw_w, R.pw_b, nullptr, cur, ch, len, ch, ch, true));
+            if (wide) {
+                have_pre = last && e->st[i + 1].planes && small_tiles(len, ch);
+                VX_CHECK(plane_linear(ctx, d.yh, d.yl, 0u, 0u, R.pf, R.pw_b, nullptr, cur, len, ch, ch,
+                                      have_pre ? e->st[i + 1].pre : nullptr,
+                                      have_pre ? planes_of(e->st[i + 1], len) : VaePlanes()));
+            } else {
+                VX_CHECK(linear(ctx, tmp, ch, R.pw_w, R.pw_b, nullptr, cur, ch, len, ch, ch, true));
+            }
         }
     }
     ProfSpan sp(ctx, "audiovae.head");
@@ -338,7 +441,9 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
     uint32_t din = c.decoder_dim;
     for (uint32_t i = 0; i < kStages; ++i) {
         const uint32_t s = c.decoder_rates[i], dout = din / 2u;
-        arena += up256((uint64_t)s * dout * 2u * din * 2u) + up256((uint64_t)s * dout * 4u) + up256(din * 16u);
+        arena += up256(prefill_matrix_bytes(WT_F16, s * dout, 2u * din)) + up256((uint64_t)s * dout * 4u) +
+                 up256(din * 16u);
+        if (wide_unit(dout)) arena += 3u * up256(prefill_matrix_bytes(WT_F16, dout, dout));
         if (vae_unit_channels(dout)) arena += 3u * (up256(dout * 52u) + up256((uint64_t)dout * dout * 2u));
         din = dout;
     }
@@ -369,12 +474,14 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
             (st = conv(model, p + ".block.1", din, dout, 2u * s, 1, true, &ctw, &ctb)))
             return bail(st);
         S.ct_w = reinterpret_cast<__half *>(cur);
-        cur += up256((uint64_t)s * dout * 2u * din * 2u);
+        cur += up256(prefill_matrix_bytes(WT_F16, s * dout, 2u * din));
+        S.planes = din % 32u == 0u;
         S.ct_b = reinterpret_cast<float *>(cur);
         cur += up256((uint64_t)s * dout * 4u);
         S.pre = reinterpret_cast<float *>(cur);
         cur += up256(din * 16u);
-        if ((st = launch_vae_repack_convt(ctx->stream, ctw, ctb, din, dout, s, S.ct_w, S.ct_b)) ||
+        if ((st = launch_vae_repack_convt(ctx->stream, ctw, ctb, din, dout, s, S.planes ? 1u : 0u, S.ct_w,
+                                          S.ct_b)) ||
             (st = launch_vae_repack_pre(ctx->stream, S.scale, S.bias, S.alpha, din, S.pre)))
             return bail(st);
         static const uint32_t dil[3] = {1, 3, 9};
@@ -387,6 +494,11 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
                 (st = alpha(model, q + ".2.alpha", dout, &R.a2)) ||
                 (st = conv(model, q + ".3", dout, dout, 1, 1, false, &R.pw_w, &R.pw_b)))
                 return bail(st);
+            if (wide_unit(dout)) {
+                R.pf = reinterpret_cast<__half *>(cur);
+                cur += up256(prefill_matrix_bytes(WT_F16, dout, dout));
+                if ((st = launch_repack_prefill_f16(ctx->stream, R.pw_w, nullptr, dout, dout, R.pf))) return bail(st);
+            }
             if (!vae_unit_channels(dout)) continue;
             R.p = reinterpret_cast<float *>(cur);
             cur += up256(dout * 52u);

@@ -161,7 +161,7 @@ struct Src {
 template <bool XB>
 __device__ __forceinline__ int64_t x_offset(const GemmArgs &a, uint32_t blk) {
     if constexpr (!XB) return (int64_t)blk * kXBytes;
-    return blk < a.x_shift ? (int64_t)(blk * a.x_block) - 64 : (int64_t)((blk - a.x_shift) * a.x_block);
+    return blk < a.x_shift ? (int64_t)blk * a.x_block - 64 : (int64_t)(blk - a.x_shift) * a.x_block;
 }
 
 template <int WK, bool XB>
@@ -1001,7 +1001,6 @@ int launch_gemm_pf(hipStream_t s, GemmArgs a) {
     VX_PF_CASE(WT_F16, GEPI_RESIDUAL, false)
     VX_PF_CASE(WT_F16, GEPI_SWIGLU, false)
     VX_PF_CASE(WT_F16, GEPI_STORE, true)
-    VX_PF_CASE(WT_F16, GEPI_RESIDUAL, true)
 #undef VX_PF_CASE
     return fail(VX_ERR_UNSUPPORTED, "gemm: epilogue %u", a.epi);
 }

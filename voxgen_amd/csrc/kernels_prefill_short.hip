@@ -23,7 +23,7 @@
 // workgroup reads all of X), 26 with 128 (too few workgroups); eight waves: 18. The
 // split projections are the other way round (their K ranges are short): 9 us with 32
 // rows, 11 with 64; one workgroup per CU beat two (X again) by 10%.
-#include "vx_internal.h"
+#include "vae_dev.h"
 
 namespace vx {
 namespace {
@@ -70,14 +70,14 @@ struct Ops<WT_Q8, MT, NF> {
     float d[NF];
 };
 
-// Grid: a.ntn row tiles x a.ksplit K ranges.
-template <int WK, int EPI, int MT>
+// Grid: a.ntn row tiles x a.ntm token tiles x a.ksplit K ranges. XB: block-major planes.
+template <int WK, int EPI, int MT, int NF, bool XB>
 __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
-    constexpr int NF = EPI == GEPI_SWIGLU ? 4 : 2;
     constexpr uint32_t kRows = 16u * NF;   // weight rows of the workgroup
     __shared__ f4 red[NW / 2][MT][NF][64];   // partial tiles [wave][token fragment][row fragment][lane]
     constexpr int DEPTH = MT <= 4 ? 4 : 3;
-    const uint32_t tile = blockIdx.x % a.ntn, ks = blockIdx.x / a.ntn;
+    const uint32_t tile = blockIdx.x % a.ntn, ks = blockIdx.x / a.ntn / a.ntm;
+    const uint32_t m0 = blockIdx.x / a.ntn % a.ntm * (16u * MT);   // first token
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r16 = lane & 15u, g = lane >> 4;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t seg = 0;
@@ -100,11 +100,15 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
         dr[f] = WK == WT_Q8 ? sg.pd + piece * kPiece + n : nullptr;
     }
     const uint8_t *const xh = reinterpret_cast<const uint8_t *>(a.xh), *const xl = reinterpret_cast<const uint8_t *>(a.xl);
-    uint32_t xo[MT];   // rows past T of the 128-row tile are multiplied and never stored
+    // Rows past T of the 128-row tile are multiplied and never stored. Rows read one
+    // earlier (xs) carry the permutation of that row.
+    uint32_t xo[MT], xs[XB ? MT : 1];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        const uint32_t t = 16u * mt + r16;
-        xo[mt] = t * 64u + 16u * (g ^ xperm(t));
+        const uint32_t t = m0 + 16u * mt + r16;
+        const uint32_t row = XB ? t * 64u : (t / kPiece * nblk * kPiece + t % kPiece) * 64u;
+        xo[mt] = row + 16u * (g ^ xperm(t));
+        if constexpr (XB) xs[mt] = row + 16u * (g ^ xperm(t - 1u));
     }
     const uint32_t s0 = ks * nblk / a.ksplit, s1 = (ks + 1u) * nblk / a.ksplit;
     const int n_it = s0 + wv < s1 ? (int)((s1 - s0 - wv + NW - 1u) / NW) : 0;
@@ -126,10 +130,15 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
                 o.w[f] = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(wr[f] + blk * (kPiece * 64u)));
             }
         }
+        const bool shifted = XB && blk < a.x_shift;
+        const ptrdiff_t xb = !XB       ? (ptrdiff_t)(blk * (kPiece * 64u))
+                             : shifted ? (ptrdiff_t)(blk * a.x_block) - 64
+                                       : (ptrdiff_t)((blk - a.x_shift) * a.x_block);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            o.xh[mt] = *reinterpret_cast<const u4v *>(xh + blk * (kPiece * 64u) + xo[mt]);
-            o.xl[mt] = *reinterpret_cast<const u4v *>(xl + blk * (kPiece * 64u) + xo[mt]);
+            const uint32_t x = XB && shifted ? xs[XB ? mt : 0] : xo[mt];
+            o.xh[mt] = *reinterpret_cast<const u4v *>(xh + xb + x);
+            o.xl[mt] = *reinterpret_cast<const u4v *>(xl + xb + x);
         }
     };
     auto mma = [&](const Ops<WK, MT, NF> &o) {
@@ -196,10 +205,10 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
         constexpr uint32_t kPairs = kRows / 2u;
         for (uint32_t o = tid; o < kPairs * 16u * MT; o += 64u * NW) {
             const uint32_t nl = o % kPairs, tok = o / kPairs, row = kPairs * tile + nl, f = nl >> 4, n = nl & 15u;
-            if (tok >= a.T || row >= sg.rows) continue;
+            if (m0 + tok >= a.T || row >= sg.rows) continue;
             const float gv = part(tok, f, n), uv = part(tok, f + 2u, n);
             const float v = gv / (1.0f + expf(-gv)) * uv;   // matvec_swiglu.comp:67
-            const size_t po = tiled_plane_index(tok, row, a.ldp);
+            const size_t po = tiled_plane_index(m0 + tok, row, a.ldp);
             const _Float16 hv = (_Float16)v;
             a.oh[po] = __builtin_bit_cast(__half, hv);
             a.ol[po] = __builtin_bit_cast(__half, (_Float16)(v - (float)hv));
@@ -211,14 +220,32 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
                                              : sg.out;
         for (uint32_t o = tid; o < kRows * 16u * MT; o += 64u * NW) {
             const uint32_t nl = o % kRows, tok = o / kRows, row = kRows * (tile - sg.tile0) + nl;
-            if (tok >= a.T || row >= sg.rows) continue;
+            if (m0 + tok >= a.T || row >= sg.rows) continue;
             float v = part(tok, nl >> 4, nl & 15u);
             if constexpr (WK == WT_F16) {
                 if (sg.bias && ks == 0u)
                     v += sg.bias_dtype == 0 ? static_cast<const float *>(sg.bias)[row]
                                             : __half2float(static_cast<const __half *>(sg.bias)[row]);
             }
-            float *const dst = out + (size_t)tok * sg.ldo + row;
+            float *const dst = out + (size_t)(m0 + tok) * sg.ldo + row;
+            if constexpr (EPI == GEPI_RESIDUAL && NF == 1) {
+                if (a.pre) {
+                    const float y = fmaf(*dst + v, a.pre[row], a.pre[sg.rows + row]), sn = a.pre[2u * sg.rows + row] * y;
+                    const float sq = fabsf(sn) < kSinSqMax ? sin_sq(sn) : sin_sq_any(sn);
+                    const float p = fmaf(sq, a.pre[3u * sg.rows + row], y);
+                    const _Float16 hv = (_Float16)p;
+                    const uint32_t t = m0 + tok;
+                    const size_t po = (size_t)(row >> 5) * (a.o_block / 2u) + (size_t)t * 32u +
+                                      8u * (((row >> 3) & 3u) ^ xperm(t)) + (row & 7u);
+                    a.oh[po] = __builtin_bit_cast(__half, hv);
+                    a.ol[po] = __builtin_bit_cast(__half, (_Float16)(p - (float)hv));
+                    if (t == 0u) {
+                        const ptrdiff_t z = (ptrdiff_t)((size_t)(row >> 5) * (a.o_block / 2u) + (row & 31u)) - 32;
+                        a.oh[z] = a.ol[z] = __float2half(0.f);
+                    }
+                    continue;
+                }
+            }
             if constexpr (EPI == GEPI_STORE)
                 *dst = v * a.alpha;
             else
@@ -227,27 +254,37 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_ps(GemmArgs a) {
     }
 }
 
+#define VX_PS_CASE(M, NF, XB)                                                    \
+    if (mt == M) {                                                               \
+        k_gemm_ps<WK, EPI, M, NF, XB><<<grid, 64 * NW, 0, s>>>(a);               \
+        VX_LAUNCHED("k_gemm_ps");                                                \
+        return VX_OK;                                                            \
+    }
+// One token tile of up to 128 rows.
 template <int WK, int EPI>
 int launch_ps(hipStream_t s, const GemmArgs &a, uint32_t grid) {
-    switch ((a.T + 15u) / 16u) {
-#define VX_PS_CASE(M)                                           \
-    case M:                                                     \
-        k_gemm_ps<WK, EPI, M><<<grid, 64 * NW, 0, s>>>(a);  \
-        break;
-        VX_PS_CASE(1)
-        VX_PS_CASE(2)
-        VX_PS_CASE(3)
-        VX_PS_CASE(4)
-        VX_PS_CASE(5)
-        VX_PS_CASE(6)
-        VX_PS_CASE(7)
-        VX_PS_CASE(8)
-#undef VX_PS_CASE
-        default: return fail(VX_ERR_UNSUPPORTED, "short prefill gemm: %u rows", a.T);
-    }
-    VX_LAUNCHED("k_gemm_ps");
-    return VX_OK;
+    constexpr int NF = EPI == GEPI_SWIGLU ? 4 : 2;
+    const uint32_t mt = (a.T + 15u) / 16u;
+    VX_PS_CASE(1, NF, false)
+    VX_PS_CASE(2, NF, false)
+    VX_PS_CASE(3, NF, false)
+    VX_PS_CASE(4, NF, false)
+    VX_PS_CASE(5, NF, false)
+    VX_PS_CASE(6, NF, false)
+    VX_PS_CASE(7, NF, false)
+    VX_PS_CASE(8, NF, false)
+    return fail(VX_ERR_UNSUPPORTED, "short prefill gemm: %u rows", a.T);
 }
+// Token tiles of mt fragments.
+template <int EPI, int NF, bool XB>
+int launch_ps_tiles(hipStream_t s, const GemmArgs &a, uint32_t grid, uint32_t mt) {
+    constexpr int WK = WT_F16;
+    VX_PS_CASE(1, NF, XB)
+    VX_PS_CASE(2, NF, XB)
+    VX_PS_CASE(4, NF, XB)
+    return fail(VX_ERR_UNSUPPORTED, "short gemm: token tile of %u fragments", mt);
+}
+#undef VX_PS_CASE
 
 }  // namespace
 
@@ -287,6 +324,36 @@ int launch_gemm_ps(hipStream_t s, GemmArgs a) {
     VX_PS_KIND(WT_F16, GEPI_SWIGLU)
 #undef VX_PS_KIND
     return fail(VX_ERR_UNSUPPORTED, "gemm: epilogue %u", a.epi);
+}
+
+// F16, no split: 32-row tiles of 64 tokens, and smaller ones while they leave CUs idle.
+// The AudioVAE's up-convolutions and 1x1 convolutions of a 4-frame patch, against k_gemm's
+// tiles with atomic sums into a cleared output (two launches): 21 + 2 -> 14.7 us for the
+// 67 MB of the first (13 us at the copy rate), 11 + 2 -> 9.4 for the second, 9 -> 7 for a
+// 1x1 convolution.
+int launch_gemm_ps_tiles(hipStream_t s, GemmArgs a) {
+    if (a.wk != WT_F16 || a.nseg != 1 || a.ksplit > 1u || a.T == 0 || a.K % 32u || !a.seg[0].pq || !a.xh || !a.xl ||
+        !a.seg[0].out || !a.seg[0].rows)
+        return fail(VX_ERR_INVALID_ARG, "short gemm: one F16 matrix in the prefill layout, K %% 32, no split");
+    if ((a.epi == GEPI_STORE) != (a.x_block != 0u) || (a.epi != GEPI_STORE && a.epi != GEPI_RESIDUAL))
+        return fail(VX_ERR_UNSUPPORTED, "short gemm: block-major store or tiled residual");
+    if (a.pre && (a.epi != GEPI_RESIDUAL || !a.oh || !a.ol || a.o_block % 64u || a.o_block / 64u <= a.T ||
+                  a.seg[0].rows % 32u || a.seg[0].ldo != a.seg[0].rows))
+        return fail(VX_ERR_INVALID_ARG, "short gemm: planes of %u rows, block %u", a.T, a.o_block);
+    uint32_t mt = a.T <= 16u ? 1u : a.T <= 32u ? 2u : 4u, nf = 2;
+    const uint64_t ntn = (a.seg[0].rows + 31u) / 32u;
+    if (a.pre || ntn * ((a.T + 16u * mt - 1u) / (16u * mt)) <= 96u) nf = 1;
+    a.ksplit = 1;
+    a.seg[0].tile0 = 0;
+    a.ntn = (a.seg[0].rows + 16u * nf - 1u) / (16u * nf);
+    a.ntm = (a.T + 16u * mt - 1u) / (16u * mt);
+    const uint64_t grid = (uint64_t)a.ntn * a.ntm;
+    if (grid > 0x7fffffffull) return fail(VX_ERR_UNSUPPORTED, "short gemm: grid too large");
+    if (a.epi == GEPI_STORE)
+        return nf == 1 ? launch_ps_tiles<GEPI_STORE, 1, true>(s, a, (uint32_t)grid, mt)
+                       : launch_ps_tiles<GEPI_STORE, 2, true>(s, a, (uint32_t)grid, mt);
+    return nf == 1 ? launch_ps_tiles<GEPI_RESIDUAL, 1, false>(s, a, (uint32_t)grid, mt)
+                   : launch_ps_tiles<GEPI_RESIDUAL, 2, false>(s, a, (uint32_t)grid, mt);
 }
 
 }  // namespace vx

@@ -13,6 +13,10 @@
 namespace vx {
 namespace {
 
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+
+
 __device__ __forceinline__ float hf(__half v) { return __half2float(v); }
 
 // A model scalar of GGML dtype 1 (F16) or 0 (F32).
@@ -185,6 +189,16 @@ __global__ __launch_bounds__(256) void k_vae_dwconv_tiled_fm(VaeDwArgs a, uint32
             if ((uint32_t)k < a.kernel) sum += xs[((r + k * a.dilation) << cb_shift) + cc] * wk[k];
         return sum;
     };
+    auto put = [&](uint32_t t, float v) {
+        if (!a.yh) {
+            a.y[(size_t)t * C + c] = v;
+            return;
+        }
+        const size_t o = tiled_plane_index(t, c, C);
+        const _Float16 h = (_Float16)v;
+        a.yh[o] = __builtin_bit_cast(__half, h);
+        a.yl[o] = __builtin_bit_cast(__half, (_Float16)(v - (float)h));
+    };
     big = 0.f;
 #pragma unroll
     for (uint32_t i = 0; i < 8u; ++i) {   // TB * CB = 2048 outputs, 8 per thread
@@ -192,7 +206,7 @@ __global__ __launch_bounds__(256) void k_vae_dwconv_tiled_fm(VaeDwArgs a, uint32
         if (t >= a.length || !cval) continue;
         const float sum = conv(r);
         big = fmaxf(big, fabsf(aout * sum));
-        a.y[(size_t)t * C + c] = a.alpha_out ? snake_fm(sum, aout * sum, iout) : sum;
+        put(t, a.alpha_out ? snake_fm(sum, aout * sum, iout) : sum);
     }
     if (a.alpha_out && any_large(big)) {
 #pragma unroll 1
@@ -200,9 +214,76 @@ __global__ __launch_bounds__(256) void k_vae_dwconv_tiled_fm(VaeDwArgs a, uint32
             const uint32_t r = (tid + 256u * i) >> cb_shift, t = t0 + r;
             if (t >= a.length || !cval) continue;
             const float sum = conv(r);
-            a.y[(size_t)t * C + c] = snake_any(sum, aout * sum, iout);
+            put(t, snake_any(sum, aout * sum, iout));
         }
     }
+}
+
+// Seven taps over few rows: a thread computes two neighbouring channels of one row
+// straight from the input, all loads issued before the first is used. Against the tiled
+// kernel this takes the snake of every input up to seven times, but has a thread for
+// every pair of outputs, no LDS and no barrier (32 rows of 1024 channels are 16 tiled
+// workgroups: 8.8 -> 4.3 us). Below 1.5 M outputs only: the snakes are then under 4 us of
+// the chip.
+__global__ __launch_bounds__(256) void k_vae_dw7_fm(VaeDwArgs a) {
+    const uint32_t i = 2u * (blockIdx.x * 256u + threadIdx.x), C = a.channels;
+    if (i >= a.length * C) return;
+    const uint32_t t = i / C, c = i - t * C;
+    float2 x[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+        const int r = (int)(t + (uint32_t)k * a.dilation) - (int)a.left_pad;
+        x[k] = r >= 0 ? *reinterpret_cast<const float2 *>(a.x + (size_t)r * C + c) : make_float2(0.f, 0.f);
+    }
+    float w[2][7], sum[2], ai[2] = {0.f, 0.f}, ao[2] = {0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int k = 0; k < 7; ++k) w[j][k] = hf(a.w[(c + j) * 7u + k]);
+        sum[j] = hf(a.b[c + j]);
+        if (a.alpha_in) ai[j] = hf(a.alpha_in[c + j]);
+        if (a.alpha_out) ao[j] = hf(a.alpha_out[c + j]);
+    }
+    float big = 0.f;
+    if (a.alpha_in) {
+        const float inv0 = snake_inv(ai[0]), inv1 = snake_inv(ai[1]);
+#pragma unroll
+        for (int k = 0; k < 7; ++k) {   // snake(0) = 0: the padding stays zero
+            const float s0 = ai[0] * x[k].x, s1 = ai[1] * x[k].y;
+            big = fmaxf(big, fmaxf(fabsf(s0), fabsf(s1)));
+            x[k] = make_float2(snake_fm(x[k].x, s0, inv0), snake_fm(x[k].y, s1, inv1));
+        }
+        if (any_large(big)) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) {
+                const int r = (int)(t + (uint32_t)k * a.dilation) - (int)a.left_pad;
+                if (r < 0) continue;
+                const float2 v = *reinterpret_cast<const float2 *>(a.x + (size_t)r * C + c);
+                x[k] = make_float2(snake_any(v.x, ai[0] * v.x, inv0), snake_any(v.y, ai[1] * v.y, inv1));
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+        sum[0] += x[k].x * w[0][k];
+        sum[1] += x[k].y * w[1][k];
+    }
+    if (a.alpha_out) {
+        const bool large = any_large(fmaxf(fabsf(ao[0] * sum[0]), fabsf(ao[1] * sum[1])));
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            sum[j] = large ? snake_any(sum[j], ao[j] * sum[j], snake_inv(ao[j]))
+                           : snake_fm(sum[j], ao[j] * sum[j], snake_inv(ao[j]));
+    }
+    if (!a.yh) {
+        *reinterpret_cast<float2 *>(a.y + i) = make_float2(sum[0], sum[1]);
+        return;
+    }
+    const size_t o = tiled_plane_index(t, c, C);
+    const h2v hv = {(_Float16)sum[0], (_Float16)sum[1]};
+    const h2v lv = {(_Float16)(sum[0] - (float)hv[0]), (_Float16)(sum[1] - (float)hv[1])};
+    *reinterpret_cast<h2v *>(a.yh + o) = hv;
+    *reinterpret_cast<h2v *>(a.yl + o) = lv;
 }
 
 // The input of a stage's transposed convolution, P = snake_pa(x * ps + pt) per
@@ -244,6 +325,62 @@ __global__ __launch_bounds__(256) void k_vae_pre_fm(const float *x, float *y, co
         y[i] = v[0];
 }
 
+// P as block-major planes: one thread per eight channels of a row, the threads of a
+// 32-channel block consecutive, so that a wave reads 128-byte runs and writes one of
+// 1 KB a plane (row by row, with 64-byte runs: 20 us at 2016 x 1024, this way 5.5); the
+// threads of row 0 also zero row -1.
+__global__ __launch_bounds__(256) void k_vae_pre_planes(const float *x, VaePlanes y, const float *pre, uint32_t C,
+                                                        uint32_t length) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, t = i >> 2, c = blockIdx.y * 32u + 8u * (i & 3u);
+    if (t >= length) return;
+    float v[8], s[8], inv[8], big = 0.f;
+    const float *const xr = x + (size_t)t * C + c;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const float4 q = *reinterpret_cast<const float4 *>(xr + 4 * h);
+        const float4 p[4] = {*reinterpret_cast<const float4 *>(pre + c + 4 * h),
+                             *reinterpret_cast<const float4 *>(pre + C + c + 4 * h),
+                             *reinterpret_cast<const float4 *>(pre + 2u * C + c + 4 * h),
+                             *reinterpret_cast<const float4 *>(pre + 3u * C + c + 4 * h)};
+        const float qv[4] = {q.x, q.y, q.z, q.w}, ps[4] = {p[0].x, p[0].y, p[0].z, p[0].w},
+                    pt[4] = {p[1].x, p[1].y, p[1].z, p[1].w}, pa[4] = {p[2].x, p[2].y, p[2].z, p[2].w},
+                    pi[4] = {p[3].x, p[3].y, p[3].z, p[3].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[4 * h + j] = fmaf(qv[j], ps[j], pt[j]);
+            s[4 * h + j] = pa[j] * v[4 * h + j];
+            inv[4 * h + j] = pi[j];
+            big = fmaxf(big, fabsf(s[4 * h + j]));
+        }
+    }
+    __half *const yh = y.h + (size_t)blockIdx.y * (y.block / 2u), *const yl = y.l + (size_t)blockIdx.y * (y.block / 2u);
+    const size_t o = (size_t)t * 32u + 8u * ((i & 3u) ^ (((t >> 1) ^ (t >> 3)) & 3u));
+    if (t == 0u) {
+        *reinterpret_cast<h8v *>(yh + 8u * (i & 3u) - 32) = h8v{};
+        *reinterpret_cast<h8v *>(yl + 8u * (i & 3u) - 32) = h8v{};
+    }
+    if (any_large(big)) {
+#pragma unroll 1
+        for (uint32_t j = 0; j < 8u; ++j) {
+            const float w = fmaf(xr[j], pre[c + j], pre[C + c + j]);
+            const float r = snake_any(w, pre[2u * C + c + j] * w, pre[3u * C + c + j]);
+            const _Float16 h = (_Float16)r;
+            yh[o + j] = __builtin_bit_cast(__half, h);
+            yl[o + j] = __builtin_bit_cast(__half, (_Float16)(r - (float)h));
+        }
+        return;
+    }
+    h8v hv, lv;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float r = snake_fm(v[j], s[j], inv[j]);
+        hv[j] = (_Float16)r;
+        lv[j] = (_Float16)(r - (float)hv[j]);
+    }
+    *reinterpret_cast<h8v *>(yh + o) = hv;
+    *reinterpret_cast<h8v *>(yl + o) = lv;
+}
+
 __global__ __launch_bounds__(256) void k_vae_repack_pre(const __half *scale, const __half *bias, const __half *alpha,
                                                         uint32_t C, float *pre) {
     const uint32_t c = blockIdx.x * 256u + threadIdx.x;
@@ -258,13 +395,17 @@ __global__ __launch_bounds__(256) void k_vae_repack_pre(const __half *scale, con
 // the GEMM form: W'[(r Cout + oc)][(1 - tap) Cin + ic] = W[ic][oc][r + tap s] (tap 1
 // multiplies the earlier row, which comes first), and the bias tiled over the s phases, b'[r Cout + oc] = b[oc].
 __global__ __launch_bounds__(256) void k_vae_repack_convt(const __half *w, const __half *b, uint32_t cin,
-                                                          uint32_t cout, uint32_t s, __half *wp, float *bp) {
+                                                          uint32_t cout, uint32_t s, uint32_t prefill_layout,
+                                                          __half *wp, float *bp) {
     const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
     const uint64_t n = (uint64_t)s * cout * 2u * cin;
     if (i < n) {
         const uint32_t row = (uint32_t)(i / (2u * cin)), col = (uint32_t)(i - (uint64_t)row * 2u * cin);
         const uint32_t r = row / cout, oc = row - r * cout, tap = col / cin, ic = col - tap * cin;
-        wp[i] = w[((size_t)ic * cout + oc) * (2u * s) + r + (1u - tap) * s];
+        wp[prefill_layout ? tiled_plane_index(row, col, 2u * cin) : i] =
+            w[((size_t)ic * cout + oc) * (2u * s) + r + (1u - tap) * s];
+    } else if (prefill_layout && i < (uint64_t)((s * cout + 127u) / 128u * 128u) * 2u * cin) {   // padding rows
+        wp[tiled_plane_index((uint32_t)(i / (2u * cin)), (uint32_t)(i % (2u * cin)), 2u * cin)] = __float2half(0.f);
     }
     if (i < (uint64_t)s * cout) bp[i] = hf(b[i % cout]);
 }
@@ -506,6 +647,13 @@ int launch_vae_tanh(hipStream_t s, float *x, uint32_t n) {
 int launch_vae_dwconv_fm(hipStream_t s, const VaeDwArgs &a) {
     const uint64_t n = (uint64_t)a.length * a.channels;
     if (!n) return VX_OK;
+    if (a.yh && (!a.yl || a.channels % 32u)) return fail(VX_ERR_INVALID_ARG, "vae depthwise: planes need channels %% 32");
+    if (a.kernel == 7u && a.left_pad == 6u * a.dilation && a.channels % 2u == 0u && n <= 1572864u &&
+        ((uintptr_t)a.x & 7u) == 0 && ((uintptr_t)a.y & 7u) == 0) {
+        k_vae_dw7_fm<<<grid1(n / 2u), 256, 0, s>>>(a);
+        VX_LAUNCHED("k_vae_dw7_fm");
+        return VX_OK;
+    }
     if (a.kernel >= 1u && a.kernel <= 8u && a.left_pad == (a.kernel - 1u) * a.dilation && a.left_pad <= 54u) {
         const uint32_t CB = a.channels < 64u ? a.channels : 64u;   // >= 1; 2048 / CB rows per workgroup
         if ((CB & (CB - 1u)) == 0) {
@@ -516,6 +664,7 @@ int launch_vae_dwconv_fm(hipStream_t s, const VaeDwArgs &a) {
             return VX_OK;
         }
     }
+    if (a.yh) return fail(VX_ERR_UNSUPPORTED, "vae depthwise: planes of this shape");
     k_vae_dwconv_fm<<<grid1(n), 256, 0, s>>>(a);
     VX_LAUNCHED("k_vae_dwconv_fm");
     return VX_OK;
@@ -532,6 +681,18 @@ int launch_vae_pre_fm(hipStream_t s, const float *x, float *y, const float *pre,
     return VX_OK;
 }
 
+int launch_vae_pre_planes(hipStream_t s, const float *x, const VaePlanes &y, const float *pre, uint32_t channels,
+                          uint32_t length) {
+    const uint64_t n = (uint64_t)length * channels;
+    if (!n) return VX_OK;
+    if (channels % 32u || !y.h || !y.l || y.block % 64u || y.block / 64u <= length ||
+        ((uintptr_t)x | (uintptr_t)y.h | (uintptr_t)y.l | (uintptr_t)pre) & 15u || length > 0x3fffffffu)
+        return fail(VX_ERR_INVALID_ARG, "vae pre: planes of %u channels, block %u", channels, y.block);
+    k_vae_pre_planes<<<dim3(grid1(4ull * length), channels / 32u), 256, 0, s>>>(x, y, pre, channels, length);
+    VX_LAUNCHED("k_vae_pre_planes");
+    return VX_OK;
+}
+
 int launch_vae_repack_pre(hipStream_t s, const __half *scale, const __half *bias, const __half *alpha,
                           uint32_t channels, float *pre) {
     k_vae_repack_pre<<<grid1(channels), 256, 0, s>>>(scale, bias, alpha, channels, pre);
@@ -540,9 +701,9 @@ int launch_vae_repack_pre(hipStream_t s, const __half *scale, const __half *bias
 }
 
 int launch_vae_repack_convt(hipStream_t s, const __half *w, const __half *b, uint32_t cin, uint32_t cout,
-                            uint32_t stride, __half *wp, float *bp) {
-    const uint64_t n = (uint64_t)stride * cout * 2u * cin;
-    k_vae_repack_convt<<<grid1(n), 256, 0, s>>>(w, b, cin, cout, stride, wp, bp);
+                            uint32_t stride, uint32_t prefill_layout, __half *wp, float *bp) {
+    const uint64_t rows = prefill_layout ? (stride * cout + 127u) / 128u * 128u : stride * cout;
+    k_vae_repack_convt<<<grid1(rows * 2u * cin), 256, 0, s>>>(w, b, cin, cout, stride, prefill_layout, wp, bp);
     VX_LAUNCHED("k_vae_repack_convt");
     return VX_OK;
 }

@@ -20,7 +20,9 @@
 // LDS in one pass (64, 32): 256 channels 152 -> 63 us, 128 channels 110 -> 56, 64
 // channels 91 -> 41, 32 channels 62 -> 34. Larger tiles of 256 and 128 channels at one
 // workgroup of eight waves per CU were slower (79 and 60 us), and so was holding them
-// to 128 vector registers for two (140 and 100 us: spills).
+// to 128 vector registers for two (140 and 100 us: spills). The unit that ends a stage
+// writes the next stage's planes: 15 us more at 256 channels (20 with an address a store), where a pass of its own
+// over f32 would read and write 120 MB.
 #include "vae_dev.h"
 
 namespace vx {
@@ -68,6 +70,12 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, hs = lane >> 5;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wv / WN, wn = wv % WN;
     const bool mul = wv < (uint32_t)(WM * WN);
+    if (a.pre && blockIdx.x == 0) {   // row -1 of the planes
+        for (uint32_t i = tid; i < (uint32_t)C / 4u; i += NT) {   // plane, block, 16-byte chunk
+            __half *const p = (i & 4u ? a.planes.l : a.planes.h) + (size_t)(i >> 3) * (a.planes.block / 2u);
+            *reinterpret_cast<uint4 *>(p - 32 + 8 * (int)(i & 3u)) = make_uint4(0, 0, 0, 0);
+        }
+    }
     const uint32_t t0 = blockIdx.x * TB, halo = 6u * a.dilation, rows = TB + halo;
     const uint32_t c4 = 4u * (tid % G4), r0 = tid / G4;
     // Uniform bases with 32-bit offsets: rows of the tile from its history on (rows
@@ -239,6 +247,15 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
         store();
         return;
     }
+    // The next stage's planes. A row's 32 channels are one 64-byte run per plane, its
+    // 16-byte chunks permuted by the row; lanes pair up, the even one storing both high
+    // halves and the odd one both low halves.
+    const VaePlanes &P = a.planes;
+    auto po = [&](int n, uint32_t t) {   // halves from the tile's row 0 of block 0, this lane's channel
+        return (size_t)(wn * NTL + n) * (P.block / 2u) + t * 32u +
+               8u * ((l32 >> 3) ^ (((t >> 1) ^ (t >> 3)) & 3u)) + (l32 & 7u);
+    };
+    __half *const yh = P.h + (size_t)t0 * 32u, *const yl = P.l + (size_t)t0 * 32u;
     float ps[NTL], pt[NTL], pa[NTL], pi[NTL], big = 0.f;
 #pragma unroll
     for (int n = 0; n < NTL; ++n) {
@@ -250,20 +267,64 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
         big = fmaxf(big, fabsf(pa[n] * v));
         return v;
     });
-    if (any_large(big)) {   // stored unfinished, then finished one by one by the same lane
-        store();
+    if (any_large(big)) {
+        // The bits are stored unfinished (upper half in one plane, lower in the other),
+        // then finished one by one by the same lane.
+        each([&](int n, uint32_t t, uint32_t, float v) {
+            if (t < have) {
+                const uint32_t b = __builtin_bit_cast(uint32_t, v);
+                yh[po(n, t)] = __builtin_bit_cast(__half, (unsigned short)(b >> 16));
+                yl[po(n, t)] = __builtin_bit_cast(__half, (unsigned short)b);
+            }
+            return v;
+        });
 #pragma unroll 1
         for (uint32_t i = 0; i < (uint32_t)(NTL * MT * 16); ++i) {
             const uint32_t n = i / (MT * 16), m = i / 16 % MT, r = i % 16;
             const uint32_t ch = 32u * (wn * NTL + n) + l32, t = tb + 32u * m + 8u * (r >> 2) + (r & 3);
             if (t >= have) continue;
-            const float v = yt[t * C + ch];
-            yt[t * C + ch] = fmaf(sin_sq_any(a.pre[2 * C + ch] * v), a.pre[3 * C + ch], v);
+            const size_t o = po((int)n, t);
+            float v = __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(unsigned short, yh[o]) << 16 |
+                                                    __builtin_bit_cast(unsigned short, yl[o]));
+            v = fmaf(sin_sq_any(a.pre[2 * C + ch] * v), a.pre[3 * C + ch], v);
+            const _Float16 h = (_Float16)v;
+            yh[o] = __builtin_bit_cast(__half, h);
+            yl[o] = __builtin_bit_cast(__half, (_Float16)(v - (float)h));
         }
         return;
     }
-    each([&](int n, uint32_t, uint32_t, float v) { return fmaf(sin_sq(pa[n] * v), pi[n], v); });
-    store();
+    const uint32_t odd = lane & 1u, sel = odd ? 0x03020706u : 0x05040100u;   // of (other, own)
+    // Row 4 hs + 8 q + j of 32 has chunk (l32 / 8) ^ 2 hs ^ (q ^ j / 2): four lane
+    // addresses a channel tile, and the rows are immediate offsets from them.
+    __half *yx[NTL][4];
+#pragma unroll
+    for (int n = 0; n < NTL; ++n)
+#pragma unroll
+        for (uint32_t x = 0; x < 4u; ++x)
+            yx[n][x] = (odd ? yl : yh) - odd + (size_t)(wn * NTL + n) * (P.block / 2u) + tb * 32u +
+                       8u * ((l32 >> 3) ^ (2u * hs) ^ x) + (l32 & 7u);
+    auto finish = [&](auto keep) {
+#pragma unroll
+        for (int n = 0; n < NTL; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = 32 * m + 8 * (r >> 2) + (r & 3);
+                    const float v = fmaf(sin_sq(pa[n] * acc[m][n][r]), pi[n], acc[m][n][r]);
+                    const _Float16 h = (_Float16)v, l = (_Float16)(v - (float)h);
+                    const uint32_t own = (uint32_t)__builtin_bit_cast(unsigned short, h) |
+                                         (uint32_t)__builtin_bit_cast(unsigned short, l) << 16;
+                    const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0xB1, 0xf, 0xf, true);
+                    if (keep(tb + row))
+                        *reinterpret_cast<uint32_t *>(yx[n][(r >> 2) ^ ((r & 3) >> 1)] + 32 * row) =
+                            __builtin_amdgcn_perm(other, own, sel);
+                }
+    };
+    if (full)
+        finish([](uint32_t) { return true; });
+    else
+        finish([&](uint32_t t) { return t < have; });
 }
 
 // A unit's parameters as f32 [C / KB][13][KB], KB = min(C, 64): a1, 1/(a1 + 1e-9), a2,
@@ -298,7 +359,7 @@ int launch_unit(hipStream_t s, const VaeUnitArgs &a) {
 
 }  // namespace
 
-bool vae_unit_channels(uint32_t c) { return c == 32u || c == 64u || c == 128u || c == 256u; }
+bool vae_unit_channels(uint32_t c) { return c == 32u || c == 64u || c == 128u || c == 256u || c == 512u; }
 
 int launch_vae_repack_unit(hipStream_t s, const __half *a1, const __half *dw, const __half *db, const __half *a2,
                            const __half *pw, const __half *pb, uint32_t channels, float *p, __half *w) {
@@ -311,6 +372,8 @@ int launch_vae_unit(hipStream_t s, const VaeUnitArgs &a) {
     if (!a.length) return VX_OK;
     if (!vae_unit_channels(a.channels) || !a.dilation || 6u * a.dilation > kMaxHalo || a.x == a.y)
         return fail(VX_ERR_UNSUPPORTED, "vae residual unit: %u channels, dilation %u", a.channels, a.dilation);
+    if (a.pre && (!a.planes.h || !a.planes.l || a.planes.block % 64u || a.planes.block / 64u <= a.length))
+        return fail(VX_ERR_INVALID_ARG, "vae residual unit: planes of %u rows, block %u", a.length, a.planes.block);
     // Tiles of 128 or 64 rows (less history per row) once they give every CU one, else
     // of 32 (4 frames, 256 channels: 15 workgroups of 64 rows on 256 CUs).
     switch (a.channels) {
@@ -320,6 +383,8 @@ int launch_vae_unit(hipStream_t s, const VaeUnitArgs &a) {
         return a.length >= 128u * 256u ? launch_unit<64, 128, 8, 4, 2, 4>(s, a) : launch_unit<64, 32, 4, 1, 2, 2>(s, a);
     case 128:
         return a.length >= 64u * 256u ? launch_unit<128, 64, 4, 1, 4, 2>(s, a) : launch_unit<128, 32, 4, 1, 4, 2>(s, a);
+    case 512:
+        return launch_unit<512, 32, 8, 1, 8, 2>(s, a);
     default:
         return a.length >= 64u * 256u ? launch_unit<256, 64, 4, 1, 4, 2>(s, a) : launch_unit<256, 32, 8, 1, 8, 2>(s, a);
     }

@@ -391,6 +391,11 @@ struct GemmArgs {
     // as in the tiled layout, and rows past T of the last 128-row tile may be read; the
     // first x_shift blocks of K are read one row earlier (row -1 is the row before xh).
     uint32_t x_block = 0, x_shift = 0;
+    // launch_gemm_ps_tiles with GEPI_RESIDUAL only, nullable: f32 [4][rows] as
+    // launch_vae_repack_pre; the sum goes through snake_pa(v ps + pt) to block-major
+    // planes oh, ol of o_block bytes a block (row -1 zeroed), and out is not written.
+    const float *pre = nullptr;
+    uint32_t o_block = 0;
     uint32_t o_tiled = 0;           // 1: GEPI_SWIGLU writes oh/ol in the tiled plane layout
     // GEPI_RESIDUAL with ksplit > 1 on the prefill-layout kernel: when set, split
     // s stores scale * (its partial product) to ws + s * ws_stride ([T][ldo]) with
@@ -500,6 +505,10 @@ int launch_gemm_pf(hipStream_t s, GemmArgs a);
 // picks below a whole token tile.
 bool gemm_ps_eligible(const GemmArgs &a);
 int launch_gemm_ps(hipStream_t s, GemmArgs a);
+// The same kernel over token tiles of any row count: one F16 matrix without a split,
+// GEPI_STORE from block-major planes or GEPI_RESIDUAL (a plain read and add) from tiled
+// ones.
+int launch_gemm_ps_tiles(hipStream_t s, GemmArgs a);
 // Tokens per workgroup tile of the kernel launch_gemm picks for these arguments.
 uint32_t gemm_tile_tokens(const GemmArgs &a);
 
@@ -624,18 +633,27 @@ struct VaeDwArgs {                  // depthwise conv over frame-major rows
     const __half *w = nullptr, *b = nullptr;            // [C][kernel], [C]
     const __half *alpha_in = nullptr, *alpha_out = nullptr;   // nullable snakes
     uint32_t channels = 0, length = 0, kernel = 7, dilation = 1, left_pad = 0;
+    __half *yh = nullptr, *yl = nullptr;   // instead of y: hi/lo planes in the tiled layout (channels % 32 == 0)
 };
 int launch_vae_dwconv_fm(hipStream_t s, const VaeDwArgs &a);
-// A decoder residual unit in one pass (32, 64, 128 or 256 channels), parameters and
+// Block-major hi/lo planes of a stage's input P (GemmArgs::x_block): `block` bytes
+// between 32-channel blocks of [row][32] halves, the rows' chunks permuted as in the
+// tiled layout, h and l at row 0; every block has a row -1, which the producer zeroes.
+struct VaePlanes {
+    __half *h = nullptr, *l = nullptr;
+    uint32_t block = 0;
+};
+// A decoder residual unit in one pass (32 to 512 channels, powers of two), parameters and
 // 1x1 weight as launch_vae_repack_unit lays them out; pre (nullable, f32 [4][C] as
-// launch_vae_repack_pre) also applies the next stage's input transform. y must not
-// alias x.
+// launch_vae_repack_pre) also applies the next stage's input transform and writes its
+// planes instead of y. y must not alias x.
 struct VaeUnitArgs {
     const float *x = nullptr;
     float *y = nullptr;
     const float *p = nullptr;
     const __half *w = nullptr;
     const float *pre = nullptr;
+    VaePlanes planes;
     uint32_t channels = 0, length = 0, dilation = 1;
 };
 bool vae_unit_channels(uint32_t channels);
@@ -644,10 +662,13 @@ int launch_vae_repack_unit(hipStream_t s, const __half *a1, const __half *dw, co
                            const __half *pw, const __half *pb, uint32_t channels, float *p, __half *w);
 // y = snake_pa(x * ps + pt) per channel, pre as launch_vae_repack_pre lays it out.
 int launch_vae_pre_fm(hipStream_t s, const float *x, float *y, const float *pre, uint32_t channels, uint32_t length);
+// The same into planes (channels % 32 == 0).
+int launch_vae_pre_planes(hipStream_t s, const float *x, const VaePlanes &y, const float *pre, uint32_t channels,
+                          uint32_t length);
 int launch_vae_repack_pre(hipStream_t s, const __half *scale, const __half *bias, const __half *alpha,
                           uint32_t channels, float *pre);
 int launch_vae_repack_convt(hipStream_t s, const __half *w, const __half *b, uint32_t cin, uint32_t cout,
-                            uint32_t stride, __half *wp, float *bp);
+                            uint32_t stride, uint32_t prefill_layout, __half *wp, float *bp);
 struct VaeLinearArgs {              // y[t][n] (+)= b[n] + x[t] . W[n], short K
     const float *x = nullptr;
     uint32_t ldx = 0;
