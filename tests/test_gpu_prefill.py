@@ -227,6 +227,32 @@ def test_batched_prefill_short_chunks(ctx, weights):
     model.free()
 
 
+@pytest.mark.parametrize("weights", ["q8_0", "f16"])
+def test_batched_prefill_long_chunks(ctx, weights):
+    """2101 tokens in one call (a whole 2048-row chunk and a short one) against the same
+    tokens in calls of 130, 500, 700, 641 and 130: other tile counts, splits and chunk
+    edges, the same cache rows and state to rounding."""
+    print(f"long chunks {weights}", flush=True)
+    cfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=2112)
+    m = synth.build_baselm(cfg, seed=0x5EED0140, weight_type=weights)
+    model = Model(ctx, m.data, m.tensors)
+    toks = [int(t) for t in synth.uniform_u32(2101, 0x5EED0141, cfg["vocab_size"])]
+    got = []
+    for calls in ([2101], [130, 500, 700, 641, 130]):
+        eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False)
+        done = 0
+        for n in calls:
+            eng.prefill_tokens_batched(toks[done:done + n])
+            done += n
+        got.append((eng.output(), kv_rows(eng, "kv_k", 2, 2112), kv_rows(eng, "kv_v", 2, 2112)))
+        eng.close()
+    assert rel_l2(got[0][0], got[1][0]) < 1e-3
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert rel_l2(f16(a[:, :2101]), f16(b[:, :2101])) < 1e-3
+        assert np.all(a[:, 2101:] == 0) and np.all(b[:, 2101:] == 0)
+    model.free()
+
+
 def test_batched_prefill_errors(ctx, small):
     cfg, m, model = small
     eng = BaseLmEngine(ctx, model, dict(cfg, active_context_length=64), exec_mode="graph", strict_geometry=False)

@@ -547,13 +547,13 @@ int enqueue_prefill_chunk(vx_baselm *e, const uint32_t *tok, uint32_t pos0, uint
     {
         ProfSpan sp(ctx, "prefill.embedding");
         VX_CHECK(launch_seq_embedding(s, e->model->raw, e->embd_offset, e->embd_dtype, nH, tok, T, c.vocab_size,
-                                      e->embedding_alpha, F(e->pf.h), nH));
+                                      e->embedding_alpha, e->pf.h, nH));
     }
     VX_CHECK(enqueue_prefill_stack(make_stack(e), pos0, T));
     if (rows) {   // every token's output_buffer (rmsnorm(h)*output_norm), as the decode step leaves it
         ProfSpan sp(ctx, "prefill.output_rows");
         SeqNormArgs n;
-        n.h = F(e->pf.h);
+        n.h = e->pf.h;
         n.ldh = nH;
         n.w = e->output_norm;
         n.n = nH;
@@ -565,7 +565,7 @@ int enqueue_prefill_chunk(vx_baselm *e, const uint32_t *tok, uint32_t pos0, uint
     // Engine state after the chunk: hidden = last token's residual stream, norm =
     // its rmsnorm(h)*output_norm (record_transformer's final residual_rmsnorm).
     ProfSpan sp(ctx, "prefill.output_norm");
-    const float *last = F(e->pf.h) + (size_t)(T - 1u) * nH;
+    const float *last = e->pf.h + (size_t)(T - 1u) * nH;
     VX_HIP(hipMemcpyAsync(e->hidden->ptr, last, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
     return launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr);
 }

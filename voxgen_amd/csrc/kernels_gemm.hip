@@ -578,9 +578,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_pf(GemmArgs a) {
         // LDS (the ring is free once every wave has drained its DMA) in two passes
         // of 64 tokens and leave as 16-byte stores, 512 contiguous bytes per token
         // row, instead of 4-byte stores scattered over every lane's 64 results.
-        // An F16 residual product without a split is added to its output the same way
-        // (Q8_0 ones that large do not occur in a 512-row chunk).
-        const bool add = WK == WT_F16 && EPI == GEPI_RESIDUAL && a.ksplit == 1u;
+        // A residual product without a split is added to its output the same way.
+        const bool add = EPI == GEPI_RESIDUAL && a.ksplit == 1u;
         const bool plain = EPI == GEPI_STORE ? (a.ksplit == 1u || a.split_store != 0u) : (add || a.ws != nullptr);
         if (plain && a.wide) {
             float *const base = EPI == GEPI_STORE ? out0 + (a.ksplit > 1u ? ks * a.ws_stride : 0u)

@@ -5,7 +5,7 @@
 //   per layer over the rows of the residual stream h:
 //     rmsnorm(h)*attn_norm -> f16 hi/lo planes        (k_seq_rmsnorm)
 //     q|k|v = planes . Wq|Wk|Wv                       (k_gemm, split-K)
-//     RoPE at pos0+t (or none), K/V rows -> f16 cache, q planes  (k_seq_rope_store)
+//     RoPE at pos0+t (or none), K/V rows -> f16 cache, q planes  (k_prefill_rope)
 //     causal attention over cache keys 0..pos0+t       (k_prefill_attn)
 //     h += scale * Wo . attn                           (k_gemm residual)
 //     rmsnorm(h)*ffn_norm -> planes                    (k_seq_rmsnorm)
@@ -14,6 +14,7 @@
 // Row t computes what the decode step computes at position pos0 + t: the same
 // KV-cache rows and the same residual stream, to rounding.
 #include <algorithm>
+#include <type_traits>
 
 #include "vx_internal.h"
 
@@ -21,8 +22,6 @@ namespace vx {
 
 namespace {
 
-inline float *F(vx_buf *b) { return static_cast<float *>(b->ptr); }
-inline __half *H(vx_buf *b) { return static_cast<__half *>(b->ptr); }
 
 // Split-K factor for a projection of n_tiles 128-row tiles and tt-token tiles:
 // as many workgroups as fit one per CU (rounded down: a second workgroup on a CU
@@ -44,6 +43,12 @@ uint32_t pick_split_short(const vx_ctx *ctx, uint32_t n_tiles, uint32_t K) {
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
     return std::max<uint32_t>(1u, std::min({cus / n_tiles, K / 128u, kPrefillMaxSplit}));
 }
+
+// Rows from one partial slab to the next, at least. Slabs close together slow the GEMM
+// that writes them and the one after it: four Q8_0 layers at 200 / 256 / 384 rows took
+// 474 / 502 / 617 us with slabs of exactly those rows (and 64 to 2048 floats more), 459 /
+// 488 / 610 with 512 rows, 455 / 473 / 602 with 1000 or 1024.
+constexpr uint32_t kSlabRows = 1024u;
 
 GemmSeg gemm_seg(const WRef &w, uint32_t rows, float *out, uint32_t ldo) {
     GemmSeg g;
@@ -134,41 +139,51 @@ int prefill_stack_alloc(vx_ctx *ctx, uint32_t cap, uint32_t nH, uint32_t nF, uin
     if (w->cap) return VX_OK;
     const uint64_t H = nH, F = nF, KV = nKV, T = cap;
     const uint64_t Tp = (T + 127u) / 128u * 128u;   // GEMM input planes: whole 128-token tiles
-    VX_CHECK(vx_alloc(ctx, T * H * 4u, &w->h));
-    VX_CHECK(vx_alloc(ctx, Tp * H * 2u, &w->xh));
-    VX_CHECK(vx_alloc(ctx, Tp * H * 2u, &w->xl));
-    VX_CHECK(vx_alloc(ctx, Tp * F * 2u, &w->ah));
-    VX_CHECK(vx_alloc(ctx, Tp * F * 2u, &w->al));
-    VX_CHECK(vx_alloc(ctx, T * H * 2u, &w->qh));
-    VX_CHECK(vx_alloc(ctx, T * H * 2u, &w->ql));
-    VX_CHECK(vx_alloc(ctx, T * H * 4u, &w->q));
-    VX_CHECK(vx_alloc(ctx, T * KV * 4u, &w->k));
-    VX_CHECK(vx_alloc(ctx, T * KV * 4u, &w->v));
     // Split-K partials: of the residual projections ([split][T][H]) and of QKV
-    // ([split][T][H + 2 KV]); the two uses never overlap in time.
-    VX_CHECK(vx_alloc(ctx, (uint64_t)kPrefillMaxSplit * T * (H + 2u * KV) * 4u, &w->ws));
+    // ([split][T][H + 2 KV]); the two uses never overlap in time. A split of more than one
+    // has at most a workgroup per CU (pick_split), which bounds split * T above kSlabRows.
+    const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
+    const uint64_t ws_rows =
+        std::max<uint64_t>(kPrefillMaxSplit * kSlabRows, 128u * (uint64_t)cus / ((H + 127u) / 128u));
     // Stream-K SwiGLU: two tile parts per workgroup and a counter per workgroup
     // boundary, one workgroup per CU; the counters start at zero.
-    const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
     w->sk_grid = cus / 8u * 8u;
-    if (w->sk_grid) {
-        VX_CHECK(vx_alloc(ctx, (uint64_t)w->sk_grid * 2u * kSkTileFloats * 4u, &w->sk_ws));
-        VX_CHECK(vx_alloc(ctx, (uint64_t)w->sk_grid * 4u, &w->sk_cnt));
-        VX_HIP(hipMemsetAsync(w->sk_cnt->ptr, 0, w->sk_cnt->bytes, ctx->stream));
-    }
+    // One allocation: a new engine's first prefill waits for each.
+    uint64_t bytes = 0;
+    uint8_t *base = nullptr;
+    auto lay = [&]() {
+        bytes = 0;
+        auto put = [&](auto *&ptr, uint64_t n) {
+            ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + bytes);
+            bytes += (n + 255u) / 256u * 256u;
+        };
+        put(w->h, T * H * 4u);
+        put(w->xh, Tp * H * 2u);
+        put(w->xl, Tp * H * 2u);
+        put(w->ah, Tp * F * 2u);
+        put(w->al, Tp * F * 2u);
+        put(w->qh, T * H * 2u);
+        put(w->ql, T * H * 2u);
+        put(w->q, T * H * 4u);
+        put(w->k, T * KV * 4u);
+        put(w->v, T * KV * 4u);
+        put(w->ws, ws_rows * (H + 2u * KV) * 4u);
+        put(w->rope, T * 64u * 8u);   // head_dim <= 128
+        put(w->sk_ws, (uint64_t)w->sk_grid * 2u * kSkTileFloats * 4u);
+        put(w->sk_cnt, (uint64_t)w->sk_grid * 4u);
+    };
+    lay();
+    VX_CHECK(vx_alloc(ctx, bytes, &w->arena));
+    base = static_cast<uint8_t *>(w->arena->ptr);
+    lay();
+    if (w->sk_grid) VX_HIP(hipMemsetAsync(w->sk_cnt, 0, (size_t)w->sk_grid * 4u, ctx->stream));
     w->cap = cap;
     return VX_OK;
 }
 
 void prefill_stack_free(vx_ctx *ctx, StackWork *w) {
-    vx_buf **bufs[] = {&w->h,  &w->xh, &w->xl, &w->ah, &w->al,    &w->qh,
-                       &w->ql, &w->q,  &w->k,  &w->v,  &w->ws, &w->sk_ws, &w->sk_cnt};
-    for (vx_buf **b : bufs) {
-        if (*b) vx_free(ctx, *b);
-        *b = nullptr;
-    }
-    w->cap = 0;
-    w->sk_grid = 0;
+    if (w->arena) vx_free(ctx, w->arena);
+    *w = StackWork();
 }
 
 int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
@@ -189,39 +204,41 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
     const uint32_t ks_qkv = split(nH, nKV, nH), ks_o = split(nH, 0, nH), ks_down = split(nH, 0, nF);
     // Split residual projections on the tiled path leave their partials in
     // the workspace; the next rmsnorm adds them to h (no atomics in the GEMM epilogue).
-    const uint64_t ws_stride = (uint64_t)w.cap * nH;
+    const uint32_t slab = std::max(T, kSlabRows);
+    const uint64_t ws_stride = (uint64_t)slab * nH;
     const bool ws_o = tiled && ks_o > 1, ws_down = tiled && ks_down > 1;
     // Split QKV on the tiled path stores its partials to the workspace as well (q, k, v
     // regions of one split, ws_qkv floats per split); the RoPE kernel sums them.
     const bool ws_qkv = tiled && ks_qkv > 1;
-    const uint64_t ws_qkv_stride = (uint64_t)w.cap * (nH + 2u * nKV);
-    float *const wq = F(w.ws), *const wk = wq + (size_t)w.cap * nH, *const wv = wk + (size_t)w.cap * nKV;
+    const uint64_t ws_qkv_stride = (uint64_t)slab * (nH + 2u * nKV);
+    float *const wq = w.ws, *const wk = wq + (size_t)slab * nH, *const wv = wk + (size_t)slab * nKV;
+    float2 *const rope = p.rope ? w.rope : nullptr;
     for (uint32_t l = 0; l < p.n_layers; ++l) {
         const StackLayer &L = p.layers[l];
         {
             ProfSpan sp(ctx, "prefill.norm");
             SeqNormArgs n;
-            n.h = F(w.h);
+            n.h = w.h;
             n.ldh = nH;
             n.w = L.attn_norm;
             if (l > 0 && ws_down) {
-                n.branch = F(w.ws);
+                n.branch = w.ws;
                 n.ldb = nH;
                 n.nbranch = ks_down;
                 n.branch_stride = ws_stride;
             }
             n.n = nH;
             n.eps = p.eps;
-            n.yh = H(w.xh);
-            n.yl = H(w.xl);
+            n.yh = w.xh;
+            n.yl = w.xl;
             n.ldp = nH;
             n.tiled = tiled ? 1u : 0u;
             if (ks_qkv > 1 && !ws_qkv) {
-                n.zero[0] = F(w.q);
+                n.zero[0] = w.q;
                 n.zero_n[0] = nH;
-                n.zero[1] = F(w.k);
+                n.zero[1] = w.k;
                 n.zero_n[1] = nKV;
-                n.zero[2] = F(w.v);
+                n.zero[2] = w.v;
                 n.zero_n[2] = nKV;
             }
             VX_CHECK(launch_seq_rmsnorm(s, n, T));
@@ -231,9 +248,9 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             GemmArgs g;
             g.wk = L.q.wt;
             g.epi = GEPI_STORE;
-            g.seg[0] = gemm_seg(L.q, nH, F(w.q), nH);
-            g.seg[1] = gemm_seg(L.k, nKV, F(w.k), nKV);
-            g.seg[2] = gemm_seg(L.v, nKV, F(w.v), nKV);
+            g.seg[0] = gemm_seg(L.q, nH, w.q, nH);
+            g.seg[1] = gemm_seg(L.k, nKV, w.k, nKV);
+            g.seg[2] = gemm_seg(L.v, nKV, w.v, nKV);
             if (tiled) {
                 const StackPrefillWeights &P = p.pw[l];
                 g.seg[0].pq = P.q.q;
@@ -247,8 +264,8 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             g.nseg = 3;
             g.K = nH;
             g.T = T;
-            g.xh = H(w.xh);
-            g.xl = H(w.xl);
+            g.xh = w.xh;
+            g.xl = w.xl;
             g.ldx = nH;
             g.ksplit = ks_qkv;
             if (ws_qkv) {
@@ -263,9 +280,9 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
         {
             ProfSpan sp(ctx, "prefill.rope_store");
             SeqRopeArgs r;
-            r.q = ws_qkv ? wq : F(w.q);
-            r.k = ws_qkv ? wk : F(w.k);
-            r.v = ws_qkv ? wv : F(w.v);
+            r.q = ws_qkv ? wq : w.q;
+            r.k = ws_qkv ? wk : w.k;
+            r.v = ws_qkv ? wv : w.v;
             if (ws_qkv) {
                 r.nsplit = ks_qkv;
                 r.split_stride = ws_qkv_stride;
@@ -280,21 +297,22 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             r.theta = p.theta;
             r.scaling = p.rope_scaling;
             r.q_inplace = 0;
-            r.qh = H(w.qh);
-            r.ql = H(w.ql);
+            r.qh = w.qh;
+            r.ql = w.ql;
             r.ldqp = nH;
             r.kc = p.kc;
             r.vc = p.vc;
             r.no_rope = p.rope ? 0u : 1u;
             r.layer = l;
             r.context = p.context;
-            VX_CHECK(launch_seq_rope_store(s, r, T));
+            if (l == 0 && rope) VX_CHECK(launch_prefill_rope_table(s, r, T, rope));
+            VX_CHECK(launch_prefill_rope(s, r, T, rope));
         }
         {
             ProfSpan sp(ctx, "prefill.attention");
             PrefillAttnArgs a;
-            a.qh = H(w.qh);
-            a.ql = H(w.ql);
+            a.qh = w.qh;
+            a.ql = w.ql;
             a.ldq = nH;
             a.kc = p.kc;
             a.vc = p.vc;
@@ -305,8 +323,8 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             a.q_heads = p.q_heads;
             a.kv_heads = p.kv_heads;
             a.head_dim = p.head_dim;
-            a.oh = H(w.xh);
-            a.ol = H(w.xl);
+            a.oh = w.xh;
+            a.ol = w.xl;
             a.ldo = nH;
             a.tiled = tiled ? 1u : 0u;
             VX_CHECK(launch_prefill_attn(s, a));
@@ -316,7 +334,7 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             GemmArgs g;
             g.wk = L.o.wt;
             g.epi = GEPI_RESIDUAL;
-            g.seg[0] = gemm_seg(L.o, nH, F(w.h), nH);
+            g.seg[0] = gemm_seg(L.o, nH, w.h, nH);
             if (tiled) {
                 g.seg[0].pq = p.pw[l].o.q;
                 g.seg[0].pd = p.pw[l].o.d;
@@ -324,13 +342,13 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             }
             g.K = nH;
             g.T = T;
-            g.xh = H(w.xh);
-            g.xl = H(w.xl);
+            g.xh = w.xh;
+            g.xl = w.xl;
             g.ldx = nH;
             g.scale = p.residual_scale;
             g.ksplit = ks_o;
             if (ws_o) {
-                g.ws = F(w.ws);
+                g.ws = w.ws;
                 g.ws_stride = ws_stride;
             }
             VX_CHECK(launch_gemm(s, g));
@@ -338,19 +356,19 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
         {
             ProfSpan sp(ctx, "prefill.norm");
             SeqNormArgs n;
-            n.h = F(w.h);
+            n.h = w.h;
             n.ldh = nH;
             n.w = L.ffn_norm;
             if (ws_o) {
-                n.branch = F(w.ws);
+                n.branch = w.ws;
                 n.ldb = nH;
                 n.nbranch = ks_o;
                 n.branch_stride = ws_stride;
             }
             n.n = nH;
             n.eps = p.eps;
-            n.yh = H(w.xh);
-            n.yl = H(w.xl);
+            n.yh = w.xh;
+            n.yl = w.xl;
             n.ldp = nH;
             n.tiled = tiled ? 1u : 0u;
             VX_CHECK(launch_seq_rmsnorm(s, n, T));
@@ -371,15 +389,15 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             g.nseg = 2;
             g.K = nH;
             g.T = T;
-            g.xh = H(w.xh);
-            g.xl = H(w.xl);
+            g.xh = w.xh;
+            g.xl = w.xl;
             g.ldx = nH;
-            g.oh = H(w.ah);
-            g.ol = H(w.al);
+            g.oh = w.ah;
+            g.ol = w.al;
             g.ldp = nF;
             if (tiled && w.sk_grid && p.schedule != VX_PREFILL_TILES) {
-                g.sk_ws = F(w.sk_ws);
-                g.sk_cnt = static_cast<uint32_t *>(w.sk_cnt->ptr);
+                g.sk_ws = w.sk_ws;
+                g.sk_cnt = w.sk_cnt;
                 g.sk_grid = w.sk_grid;
                 g.sk_tail_first = p.schedule == VX_PREFILL_STREAMK_TAIL_FIRST ? 1u : 0u;
             }
@@ -390,7 +408,7 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             GemmArgs g;
             g.wk = L.down.wt;
             g.epi = GEPI_RESIDUAL;
-            g.seg[0] = gemm_seg(L.down, nH, F(w.h), nH);
+            g.seg[0] = gemm_seg(L.down, nH, w.h, nH);
             if (tiled) {
                 g.seg[0].pq = p.pw[l].down.q;
                 g.seg[0].pd = p.pw[l].down.d;
@@ -398,13 +416,13 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             }
             g.K = nF;
             g.T = T;
-            g.xh = H(w.ah);
-            g.xl = H(w.al);
+            g.xh = w.ah;
+            g.xl = w.al;
             g.ldx = nF;
             g.scale = p.residual_scale;
             g.ksplit = ks_down;
             if (ws_down) {
-                g.ws = F(w.ws);
+                g.ws = w.ws;
                 g.ws_stride = ws_stride;
             }
             VX_CHECK(launch_gemm(s, g));
@@ -413,10 +431,10 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
     if (ws_down) {   // the last layer's down partials
         ProfSpan sp(ctx, "prefill.norm");
         SeqNormArgs n;
-        n.h = F(w.h);
+        n.h = w.h;
         n.ldh = nH;
         n.n = nH;
-        n.branch = F(w.ws);
+        n.branch = w.ws;
         n.ldb = nH;
         n.nbranch = ks_down;
         n.branch_stride = ws_stride;

@@ -636,15 +636,15 @@ int enqueue_prefill_rows(vx_residual *e, const float *rows, uint32_t T) {
         VX_HIP(hipMemcpy2DAsync(e->fuse_x->ptr, (size_t)c.fusion_input_dim * 4u, rows, (size_t)nH * 4u,
                                 (size_t)nH * 4u, T, hipMemcpyDeviceToDevice, s));
         VX_CHECK(enqueue_seq_linear(s, e->fusion.w, e->fusion.b, e->fusion.bt, nH, c.fusion_input_dim, T,
-                                    F(e->fuse_x), 0, c.fusion_input_dim, F(e->pf.h), 0, nH, 1.f));
+                                    F(e->fuse_x), 0, c.fusion_input_dim, e->pf.h, 0, nH, 1.f));
     }
-    const float *last_fused = F(e->pf.h) + (size_t)(T - 1u) * nH;
+    const float *last_fused = e->pf.h + (size_t)(T - 1u) * nH;
     VX_HIP(hipMemcpyAsync(e->fusion_snapshot->ptr, last_fused, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
     VX_HIP(hipMemcpyAsync(e->current_lm->ptr, rows + (size_t)(T - 1u) * nH, (size_t)nH * 4u,
                           hipMemcpyDeviceToDevice, s));
     VX_CHECK(enqueue_prefill_stack(make_stack(e), e->pos, T));
     ProfSpan sp(ctx, "residual.prefix_output_norm");
-    const float *last = F(e->pf.h) + (size_t)(T - 1u) * nH;
+    const float *last = e->pf.h + (size_t)(T - 1u) * nH;
     VX_HIP(hipMemcpyAsync(e->hidden->ptr, last, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
     VX_CHECK(launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr));
     e->pos += T;

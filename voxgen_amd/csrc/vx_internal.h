@@ -564,6 +564,11 @@ struct SeqRopeArgs {
     uint32_t no_rope = 0;               // 1: q/k pass through unrotated (factors unused)
 };
 constexpr uint32_t kSeqRopeMaxSplit = 8;
+// The prefill stack's form of the step below: cos and sin (times scaling) of every row's
+// position in a table [T][head_dim / 2], made once a chunk, and one pass from the sums of
+// the QKV products to q planes and cache rows (head_dim % 8 == 0, 16-byte aligned rows).
+int launch_prefill_rope_table(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens, float2 *tab);
+int launch_prefill_rope(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens, const float2 *tab);
 int launch_seq_rope_store(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens);
 
 // ------------------------------------------- token-batched decoder stack (prefill)
@@ -576,13 +581,20 @@ struct StackPrefillWeights {        // Q8_0 or F16 projections in the prefill-GE
 };
 struct StackWork {                  // activations of one chunk of rows (cap rows)
     uint32_t cap = 0;
-    vx_buf *h = nullptr;            // residual stream [cap][nH] f32: the input rows, then the output
-    vx_buf *xh = nullptr, *xl = nullptr, *ah = nullptr, *al = nullptr, *qh = nullptr, *ql = nullptr;
-    vx_buf *q = nullptr, *k = nullptr, *v = nullptr, *ws = nullptr;
-    vx_buf *sk_ws = nullptr, *sk_cnt = nullptr;   // stream-K SwiGLU tile parts and counters
+    vx_buf *arena = nullptr;        // one allocation holds everything below
+    float *h = nullptr;             // residual stream [cap][nH]: the input rows, then the output
+    __half *xh = nullptr, *xl = nullptr, *ah = nullptr, *al = nullptr, *qh = nullptr, *ql = nullptr;
+    float *q = nullptr, *k = nullptr, *v = nullptr, *ws = nullptr;
+    float2 *rope = nullptr;         // [cap][head_dim / 2] cos, sin of the chunk's positions
+    float *sk_ws = nullptr;         // stream-K SwiGLU tile parts and counters
+    uint32_t *sk_cnt = nullptr;
     uint32_t sk_grid = 0;                         // its workgroups: the CU count rounded down to 8
 };
-constexpr uint32_t kPrefillChunk = 512;     // rows per chunk
+// Rows per chunk. Against 512 (four Q8_0 layers on MI355X: 600 / 1200 / 1900 rows 1092 /
+// 1934 / 2872 us) 1024 gave 811 / 1747 / 2518 and 2048 814 / 1568 / 2190: fewer tiles run
+// beside an idle slot, the attention's workgroups overlap, and no split's slabs are
+// written and read. 2048 rows of work are 0.3 GB at the VoxCPM2 geometry.
+constexpr uint32_t kPrefillChunk = 2048;
 constexpr uint32_t kPrefillMaxSplit = 8;    // split-K factor bound
 constexpr uint32_t kSkTileFloats = 128u * 128u;   // accumulators of one 128 x 128 prefill GEMM tile
 struct PrefillStack {
