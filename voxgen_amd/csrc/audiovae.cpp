@@ -403,6 +403,42 @@ double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
+// Sum, sum of squares and largest magnitude of a wave, and whether a value is not finite.
+// Eight of each run side by side, so that the additions do not wait for one another
+// (92160 samples: 0.12 ms in one chain).
+struct WaveSums {
+    double sum = 0, sq = 0;
+    float peak = 0.f;
+    bool bad = false;
+};
+WaveSums wave_sums(const float *x, uint64_t n) {
+    constexpr uint64_t N = 8;
+    double sum[N] = {}, sq[N] = {};
+    float peak[N] = {};
+    uint32_t bad[N] = {};
+    auto take = [&](uint64_t i, uint64_t j) {
+        uint32_t bits;
+        std::memcpy(&bits, x + i, 4);
+        bad[j] |= (bits & 0x7f800000u) == 0x7f800000u ? 1u : 0u;
+        const float m = std::fabs(x[i]);
+        peak[j] = m > peak[j] ? m : peak[j];
+        sum[j] += x[i];
+        sq[j] += (double)x[i] * x[i];
+    };
+    uint64_t i = 0;
+    for (; i + N <= n; i += N)
+        for (uint64_t j = 0; j < N; ++j) take(i + j, j);
+    for (; i < n; ++i) take(i, 0);
+    WaveSums w;
+    for (uint64_t j = 0; j < N; ++j) {
+        w.sum += sum[j];
+        w.sq += sq[j];
+        w.peak = std::max(w.peak, peak[j]);
+        w.bad = w.bad || bad[j];
+    }
+    return w;
+}
+
 const void *model_ptr(const vx_model *m, uint32_t offset) { return m->raw + offset; }
 
 int check_span(const vx_model *m, uint32_t offset, uint64_t count, uint32_t dtype, const char *what) {
@@ -578,23 +614,17 @@ int vx_audiovae_decode_latents(vx_audiovae *e, const float *frame_major, uint64_
     VX_CHECK(enqueue_decode(e, F(e->io), (uint32_t)frames, F(e->wave)));
     VX_CHECK(vx_download(ctx, e->wave, 0, wave, samples * 4u));
     const double ms = now_ms() - t0;
-    double sum = 0, sq = 0;
-    float peak = 0.f;
-    for (uint64_t i = 0; i < samples; ++i) {
-        if (!std::isfinite(wave[i])) return fail(VX_ERR_STATE, "AudioVAE decoder produced NaN/inf");
-        sum += wave[i];
-        sq += (double)wave[i] * wave[i];
-        peak = std::max(peak, std::fabs(wave[i]));
-    }
+    const WaveSums w = wave_sums(wave, samples);
+    if (w.bad) return fail(VX_ERR_STATE, "AudioVAE decoder produced NaN/inf");
     if (out) {
         out->latent_frames = (uint32_t)frames;
         out->latent_patches = (uint32_t)(frames / c.patch_size);
         out->output_samples = (uint32_t)samples;
         out->output_sample_rate = c.out_sample_rate;
         out->duration_seconds = (double)samples / c.out_sample_rate;
-        out->checksum = sum;
-        out->l2 = std::sqrt(sq);
-        out->peak = peak;
+        out->checksum = w.sum;
+        out->l2 = std::sqrt(w.sq);
+        out->peak = w.peak;
         out->decode_ms = ms;
         out->scratch_bytes = vx_audiovae_scratch_bytes(e);
     }
