@@ -566,8 +566,7 @@ int enqueue_prefill_chunk(vx_baselm *e, const uint32_t *tok, uint32_t pos0, uint
     // its rmsnorm(h)*output_norm (record_transformer's final residual_rmsnorm).
     ProfSpan sp(ctx, "prefill.output_norm");
     const float *last = e->pf.h + (size_t)(T - 1u) * nH;
-    VX_HIP(hipMemcpyAsync(e->hidden->ptr, last, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
-    return launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr);
+    return launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr, F(e->hidden));
 }
 
 // Prefill n tokens at the engine position: upload the ids, run the chunks, leave

@@ -42,6 +42,44 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float *x, float *y, const
     if (advance && threadIdx.x == 0) *advance = *advance + 1u;
 }
 
+// The same for n = 1024 NV, 16-byte aligned rows: x and w in registers from one round of
+// loads (the loop above waits for each of its 2 n / 256 reads: 4.6 to 6.3 us at n = 2048
+// on MI355X). `copy` (nullable) receives x.
+template <int NV>
+__global__ __launch_bounds__(256) void k_rmsnorm4(const float *x, float *y, const float *w, float eps,
+                                                  uint32_t *advance, float *copy) {
+    __shared__ float red[4];
+    float4 v[NV], g[NV];
+    uint32_t at = 0;
+    if (advance) at = *advance;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        v[j] = reinterpret_cast<const float4 *>(x)[threadIdx.x + 256 * j];
+        g[j] = reinterpret_cast<const float4 *>(w)[threadIdx.x + 256 * j];
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) s += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    s = block_sum256(s, red);
+    const float inv_rms = 1.0f / sqrtf(s / (float)(1024 * NV) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        reinterpret_cast<float4 *>(y)[threadIdx.x + 256 * j] =
+            make_float4(v[j].x * inv_rms * g[j].x, v[j].y * inv_rms * g[j].y, v[j].z * inv_rms * g[j].z,
+                        v[j].w * inv_rms * g[j].w);
+        if (copy) reinterpret_cast<float4 *>(copy)[threadIdx.x + 256 * j] = v[j];
+    }
+    if (advance && threadIdx.x == 0) *advance = at + 1u;
+}
+
+// Two rows of n floats at once.
+__global__ __launch_bounds__(256) void k_copy_rows2(const float *a, float *ya, const float *b, float *yb, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    ya[i] = a[i];
+    yb[i] = b[i];
+}
+
 // residual_rmsnorm.comp:23-42.
 __global__ __launch_bounds__(256) void k_residual_rmsnorm(float *h, const float *branch, float *y,
                                                           const float *w, uint32_t n, float eps,
@@ -167,9 +205,28 @@ __global__ void k_fill_u32(uint32_t *dst, uint32_t value, uint64_t count) {
 }  // namespace
 
 int launch_rmsnorm(hipStream_t s, const float *x, float *y, const float *w, uint32_t n, float eps,
-                   uint32_t *advance_position) {
+                   uint32_t *advance_position, float *copy) {
+    if ((n == 1024u || n == 2048u || n == 4096u) &&
+        ((uintptr_t)x | (uintptr_t)y | (uintptr_t)w | (uintptr_t)copy) % 16u == 0) {
+        if (n == 1024u)
+            k_rmsnorm4<1><<<1, 256, 0, s>>>(x, y, w, eps, advance_position, copy);
+        else if (n == 2048u)
+            k_rmsnorm4<2><<<1, 256, 0, s>>>(x, y, w, eps, advance_position, copy);
+        else
+            k_rmsnorm4<4><<<1, 256, 0, s>>>(x, y, w, eps, advance_position, copy);
+        VX_LAUNCHED("k_rmsnorm4");
+        return VX_OK;
+    }
+    if (copy) VX_HIP(hipMemcpyAsync(copy, x, (size_t)n * 4u, hipMemcpyDeviceToDevice, s));
     k_rmsnorm<<<1, 256, 0, s>>>(x, y, w, n, eps, advance_position);
     VX_LAUNCHED("k_rmsnorm");
+    return VX_OK;
+}
+
+int launch_copy_rows2(hipStream_t s, const float *a, float *ya, const float *b, float *yb, uint32_t n) {
+    if (!n) return VX_OK;
+    k_copy_rows2<<<(n + 255u) / 256u, 256, 0, s>>>(a, ya, b, yb, n);
+    VX_LAUNCHED("k_copy_rows2");
     return VX_OK;
 }
 

@@ -639,14 +639,12 @@ int enqueue_prefill_rows(vx_residual *e, const float *rows, uint32_t T) {
                                     F(e->fuse_x), 0, c.fusion_input_dim, e->pf.h, 0, nH, 1.f));
     }
     const float *last_fused = e->pf.h + (size_t)(T - 1u) * nH;
-    VX_HIP(hipMemcpyAsync(e->fusion_snapshot->ptr, last_fused, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
-    VX_HIP(hipMemcpyAsync(e->current_lm->ptr, rows + (size_t)(T - 1u) * nH, (size_t)nH * 4u,
-                          hipMemcpyDeviceToDevice, s));
+    VX_CHECK(launch_copy_rows2(s, last_fused, F(e->fusion_snapshot), rows + (size_t)(T - 1u) * nH,
+                               F(e->current_lm), nH));
     VX_CHECK(enqueue_prefill_stack(make_stack(e), e->pos, T));
     ProfSpan sp(ctx, "residual.prefix_output_norm");
     const float *last = e->pf.h + (size_t)(T - 1u) * nH;
-    VX_HIP(hipMemcpyAsync(e->hidden->ptr, last, (size_t)nH * 4u, hipMemcpyDeviceToDevice, s));
-    VX_CHECK(launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr));
+    VX_CHECK(launch_rmsnorm(s, last, F(e->norm), e->output_norm, nH, c.rms_epsilon, nullptr, F(e->hidden)));
     e->pos += T;
     return launch_set_step(s, nullptr, U(e->position), e->pos, 0, 0);
 }

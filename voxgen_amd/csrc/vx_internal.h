@@ -317,7 +317,8 @@ int launch_attn_combine(hipStream_t s, const AttnLaunch &a);
 
 // Reference-granular kernels.
 int launch_rmsnorm(hipStream_t s, const float *x, float *y, const float *w, uint32_t n, float eps,
-                   uint32_t *advance_position);
+                   uint32_t *advance_position, float *copy = nullptr);   // copy (nullable): also y2 = x
+int launch_copy_rows2(hipStream_t s, const float *a, float *ya, const float *b, float *yb, uint32_t n);
 int launch_residual_rmsnorm(hipStream_t s, float *h, const float *branch, float *y, const float *w,
                             uint32_t n, float eps, float scale);
 int launch_rope(hipStream_t s, float *q, float *k, const float *factors, uint32_t position,
