@@ -109,8 +109,10 @@ int vx_diag_timeline_arm(vx_ctx *ctx, uint64_t waves) {
     // those stay allocated until the process ends.
     t = Timeline{};
     void *p = nullptr;
-    if (hipMalloc(&p, waves * 16u) != hipSuccess) return fail(VX_ERR_OOM, "vx_diag_timeline_arm: %llu records",
-                                                              (unsigned long long)waves);
+    if (hipMalloc(&p, waves * 16u) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(VX_ERR_OOM, "vx_diag_timeline_arm: %llu records", (unsigned long long)waves);
+    }
     VX_HIP(hipMemset(p, 0, waves * 16u));
     VX_HIP(hipDeviceSynchronize());
     t.ticks = static_cast<uint64_t *>(p);

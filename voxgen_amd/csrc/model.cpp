@@ -173,6 +173,7 @@ int vx_model_upload(vx_ctx *ctx, const void *data, uint64_t bytes, const vx_tens
     m->raw_bytes = (bytes + 255u) & ~255ull;
     hipError_t e = hipMalloc(&m->raw, m->raw_bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         delete m;
         return fail(VX_ERR_OOM, "hipMalloc of %llu-byte model region failed: %s",
                     (unsigned long long)bytes, hipGetErrorString(e));
@@ -180,6 +181,7 @@ int vx_model_upload(vx_ctx *ctx, const void *data, uint64_t bytes, const vx_tens
     if (packed_total) {
         e = hipMalloc(&m->packed, packed_total);
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             (void)hipFree(m->raw);
             delete m;
             return fail(VX_ERR_OOM, "hipMalloc of %llu-byte repack arena failed: %s",
@@ -192,6 +194,7 @@ int vx_model_upload(vx_ctx *ctx, const void *data, uint64_t bytes, const vx_tens
         e = hipMemcpyAsync(m->raw, data, bytes, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         vx_model_free(ctx, m);
         return fail(VX_ERR_HIP, "model upload failed: %s", hipGetErrorString(e));
     }
@@ -219,6 +222,7 @@ int vx_model_upload(vx_ctx *ctx, const void *data, uint64_t bytes, const vx_tens
     }
     e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         vx_model_free(ctx, m);
         return fail(VX_ERR_HIP, "model repack failed: %s", hipGetErrorString(e));
     }

@@ -48,7 +48,10 @@ static hipEvent_t take_event(vx_ctx *ctx) {
         return e;
     }
     hipEvent_t e = nullptr;
-    if (hipEventCreate(&e) != hipSuccess) return nullptr;
+    if (hipEventCreate(&e) != hipSuccess) {
+        (void)hipGetLastError();   // the span is dropped, the step goes on
+        return nullptr;
+    }
     return e;
 }
 
@@ -177,9 +180,11 @@ int vx_alloc(vx_ctx *ctx, uint64_t bytes, vx_buf **out) {
     VX_HIP(hipSetDevice(ctx->device));
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // callers may go on without the buffer
         return fail(VX_ERR_OOM, "hipMalloc(%llu) failed: %s", (unsigned long long)bytes,
                     hipGetErrorString(e));
+    }
     vx_buf *b = new vx_buf();
     b->ptr = p;
     b->bytes = bytes;
@@ -278,6 +283,7 @@ int vx_graph_end(vx_ctx *ctx, vx_graph **out) {
     hipGraphExec_t ex = nullptr;
     hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         (void)hipGraphDestroy(g);
         return fail(VX_ERR_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
     }

@@ -20,12 +20,17 @@ void set_error_v(const char *fmt, va_list ap);
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 void clear_error();
 
+// A failed call stays the thread's last HIP error, through later calls that succeed,
+// until it is read: whoever reports one reads it, or the next launch check would find
+// it and report a launch that was fine.
 #define VX_HIP(call)                                                                      \
     do {                                                                                  \
         hipError_t e_ = (call);                                                           \
-        if (e_ != hipSuccess)                                                             \
+        if (e_ != hipSuccess) {                                                           \
+            (void)hipGetLastError();                                                      \
             return ::vx::fail(VX_ERR_HIP, "%s failed: %s (%s:%d)", #call,                 \
                               hipGetErrorString(e_), __FILE__, __LINE__);                 \
+        }                                                                                 \
     } while (0)
 
 #define VX_CHECK(expr)                        \
