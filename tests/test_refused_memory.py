@@ -84,6 +84,51 @@ assert launches("k_repack_prefill_f16") == 12 and launches("k_gemm_ps") == 8
 """)
 
 
+def test_text_prefix_workspace_refused_in_part(fake):
+    """Each buffer of the ResidualLM's batched prefix refused in turn: the call fails,
+    and the call after it, with room again, allocates what is missing and runs. The
+    weight copy comes last, so that it cannot take the room of what is needed."""
+    child(fake, """
+cfg = synth.acoustic_config(layers=2, hidden=256, ffn=512, q_heads=2, kv_heads=1, latent=64, active_context=256)
+m = synth.build_acoustic(cfg, seed=2)
+model = Model(ctx, m.data, m.tensors)
+rows = ctx.zeros(256 * 256 * 4)
+copy = 2 * 2 * (2 * 256 * 256 + 2 * 128 * 256 + 3 * 512 * 256)
+for part in ((256 * 512 * 4,) * 2, (256 * 256 * 4,) * 2, (4 << 20, 1 << 40)):   # fusion input, rows, workspace
+    eng = ResidualFsqEngine(ctx, model, cfg, strict_geometry=False)
+    repacks = launches("k_repack_prefill")
+    refuse(*part)
+    for _ in range(2):
+        assert refused(eng.prefill_text_from_gpu_rows, rows, 37) == "VX_ERR_OOM"
+    assert launches("k_repack_prefill") == repacks and eng.position == 0
+    refuse(0, 0)
+    eng.prefill_text_from_gpu_rows(rows, 37)
+    assert launches("k_repack_prefill") == repacks + 12 and eng.position == 37
+    eng.close()
+eng = ResidualFsqEngine(ctx, model, cfg, strict_geometry=False)
+before = launches("k_gemm_ps")
+refuse(copy, copy + 2 * 6 * 256)
+eng.prefill_text_from_gpu_rows(rows, 37)
+assert eng.position == 37 and launches("k_gemm_ps") == before
+""")
+
+
+def test_baselm_prefill_token_buffer_refused(fake):
+    """The BaseLM's token buffer refused after its workspace: the next call allocates it."""
+    child(fake, """
+cfg = synth.baselm_config(layers=1, hidden=256, ffn=512, vocab=64, q_heads=2, kv_heads=1, context_length=320,
+                          active_context=320)
+m = synth.build_baselm(cfg, seed=1, weight_type="f16")
+model = Model(ctx, m.data, m.tensors)
+eng = BaseLmEngine(ctx, model, cfg, strict_geometry=False)
+refuse(320 * 4, 320 * 4)
+assert refused(eng.prefill_tokens_batched_gpu_only, [1] * 5) == "VX_ERR_OOM"
+refuse(0, 0)
+eng.prefill_tokens_batched_gpu_only([1] * 5)
+assert eng.position == 5
+""")
+
+
 @pytest.mark.gpu
 def test_refused_device_allocation_leaves_no_error_behind(ctx):
     """The same on the device: 2^50 bytes are more than any card has."""

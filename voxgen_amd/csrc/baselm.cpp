@@ -495,11 +495,10 @@ int run_step(vx_baselm *e, bool with_embedding, uint32_t token, bool logits) {
 // This computes what prefill_tokens (baselm.rs:823-839) computes one token at a
 // time: the same KV-cache rows and the same final state, to rounding.
 int ensure_prefill_work(vx_baselm *e) {
-    if (e->pf.cap) return VX_OK;
     const vx_baselm_config &c = e->cfg;
     const uint32_t cap = std::min<uint32_t>(kPrefillChunk, c.active_context_length);
     VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
-    return alloc(e->ctx, (uint64_t)c.active_context_length * 4u, &e->pf_tok);
+    return e->pf_tok ? VX_OK : alloc(e->ctx, (uint64_t)c.active_context_length * 4u, &e->pf_tok);
 }
 
 // The BaseLM layers as a token-batched stack (RoPE on, the engine's KV caches).

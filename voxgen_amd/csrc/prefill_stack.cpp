@@ -129,6 +129,8 @@ int prefill_stack_weights(vx_ctx *ctx, const StackLayer *layers, uint32_t n_laye
             (st = place(P.v, L.v, nullptr, nKV, nH)) || (st = place(P.o, L.o, nullptr, nH, nH)) ||
             (st = place(P.gu, L.gate, &L.up, nF, nH)) || (st = place(P.down, L.down, nullptr, nH, nF))) {
             pw->clear();
+            vx_free(ctx, *arena);
+            *arena = nullptr;
             return st;
         }
     }
@@ -176,7 +178,13 @@ int prefill_stack_alloc(vx_ctx *ctx, uint32_t cap, uint32_t nH, uint32_t nF, uin
     VX_CHECK(vx_alloc(ctx, bytes, &w->arena));
     base = static_cast<uint8_t *>(w->arena->ptr);
     lay();
-    if (w->sk_grid) VX_HIP(hipMemsetAsync(w->sk_cnt, 0, (size_t)w->sk_grid * 4u, ctx->stream));
+    if (w->sk_grid) {
+        const int st = launch_fill_u32(ctx->stream, w->sk_cnt, 0u, w->sk_grid);
+        if (st != VX_OK) {
+            prefill_stack_free(ctx, w);
+            return st;
+        }
+    }
     w->cap = cap;
     return VX_OK;
 }

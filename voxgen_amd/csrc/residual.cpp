@@ -78,6 +78,7 @@ struct vx_residual {
     std::vector<StackPrefillWeights> pw;   // the layers' prefill-layout weights ...
     vx_buf *pw_arena = nullptr;            // ... and their memory
     vx_buf *fuse_x = nullptr, *rows = nullptr;
+    bool pf_ready = false;   // all of the above exist (the weight copy if there was room)
 };
 
 namespace {
@@ -579,16 +580,16 @@ int predict_stop(vx_residual *e, const float *x, vx_stop_prediction *out) {
 // The engine state afterwards is the last position's, as after the per-position
 // steps: hidden, norm (output), fusion snapshot and current_lm (the raw row).
 int ensure_prefill_work(vx_residual *e) {
-    if (e->pf.cap) return VX_OK;
+    if (e->pf_ready) return VX_OK;
     const vx_acoustic_config &c = e->cfg;
     const uint32_t cap = std::min<uint32_t>(kPrefillChunk, c.active_context_length);
-    if (!e->pw_arena)
-        VX_CHECK(prefill_stack_weights(e->ctx, e->layers.data(), c.residual_block_count, c.embedding_length,
-                                       c.feed_forward_length, c.kv_dim, &e->pw, &e->pw_arena));
     VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
-    VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.fusion_input_dim * 4u, &e->fuse_x));
-    VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.embedding_length * 4u, &e->rows));
+    if (!e->fuse_x) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.fusion_input_dim * 4u, &e->fuse_x));
+    if (!e->rows) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.embedding_length * 4u, &e->rows));
     VX_HIP(hipMemsetAsync(e->fuse_x->ptr, 0, e->fuse_x->bytes, e->ctx->stream));
+    VX_CHECK(prefill_stack_weights(e->ctx, e->layers.data(), c.residual_block_count, c.embedding_length,
+                                   c.feed_forward_length, c.kv_dim, &e->pw, &e->pw_arena));
+    e->pf_ready = true;
     return VX_OK;
 }
 

@@ -620,7 +620,8 @@ int prefill_stack_check(const PrefillStack &p);
 // Repacks every layer's projections into the prefill-GEMM layout (53 MB a layer of
 // Q8_0, 94 MB of F16 at the VoxCPM2 geometry). Leaves *pw empty, so that prefill uses
 // the general GEMM, where the projections are not all Q8_0 or all F16, a width does
-// not fit, or the device has no room for the F16 copy.
+// not fit, or the device has no room for the F16 copy: call it after what the engine cannot
+// do without has been allocated.
 int prefill_stack_weights(vx_ctx *ctx, const StackLayer *layers, uint32_t n_layers, uint32_t nH, uint32_t nF,
                           uint32_t nKV, std::vector<StackPrefillWeights> *pw, vx_buf **arena);
 int prefill_stack_alloc(vx_ctx *ctx, uint32_t cap, uint32_t nH, uint32_t nF, uint32_t nKV, StackWork *w);
