@@ -177,3 +177,54 @@ def test_decode_errors(ctx):
     assert e.value.name == "VX_ERR_UNSUPPORTED"
     eng.close()
     model.free()
+
+
+def edited_case(ctx, dd, seed, edits):
+    """An engine and oracle over a synthetic decoder some of whose tensors (name ending
+    -> (mean, std) of normal values, clipped to the f16 range) are replaced."""
+    cfg = synth.audiovae_config(decoder_dim=dd)
+    m = synth.build_audiovae(cfg, seed=seed)
+    rng = np.random.default_rng(seed)
+    for t in m.tensors:
+        for end, (mean, std) in edits.items():
+            if t.name.endswith(end):
+                v = m.data[t.offset:t.offset + t.nbytes].view(np.float16)
+                v[:] = np.clip(rng.normal(mean, std, v.size), -65000, 65000).astype(np.float16)
+    model = Model(ctx, m.data, m.tensors)
+    eng = AudioVaeEngine(ctx, model, cfg, strict_geometry=False)
+    return model, eng, voxref.AudioVae(m.data, {t.name: t for t in m.tensors}, cfg)
+
+
+# The input of a 1x1 convolution, h = snake(depthwise), and of a transposed one, P =
+# snake(x scale + bias), far above the f16 range or far below it, with weights that bring
+# the result back: (std of the tensors before, after, snake alpha). With alphas of 1 the
+# snake's arguments also leave the reduced-range sine.
+SCALES = {"large": (3e4, 2e-6, 0.01), "large sine": (3e4, 2e-6, 1.0), "small": (3e-6, 2e4, 1.0)}
+
+
+@pytest.mark.parametrize("scale", list(SCALES))
+@pytest.mark.parametrize("dd,kind,stage", [(192, "unit", 2), (192, "convt", 3), (256, "convt", 5)])
+def test_narrow_products_keep_range_and_bits(ctx, dd, kind, stage, scale):
+    """Widths whose products are f32 (the 1x1 convolution of 96 channels, the transposed
+    ones from 96 and 32). f16 planes of such values would overflow, or keep a few bits
+    of them."""
+    print(f"vae narrow products {dd} {kind} stage {stage} {scale}", flush=True)
+    pre, post, al = SCALES[scale]
+    if kind == "unit":
+        p = "decoder.model.%d.block.{}.block." % stage
+        edits = {}
+        for r in (2, 3, 4):
+            edits |= {p.format(r) + "1": (0.0, pre), p.format(r) + "1.bias": (0.0, pre),
+                      p.format(r) + "2.alpha": (al, 0.1 * al), p.format(r) + "3": (0.0, post)}
+    else:
+        edits = {f"sr_cond_model.{stage}.scale_embed": (0.0, pre), f"sr_cond_model.{stage}.bias_embed": (0.0, pre),
+                 f"decoder.model.{stage}.block.0.alpha": (al, 0.1 * al),
+                 f"decoder.model.{stage}.block.1": (0.0, post)}
+    model, eng, o = edited_case(ctx, dd, 0x5EED0560 + dd, edits)
+    lat = synth.normal_f32(8 * 64, 0x5EED0561)
+    wave, want = eng.decode_latents(lat)[1], o.decode(lat)
+    err = rel_l2(wave, want)
+    print(f"rel_l2 {err:.2e} peak {np.abs(want).max():.2f}", flush=True)
+    assert np.abs(want).max() > 0.05 and err < 1e-5
+    eng.close()
+    model.free()

@@ -14,7 +14,8 @@
 //               32 to 512 channels: one pass             k_vae_unit
 //               else snake -> depthwise k=7 -> snake     k_vae_dw7_fm / k_vae_dwconv_*
 //               and x += 1x1 conv + bias                 k_gemm_pf / k_gemm_ps
-//             (widths that are no multiple of 32: P in f32, k_vae_linear_fm)
+//             (Cin no multiple of 64, or a 1x1 conv over channels that are none of 128:
+//             f32 products instead of planes, k_vae_linear_fm)
 //   head      snake -> conv k=7 to one channel -> tanh   k_vae_head_fm
 // Row j of the transposed convolution's output phases r = 0..s-1 is output time
 // s j + r, so the GEMM's [L][s Cout] output is the frame-major [s L][Cout] output.
@@ -44,7 +45,7 @@ struct Stage {
     const __half *scale = nullptr, *bias = nullptr, *alpha = nullptr;   // scale/bias rows of the bucket
     float *pre = nullptr;      // the same as f32 [4][Cin] (launch_vae_repack_pre)
     __half *ct_w = nullptr;    // [s Cout][2 Cin], in the prefill layout when planes
-    bool planes = false;       // P is kept as block-major planes (Cin % 32 == 0)
+    bool planes = false;       // P is kept as block-major planes, else in f32
     float *ct_b = nullptr;     // [s Cout]
     uint32_t stride = 1, cin = 0, cout = 0;
     Res res[3];
@@ -145,9 +146,17 @@ int grow(vx_ctx *ctx, vx_buf **b, uint64_t *cap, uint64_t floats) {
 // frames: 244 against 250 us).
 inline bool wide_run(uint32_t channels, uint32_t len) { return channels > 256u && (channels != 512u || len < 2048u); }
 
+// Whether a 1x1 or transposed convolution over `channels` (K of a product's columns)
+// takes its input as f16 hi and lo planes: 22 bits of a value, and 65504 is the largest.
+// The f32 kernel keeps every bit and the whole range; it takes the sums that are short
+// or odd (K no multiple of 128) up to its longest one.
+inline bool plane_products(uint32_t channels, uint32_t K) {
+    return channels % 32u == 0u && (K % 128u == 0u || K > kVaeLinearMaxK);
+}
+
 // Units whose 1x1 weight is kept for that GEMM.
 inline bool wide_unit(uint32_t channels) {
-    return channels % 32u == 0u && (!vae_unit_channels(channels) || wide_run(channels, 0u));
+    return plane_products(channels, channels) && (!vae_unit_channels(channels) || wide_run(channels, 0u));
 }
 // How plane_linear runs T rows of N outputs: small tiles of the register-streamed kernel
 // up to 64 tiles of 128 x 128, a quarter of the CUs (a limit of 16 or 160: 48 frames 511
@@ -326,7 +335,7 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
                 u.channels = ch;
                 u.length = len;
                 u.dilation = R.dilation;
-                have_pre = last;
+                have_pre = last && e->st[i + 1].planes;
                 if (have_pre) {
                     u.pre = e->st[i + 1].pre;
                     u.planes = planes_of(e->st[i + 1], len);
@@ -511,7 +520,7 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
             return bail(st);
         S.ct_w = reinterpret_cast<__half *>(cur);
         cur += up256(prefill_matrix_bytes(WT_F16, s * dout, 2u * din));
-        S.planes = din % 32u == 0u;
+        S.planes = plane_products(din, 2u * din);
         S.ct_b = reinterpret_cast<float *>(cur);
         cur += up256((uint64_t)s * dout * 4u);
         S.pre = reinterpret_cast<float *>(cur);

@@ -719,7 +719,7 @@ int launch_vae_repack_convt(hipStream_t s, const __half *w, const __half *b, uin
 
 int launch_vae_linear_fm(hipStream_t s, const VaeLinearArgs &a) {
     if (!a.T || !a.N) return VX_OK;
-    if (a.K > 4096u) return fail(VX_ERR_UNSUPPORTED, "vae linear: K %u > 4096", a.K);
+    if (a.K > kVaeLinearMaxK) return fail(VX_ERR_UNSUPPORTED, "vae linear: K %u > %u", a.K, kVaeLinearMaxK);
     const bool chunks = a.K % 8u == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0;
     const uint32_t NB = a.N < 256u ? a.N : 256u, G = 256u / NB;
     uint32_t rpt = 8192u / (G * a.K);

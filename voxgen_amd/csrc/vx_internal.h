@@ -699,6 +699,7 @@ struct VaeLinearArgs {              // y[t][n] (+)= b[n] + x[t] . W[n], short K
     uint32_t T = 0, N = 0, K = 0;
     uint32_t residual = 0;
 };
+constexpr uint32_t kVaeLinearMaxK = 4096;
 int launch_vae_linear_fm(hipStream_t s, const VaeLinearArgs &a);
 struct VaeHeadArgs {                // snake -> k-tap conv to one channel -> tanh
     const float *x = nullptr;
