@@ -203,10 +203,12 @@ SCALES = {"large": (3e4, 2e-6, 0.01), "large sine": (3e4, 2e-6, 1.0), "small": (
 
 
 @pytest.mark.parametrize("scale", list(SCALES))
-@pytest.mark.parametrize("dd,kind,stage", [(192, "unit", 2), (192, "convt", 3), (256, "convt", 5)])
+@pytest.mark.parametrize("dd,kind,stage", [(192, "unit", 2), (192, "convt", 3), (256, "convt", 5),
+                                           (256, "unit", 3), (256, "unit", 4)])
 def test_narrow_products_keep_range_and_bits(ctx, dd, kind, stage, scale):
     """Widths whose products are f32 (the 1x1 convolution of 96 channels, the transposed
-    ones from 96 and 32). f16 planes of such values would overflow, or keep a few bits
+    ones from 96 and 32) and those whose rows are scaled into the planes (the units of 64
+    and 32 channels). Plain f16 planes of such values would overflow, or keep a few bits
     of them."""
     print(f"vae narrow products {dd} {kind} stage {stage} {scale}", flush=True)
     pre, post, al = SCALES[scale]

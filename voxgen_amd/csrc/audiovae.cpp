@@ -489,7 +489,7 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
         arena += up256(prefill_matrix_bytes(WT_F16, s * dout, 2u * din)) + up256((uint64_t)s * dout * 4u) +
                  up256(din * 16u);
         if (wide_unit(dout)) arena += 3u * up256(prefill_matrix_bytes(WT_F16, dout, dout));
-        if (vae_unit_channels(dout)) arena += 3u * (up256(dout * 52u) + up256((uint64_t)dout * dout * 2u));
+        if (vae_unit_channels(dout)) arena += 3u * (up256(dout * kVaeUnitParams * 4u) + up256((uint64_t)dout * dout * 2u));
         din = dout;
     }
     if ((st = vx_alloc(ctx, arena, &e->arena))) return bail(st);
@@ -546,7 +546,7 @@ int vx_audiovae_create(vx_ctx *ctx, const vx_model *model, const vx_audiovae_con
             }
             if (!vae_unit_channels(dout)) continue;
             R.p = reinterpret_cast<float *>(cur);
-            cur += up256(dout * 52u);
+            cur += up256(dout * kVaeUnitParams * 4u);
             R.w = reinterpret_cast<__half *>(cur);
             cur += up256((uint64_t)dout * dout * 2u);
             if ((st = launch_vae_repack_unit(ctx->stream, R.a1, R.dw_w, R.dw_b, R.a2, R.pw_w, R.pw_b, dout, R.p, R.w)))

@@ -13,12 +13,20 @@
 // The planes are kept [row][KB] with the 16-byte chunks of a row permuted by the row
 // index, so that the A reads of 8 consecutive rows cover all banks.
 //
+// A pair of planes holds 22 bits of |h| < 65504, and from 2^-14 down fewer. Units of 32
+// and 64 channels, where f32 products are a choice, scale each row by a power of two
+// into the planes and back after the products, so that neither the range nor small rows
+// lose: 3 us a unit at 252 frames (64 channels 41.0 -> 44.2, 32 channels 32.8 -> 35.5).
+// Error of a decode against 64 bits, f32 products -> this: 1.7e-6 -> 1.5e-6, with h
+// around 1e5 in these units 4.1e-6 -> 3.5e-6, around 1e-5 2.8e-6 -> 2.5e-6 (unscaled:
+// not finite, 9e-3). Wider units keep the plain range of the GEMMs around them.
+//
 // Bound: x in and y out (8 bytes an element, 24 us a unit at 252 frames) against the
 // two snakes' vector work (about 60 instructions an element with the history rows, as
 // long again). Mean of the three units of a stage at 252 frames on MI355X, against a
 // depthwise pass and a GEMM with atomic adds (256, 128 channels) or f32 products from
 // LDS in one pass (64, 32): 256 channels 152 -> 63 us, 128 channels 110 -> 56, 64
-// channels 91 -> 41, 32 channels 62 -> 34. Larger tiles of 256 and 128 channels at one
+// channels 91 -> 44, 32 channels 62 -> 35. Larger tiles of 256 and 128 channels at one
 // workgroup of eight waves per CU were slower (79 and 60 us), and so was holding them
 // to 128 vector registers for two (140 and 100 us: spills). The unit that ends a stage
 // writes the next stage's planes: 15 us more at 256 channels (20 with an address a store), where a pass of its own
@@ -48,6 +56,12 @@ __device__ __forceinline__ float4 snake4(float4 x, float4 s, float4 inv) {
                        fmaf(sin_sq(s.w), inv.w, x.w));
 }
 
+// A lane exchange inside a row of 16 lanes (gfx9 DPP controls).
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+
 // Offset (in halves) of channel c of a row in a plane of KB channels.
 template <int KB>
 __device__ __forceinline__ uint32_t plane_at(uint32_t row, uint32_t c) {
@@ -66,6 +80,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
     __shared__ __attribute__((aligned(16))) float xs[(TB + kMaxHalo) * KB];
     __shared__ __attribute__((aligned(16))) _Float16 ph[TB * KB];
     __shared__ __attribute__((aligned(16))) _Float16 pl[TB * KB];
+    // Up to 64 channels a block is the whole row: the row's largest |h| is brought into
+    // [2^14, 2^15), and un[row] takes that back.
+    constexpr bool kScaled = NKB == 1;
+    __shared__ __attribute__((aligned(16))) float un[kScaled ? TB : 4];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, hs = lane >> 5;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wv / WN, wn = wv % WN;
@@ -92,7 +110,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
     for (uint32_t kb = 0; kb < (uint32_t)NKB; ++kb) {
         // Uniform bases of this block, opaque so that the loads keep them in scalar
         // registers with one lane offset instead of an address each in vector ones.
-        const float *pk = a.p + kb * (13u * KB);
+        const float *pk = a.p + kb * (kVaeUnitParams * KB);
         const __half *wk0 = a.w + ((size_t)(wn * NTL) * (C / 16) + kb * KS) * 512u;
         asm volatile("" : "+s"(pk), "+s"(wk0));
         float4 xv[NS];
@@ -161,6 +179,18 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
                 return s;
             };
             auto put = [&](uint32_t r, float4 v) {
+                if constexpr (kScaled) {
+                    // The largest of the row's G4 lanes, as bits (they order like the values).
+                    uint32_t m = max(__builtin_bit_cast(uint32_t, max4abs(0.f, v)), 15u << 23);
+                    m = max(m, dpp_u<0xb1>(m));    // quad_perm [1,0,3,2]
+                    m = max(m, dpp_u<0x4e>(m));    // quad_perm [2,3,0,1]
+                    m = max(m, dpp_u<0x141>(m));   // row_half_mirror
+                    if constexpr (G4 == 16) m = max(m, dpp_u<0x140>(m));   // row_mirror
+                    m &= 0x7f800000u;   // 2^(14 - e), and 2^(e - 14) to come back, of exponent e >= -112
+                    const float sc = __builtin_bit_cast(float, (268u << 23) - m);
+                    v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
+                    if (tid % G4 == 0u) un[r] = __builtin_bit_cast(float, m - (14u << 23));
+                }
                 const h4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
                 const h4 l = {(_Float16)(v.x - (float)h[0]), (_Float16)(v.y - (float)h[1]),
                               (_Float16)(v.z - (float)h[2]), (_Float16)(v.w - (float)h[3])};
@@ -179,17 +209,33 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
                 }
             }
             if (any_large(big)) {
+                if constexpr (kScaled) {
 #pragma unroll 1
-                for (uint32_t i = 4u * r0; i < 4u * TB; i = (i & 3u) == 3u ? i - 3u + 4u * RPP : i + 1u) {
-                    const uint32_t r = i >> 2, ce = c4 + (i & 3u);
-                    float u = pk[4 * KB + ce];
+                    for (uint32_t r = r0; r < (uint32_t)TB; r += RPP) {
+                        const float4 u = conv(r);
+                        float4 v = u, s = mul4(a2, u), q = i2;
 #pragma unroll 1
-                    for (uint32_t k = 0; k < 7u; ++k)
-                        u = fmaf(xs[(r + k * a.dilation) * KB + ce], pk[(6u + k) * KB + ce], u);
-                    u = fmaf(sin_sq_any(pk[2 * KB + ce] * u), pk[3 * KB + ce], u);
-                    const _Float16 h = (_Float16)u;
-                    ph[plane_at<KB>(r, ce)] = h;
-                    pl[plane_at<KB>(r, ce)] = (_Float16)(u - (float)h);
+                        for (int j = 0; j < 4; ++j) {   // the four channels in turn through the first place
+                            const float h = fmaf(sin_sq_any(s.x), q.x, v.x);
+                            v = make_float4(v.y, v.z, v.w, h);
+                            s = make_float4(s.y, s.z, s.w, s.x);
+                            q = make_float4(q.y, q.z, q.w, q.x);
+                        }
+                        put(r, v);
+                    }
+                } else {
+#pragma unroll 1
+                    for (uint32_t i = 4u * r0; i < 4u * TB; i = (i & 3u) == 3u ? i - 3u + 4u * RPP : i + 1u) {
+                        const uint32_t r = i >> 2, ce = c4 + (i & 3u);
+                        float u = pk[4 * KB + ce];
+#pragma unroll 1
+                        for (uint32_t k = 0; k < 7u; ++k)
+                            u = fmaf(xs[(r + k * a.dilation) * KB + ce], pk[(6u + k) * KB + ce], u);
+                        u = fmaf(sin_sq_any(pk[2 * KB + ce] * u), pk[3 * KB + ce], u);
+                        const _Float16 h = (_Float16)u;
+                        ph[plane_at<KB>(r, ce)] = h;
+                        pl[plane_at<KB>(r, ce)] = (_Float16)(u - (float)h);
+                    }
                 }
             }
         }
@@ -210,6 +256,21 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
         }
     }
     if (!mul) return;
+    if constexpr (kScaled) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const float4 f = ld4(un + 32 * (wm * MT + m) + 8 * (r >> 2) + 4 * hs);
+#pragma unroll
+                for (int n = 0; n < NTL; ++n) {
+                    acc[m][n][r] *= f.x;
+                    acc[m][n][r + 1] *= f.y;
+                    acc[m][n][r + 2] *= f.z;
+                    acc[m][n][r + 3] *= f.w;
+                }
+            }
+    }
 
     // Lane (l32, hs) holds channel n = 32 tile + l32 of rows 8 (r / 4) + 4 hs + r % 4.
     const uint32_t tb = 32u * wm * MT + 4u * hs;
@@ -224,16 +285,17 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
                     acc[m][n][r] = f(n, t, t * C + 32u * (wn * NTL + n) + l32, acc[m][n][r]);
                 }
     };
-    float pb[NTL];
+    float pb[NTL], ws[NTL];
 #pragma unroll
     for (int n = 0; n < NTL; ++n) {
         const uint32_t ch = 32u * (wn * NTL + n) + l32;
-        pb[n] = a.p[(ch / KB * 13u + 5u) * KB + ch % KB];
+        const float *const q = a.p + ch / KB * (kVaeUnitParams * KB) + ch % KB;
+        pb[n] = q[5 * KB], ws[n] = q[13 * KB];
     }
     if (full)
-        each([&](int n, uint32_t, uint32_t o, float v) { return xt[o] + (v + pb[n]); });
+        each([&](int n, uint32_t, uint32_t o, float v) { return xt[o] + fmaf(v, ws[n], pb[n]); });
     else
-        each([&](int n, uint32_t t, uint32_t o, float v) { return (t < have ? xt[o] : 0.f) + (v + pb[n]); });
+        each([&](int n, uint32_t t, uint32_t o, float v) { return (t < have ? xt[o] : 0.f) + fmaf(v, ws[n], pb[n]); });
     auto store = [&]() {
         if (full)
             each([&](int, uint32_t, uint32_t o, float v) { return yt[o] = v; });
@@ -327,27 +389,43 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
         finish([&](uint32_t t) { return t < have; });
 }
 
-// A unit's parameters as f32 [C / KB][13][KB], KB = min(C, 64): a1, 1/(a1 + 1e-9), a2,
-// 1/(a2 + 1e-9), db, pb, dw[7]; and its 1x1 weight in fragment order: block (n / 32,
+// A unit's parameters as f32 [C / KB][14][KB], KB = min(C, 64): a1, 1/(a1 + 1e-9), a2,
+// 1/(a2 + 1e-9), db, pb, dw[7], ws; and its 1x1 weight in fragment order: block (n / 32,
 // c / 16) of 64 lanes x 8 halves, lane l holding row n % 32 = l % 32, columns 8 (l / 32)...
+// Rows of the weight are multiplied by the power of two 1/ws that brings their largest
+// value into [2^14, 2^15): exact, and no weight is left subnormal whose products the
+// matrix cores would sum with fewer bits (error of a decode with weights of 2e-6 against
+// 64 bits: 8.0e-6 as they are, 3.5e-6 so, 4.1e-6 with f32 products). One workgroup a row.
 __global__ __launch_bounds__(256) void k_vae_repack_unit(const __half *a1, const __half *dw, const __half *db,
                                                          const __half *a2, const __half *pw, const __half *pb,
                                                          uint32_t C, float *p, __half *w) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x, KB = C < 64u ? C : 64u;
-    if (i < C) {
-        float *q = p + (i / KB) * 13u * KB + i % KB;
-        q[0] = vae_h2f(a1[i]);
-        q[KB] = snake_inv(vae_h2f(a1[i]));
-        q[2u * KB] = vae_h2f(a2[i]);
-        q[3u * KB] = snake_inv(vae_h2f(a2[i]));
-        q[4u * KB] = vae_h2f(db[i]);
-        q[5u * KB] = vae_h2f(pb[i]);
-        for (uint32_t k = 0; k < 7u; ++k) q[(6u + k) * KB] = vae_h2f(dw[i * 7u + k]);
+    __shared__ float part[4];
+    const uint32_t n = blockIdx.x, tid = threadIdx.x, KB = C < 64u ? C : 64u;
+    const __half *const row = pw + (size_t)n * C;
+    float m = 0.f;
+    for (uint32_t c = tid; c < C; c += 256u) m = fmaxf(m, fabsf(vae_h2f(row[c])));
+#pragma unroll
+    for (int d = 32; d; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    if ((tid & 63u) == 0u) part[tid >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+    int k = 0;   // 2^k m in [2^14, 2^15)
+    if (m > 0.f && m < 32768.0f) k = 14 - (int)((__builtin_bit_cast(uint32_t, m) >> 23) - 127u);
+    const float up = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
+    for (uint32_t c = tid; c < C; c += 256u) {
+        const uint32_t l = (n & 31u) + 32u * ((c >> 3) & 1u), b = n / 32u * (C / 16u) + c / 16u;
+        w[b * 512u + l * 8u + (c & 7u)] = __builtin_bit_cast(__half, (_Float16)(up * vae_h2f(row[c])));
     }
-    if (i < C * C) {
-        const uint32_t j = i & 7u, l = (i >> 3) & 63u, b = i >> 9, ks = b % (C / 16u), nt = b / (C / 16u);
-        w[i] = pw[(size_t)(32u * nt + (l & 31u)) * C + 16u * ks + 8u * (l >> 5) + j];
-    }
+    if (tid) return;
+    float *const q = p + n / KB * (kVaeUnitParams * KB) + n % KB;
+    q[0] = vae_h2f(a1[n]);
+    q[KB] = snake_inv(vae_h2f(a1[n]));
+    q[2u * KB] = vae_h2f(a2[n]);
+    q[3u * KB] = snake_inv(vae_h2f(a2[n]));
+    q[4u * KB] = vae_h2f(db[n]);
+    q[5u * KB] = vae_h2f(pb[n]);
+    for (uint32_t i = 0; i < 7u; ++i) q[(6u + i) * KB] = vae_h2f(dw[n * 7u + i]);
+    q[13u * KB] = __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
 }
 
 template <int C, int TB, int NW, int WM, int WN, int OCC>
@@ -363,7 +441,7 @@ bool vae_unit_channels(uint32_t c) { return c == 32u || c == 64u || c == 128u ||
 
 int launch_vae_repack_unit(hipStream_t s, const __half *a1, const __half *dw, const __half *db, const __half *a2,
                            const __half *pw, const __half *pb, uint32_t channels, float *p, __half *w) {
-    k_vae_repack_unit<<<(channels * channels + 255u) / 256u, 256, 0, s>>>(a1, dw, db, a2, pw, pb, channels, p, w);
+    k_vae_repack_unit<<<channels, 256, 0, s>>>(a1, dw, db, a2, pw, pb, channels, p, w);
     VX_LAUNCHED("k_vae_repack_unit");
     return VX_OK;
 }

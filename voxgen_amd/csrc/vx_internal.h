@@ -675,6 +675,7 @@ struct VaeUnitArgs {
     VaePlanes planes;
     uint32_t channels = 0, length = 0, dilation = 1;
 };
+constexpr uint32_t kVaeUnitParams = 14;   // f32 values a channel (launch_vae_repack_unit)
 bool vae_unit_channels(uint32_t channels);
 int launch_vae_unit(hipStream_t s, const VaeUnitArgs &a);
 int launch_vae_repack_unit(hipStream_t s, const __half *a1, const __half *dw, const __half *db, const __half *a2,
