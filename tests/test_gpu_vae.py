@@ -230,3 +230,16 @@ def test_narrow_products_keep_range_and_bits(ctx, dd, kind, stage, scale):
     assert np.abs(want).max() > 0.05 and err < 1e-5
     eng.close()
     model.free()
+
+
+@pytest.mark.parametrize("frames", [48, 132, 252])
+def test_decode_is_the_same_bit_for_bit(ctx, frames):
+    """Equal decodes give equal bits: no sum depends on which workgroup is first. 132 and
+    252 frames are 1056 and 2016 rows of 1024 channels, half the CUs' worth of tiles."""
+    print(f"vae bits {frames}", flush=True)
+    cfg, model, eng, lat, o = engine_case(ctx, 2048, frames, 0x5EED0570)
+    first = eng.decode_latents(lat)[1]
+    for _ in range(4):
+        assert np.array_equal(eng.decode_latents(lat)[1], first)
+    eng.close()
+    model.free()

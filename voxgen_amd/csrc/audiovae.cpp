@@ -173,8 +173,10 @@ inline uint64_t plane_block(uint64_t len) { return ((len + 127u) / 128u * 128u +
 // prefill layout: block-major planes (block, shift as GemmArgs) into y, or tiled ones
 // added to y.
 // Small tiles run without a split, which would sum atomically into a cleared output (a
-// launch more); 128 x 128 tiles that leave half the CUs idle over a long K take two (252
-// frames, 2016 rows x 1024: 27 -> 24 us; the first up-convolution 60 -> 48 + 5).
+// launch more); 128 x 128 tiles that leave half the CUs idle over a long K take two into
+// a cleared output (252 frames, the first up-convolution: 60 -> 48 + 5 us). A residual
+// output keeps one: x + a + b of two halves rounds by their order of arrival, so that
+// equal calls would differ in their last bits (27 us against 24 at 2016 rows x 1024).
 int plane_linear(vx_ctx *ctx, const __half *xh, const __half *xl, uint32_t block, uint32_t shift, const __half *pf,
                  const __half *b16, const float *b32, float *y, uint32_t T, uint32_t N, uint32_t K,
                  const float *pre = nullptr, const VaePlanes &out = VaePlanes()) {
@@ -201,9 +203,9 @@ int plane_linear(vx_ctx *ctx, const __half *xh, const __half *xl, uint32_t block
     const uint64_t tiles = (uint64_t)((N + 127u) / 128u) * ((T + 127u) / 128u);
     if (small_tiles(T, N)) return launch_gemm_ps_tiles(ctx->stream, g);
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-    if (tiles * 2u <= cus && K >= 1024u) {
+    if (block && tiles * 2u <= cus && K >= 1024u) {
         g.ksplit = 2;
-        if (block) VX_CHECK(launch_fill_u32(ctx->stream, reinterpret_cast<uint32_t *>(y), 0u, (uint64_t)T * N));
+        VX_CHECK(launch_fill_u32(ctx->stream, reinterpret_cast<uint32_t *>(y), 0u, (uint64_t)T * N));
     }
     return launch_gemm_pf(ctx->stream, g);
 }
