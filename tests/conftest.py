@@ -28,3 +28,10 @@ def rel_l2(a, b) -> float:
     b = np.asarray(b, np.float64).ravel()
     den = np.linalg.norm(b)
     return float(np.linalg.norm(a - b) / (den if den > 0 else 1.0))
+
+
+def prefill_chunk() -> int:
+    """Rows of one batched-prefill chunk, as the library is built."""
+    import re
+    text = (ROOT / "voxgen_amd" / "csrc" / "vx_internal.h").read_text()
+    return int(re.search(r"constexpr uint32_t kPrefillChunk = (\d+);", text).group(1))

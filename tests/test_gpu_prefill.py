@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import voxref
-from conftest import rel_l2
+from conftest import prefill_chunk, rel_l2
 from voxgen_amd import abi, synth
 from voxgen_amd.baselm import BaseLmEngine, config_struct
 from voxgen_amd.runtime import Model
@@ -106,7 +106,7 @@ def test_batched_prefill_gate_up_schedules(ctx, small):
 
 
 def test_batched_prefill_gate_up_half_tiles(ctx, small):
-    """512 tokens (a full prefill chunk): 4 token tiles x 96 = 384 gate/up tiles, 1.5
+    """512 tokens: 4 token tiles x 96 = 384 gate/up tiles, 1.5
     per 256 CUs, so "auto" runs 256 whole tiles and 128 tiles as two K halves that
     hand over through the part slots. Against "tiles" (one tile per workgroup; fp32
     rounding only) and the oracle."""
@@ -130,8 +130,8 @@ def test_batched_prefill_gate_up_half_tiles(ctx, small):
     assert rel_l2(f16(got["auto"][1][1]), f16(got["tiles"][1][1])) < 1e-3
 
 
-def test_batched_prefill_continues_a_decode_and_spans_chunks(ctx, small):
-    """Prefill at a non-zero position, longer than one 512-token chunk, then decode on."""
+def test_batched_prefill_continues_a_decode(ctx, small):
+    """Prefill of 600 tokens at a non-zero position, then decode on."""
     cfg, m, model = small
     o = oracle_of(m, cfg)
     toks = [int(t) for t in synth.uniform_u32(606, 0x5EED0103, cfg["vocab_size"])]
@@ -153,6 +153,71 @@ def test_batched_prefill_continues_a_decode_and_spans_chunks(ctx, small):
     for l in range(2):
         assert rel_l2(f16(got[l, :606]), f16(want[l, :606])) < 1e-3, l
     eng.close()
+
+
+@pytest.mark.parametrize("weights", ["q8_0", "f16"])
+def test_batched_prefill_continues_a_decode_and_spans_chunks(ctx, weights):
+    """At position 3, a whole chunk, a second one of 53 rows (short GEMM) and then a
+    decoded token, against the decode step at every position (pinned to the oracle by
+    the engine tests): other rows, tiles and splits of the same sums."""
+    n = prefill_chunk() + 53
+    ctxlen = (3 + n + 1 + 63) // 64 * 64
+    print(f"spans chunks {weights}: {n} tokens at position 3", flush=True)
+    cfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=ctxlen)
+    m = synth.build_baselm(cfg, seed=0x5EED0150, weight_type=weights)
+    model = Model(ctx, m.data, m.tensors)
+    toks = [int(t) for t in synth.uniform_u32(3 + n + 1, 0x5EED0151, 512)]
+    got = []
+    for batched in (False, True):
+        eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False)
+        for t in toks[:3] if batched else toks[:-1]:
+            eng.decode_token_gpu_only(t)
+        if batched:
+            eng.prefill_tokens_batched_gpu_only(toks[3:-1])
+        ctx.sync()
+        assert eng.position == 3 + n
+        prefix = eng.output()
+        eng.decode_token(toks[-1])
+        got.append((prefix, eng.output(), kv_rows(eng, "kv_k", 2, ctxlen), kv_rows(eng, "kv_v", 2, ctxlen)))
+        eng.close()
+    for a, b in zip(got[0][:2], got[1][:2]):
+        assert rel_l2(b, a) < 1e-3
+    for a, b in zip(got[0][2:], got[1][2:]):
+        for l in range(2):
+            assert rel_l2(f16(b[l, :4 + n]), f16(a[l, :4 + n])) < 1e-3, l
+            assert rel_l2(f16(b[l, n - 60:4 + n]), f16(a[l, n - 60:4 + n])) < 1e-3, l   # about the chunk edge
+        assert np.all(b[:, 4 + n:] == 0)
+    model.free()
+
+
+@pytest.mark.parametrize("n", [1, 37, 130, 300])
+def test_batched_prefill_mixed_weight_types(ctx, n):
+    """A Q8_0 layer and an F16 layer: no prefill-layout copy of the weights, so the
+    general GEMM runs over row-major planes, splits adding into cleared outputs."""
+    print(f"mixed weight types n={n}", flush=True)
+    cfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=320)
+    q, h = (synth.build_baselm(cfg, seed=0x5EED0160, weight_type=w) for w in ("q8_0", "f16"))
+    shift = (q.data.size + 255) // 256 * 256
+    pick = {t.name: t for t in q.tensors if not t.name.startswith("blk.1.")}
+    for t in h.tensors:
+        if t.name.startswith("blk.1."):
+            pick[t.name] = type(t)(t.name, t.ggml_type, t.dims, t.offset + shift)
+    data = np.concatenate([q.data, np.zeros(shift - q.data.size, np.uint8), h.data])
+    model = Model(ctx, data, list(pick.values()))
+    o = voxref.BaseLm(data, pick, cfg)
+    toks = [int(t) for t in synth.uniform_u32(n, 0x5EED0161 + n, 512)]
+    eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False)
+    eng.prefill_tokens_batched(toks)
+    for p, t in enumerate(toks):
+        o.decode_token(t, p)
+    assert rel_l2(eng.output(), o.norm) < 1e-3
+    for name, ref in (("kv_k", o.kv_k), ("kv_v", o.kv_v)):
+        got, want = kv_rows(eng, name, 2, 320), ref.reshape(2, 320, 256)
+        for l in range(2):
+            assert rel_l2(f16(got[l, :n]), f16(want[l, :n])) < 1e-3, (name, l)
+        assert np.all(got[:, n:] == 0)
+    eng.close()
+    model.free()
 
 
 def test_batched_prefill_f16_weights(ctx):
@@ -196,7 +261,8 @@ def test_batched_prefill_f16_tiles(ctx, n):
             assert rel_l2(f16(rows[0, :n]), f16(ref.reshape(512, 256)[:n])) < 1e-3, name
             assert np.all(rows[:, n:] == 0)
         eng.close()
-    assert np.array_equal(got[0], got[-1])
+    if n == 300:
+        assert np.array_equal(got[0], got[1])
     model.free()
 
 
@@ -229,27 +295,29 @@ def test_batched_prefill_short_chunks(ctx, weights):
 
 @pytest.mark.parametrize("weights", ["q8_0", "f16"])
 def test_batched_prefill_long_chunks(ctx, weights):
-    """2101 tokens in one call (a whole 2048-row chunk and a short one) against the same
-    tokens in calls of 130, 500, 700, 641 and 130: other tile counts, splits and chunk
-    edges, the same cache rows and state to rounding."""
-    print(f"long chunks {weights}", flush=True)
-    cfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=2112)
+    """A whole chunk and a short one in one call against the same tokens in calls of 130,
+    500, 700, 641 and the rest: other tile counts, splits and chunk edges, the same cache
+    rows and state to rounding."""
+    total = prefill_chunk() + 53
+    ctxlen = (total + 63) // 64 * 64
+    print(f"long chunks {weights}: {total}", flush=True)
+    cfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=ctxlen)
     m = synth.build_baselm(cfg, seed=0x5EED0140, weight_type=weights)
     model = Model(ctx, m.data, m.tensors)
-    toks = [int(t) for t in synth.uniform_u32(2101, 0x5EED0141, cfg["vocab_size"])]
+    toks = [int(t) for t in synth.uniform_u32(total, 0x5EED0141, cfg["vocab_size"])]
     got = []
-    for calls in ([2101], [130, 500, 700, 641, 130]):
+    for calls in ([total], [130, 500, 700, 641, total - 1971]):
         eng = BaseLmEngine(ctx, model, cfg, exec_mode="graph", strict_geometry=False)
         done = 0
         for n in calls:
             eng.prefill_tokens_batched(toks[done:done + n])
             done += n
-        got.append((eng.output(), kv_rows(eng, "kv_k", 2, 2112), kv_rows(eng, "kv_v", 2, 2112)))
+        got.append((eng.output(), kv_rows(eng, "kv_k", 2, ctxlen), kv_rows(eng, "kv_v", 2, ctxlen)))
         eng.close()
     assert rel_l2(got[0][0], got[1][0]) < 1e-3
     for a, b in zip(got[0][1:], got[1][1:]):
-        assert rel_l2(f16(a[:, :2101]), f16(b[:, :2101])) < 1e-3
-        assert np.all(a[:, 2101:] == 0) and np.all(b[:, 2101:] == 0)
+        assert rel_l2(f16(a[:, :total]), f16(b[:, :total])) < 1e-3
+        assert np.all(a[:, total:] == 0) and np.all(b[:, total:] == 0)
     model.free()
 
 

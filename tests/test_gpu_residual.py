@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import voxref
-from conftest import rel_l2
+from conftest import prefill_chunk, rel_l2
 from voxgen_amd import abi, synth
 from voxgen_amd.residual import ResidualFsqEngine
 from voxgen_amd.runtime import Model
@@ -243,13 +243,15 @@ def _kv(eng, acfg, which, n):
 
 
 def test_prefill_from_rows_matches_per_position_steps(ctx):
-    """600 text-prefix positions from given rows (two chunks, a partial 128-row
-    tile) against the per-position text-prefix step, which the tests above pin to
-    the oracle; then one FSQ step on top of each cache."""
-    acfg = synth.acoustic_config(layers=2, active_context=640)
+    """A whole chunk of text-prefix positions from given rows and a second one with a
+    partial 128-row tile, against the per-position text-prefix step, which the tests
+    above pin to the oracle; then one FSQ step on top of each cache."""
+    n = prefill_chunk() + 150
+    print(f"prefill from rows: {n}", flush=True)
+    acfg = synth.acoustic_config(layers=2, active_context=n + 40)
     m = synth.build_acoustic(acfg, seed=0x5EED0405)
     model = Model(ctx, m.data, m.tensors)
-    H, n = acfg["embedding_length"], 600
+    H = acfg["embedding_length"]
     rows = synth.normal_f32(n * H, 0x700).reshape(n, H)
     rbuf = ctx.array(rows)
     one = ctx.array(np.zeros(H, np.float32))
@@ -268,6 +270,7 @@ def test_prefill_from_rows_matches_per_position_steps(ctx):
         a, b = _kv(bat, acfg, which, n), _kv(seq, acfg, which, n)
         for l in range(2):
             assert rel_l2(a[l], b[l]) < 1e-3, (which, l)
+            assert rel_l2(a[l, -300:], b[l, -300:]) < 1e-3, (which, l)   # both sides of the chunk edge
     base, emb = ctx.array(synth.normal_f32(H, 0x701)), ctx.array(synth.normal_f32(H, 0x702))
     seq.step_from_gpu_base_and_embedding(base, emb)
     bat.step_from_gpu_base_and_embedding(base, emb)
@@ -282,6 +285,44 @@ def test_prefill_from_rows_matches_per_position_steps(ctx):
     for x in (seq, bat, ref):
         x.close()
     model.free()
+
+
+def test_cross_engine_text_prefill_spans_chunks(ctx):
+    """A whole chunk of tokens and 37 more through both engines (BaseLM chunk, ResidualLM
+    chunk, and again) against one decode and one text-prefix step per token."""
+    from voxgen_amd.baselm import BaseLmEngine
+    from voxgen_amd.residual import prefill_text_cross_engine
+    n = prefill_chunk() + 37
+    ctxlen = (n + 63) // 64 * 64
+    print(f"cross-engine prefill: {n}", flush=True)
+    bcfg = synth.baselm_config(layers=2, vocab=512, context_length=32768, active_context=ctxlen)
+    bm = synth.build_baselm(bcfg, seed=0x5EED0408)
+    bmodel = Model(ctx, bm.data, bm.tensors)
+    acfg = synth.acoustic_config(layers=2, active_context=ctxlen)
+    am = synth.build_acoustic(acfg, seed=0x5EED0409)
+    amodel = Model(ctx, am.data, am.tensors)
+    tokens = synth.uniform_u32(n, 0x704, 512)
+    H = acfg["embedding_length"]
+    b1, b2 = (BaseLmEngine(ctx, bmodel, bcfg, strict_geometry=False) for _ in range(2))
+    r1, r2 = (ResidualFsqEngine(ctx, amodel, acfg, strict_geometry=False) for _ in range(2))
+    for t in tokens:
+        b1.decode_token_gpu_only(int(t))
+        r1.step_text_prefix_from_gpu_base_gpu_only(b1.buffer("norm"))
+    prefill_text_cross_engine(b2, r2, tokens)
+    ctx.sync()
+    assert b2.position == n and r2.position == n
+    assert rel_l2(b2.output(), b1.output()) < 1e-3
+    for name in ("output", "current_lm", "fusion_snapshot"):
+        assert rel_l2(r2.buffer(name).download(np.float32, H), r1.buffer(name).download(np.float32, H)) < 1e-3, name
+    for which in ("kv_k", "kv_v"):
+        a, b = _kv(r2, acfg, which, n), _kv(r1, acfg, which, n)
+        for l in range(2):
+            assert rel_l2(a[l], b[l]) < 1e-3, (which, l)
+            assert rel_l2(a[l, -100:], b[l, -100:]) < 1e-3, (which, l)   # both sides of the chunk edge
+    for x in (b1, r1, b2, r2):
+        x.close()
+    for x in (bmodel, amodel):
+        x.free()
 
 
 def test_cross_engine_text_prefill_matches_sequential_and_oracle(ctx):
