@@ -210,13 +210,13 @@ int plane_linear(vx_ctx *ctx, const __half *xh, const __half *xl, uint32_t block
     return launch_gemm_pf(ctx->stream, g);
 }
 
-// y[t][n] (+)= b[n] + sum_k x[t][k] W[n][k]: the MFMA GEMM when K is a multiple
-// of 128, else the short-K kernel. Few tiles: split K with atomic adds into a
-// zeroed (store) or the residual (residual) output.
+// y[t][n] (+)= b[n] + sum_k x[t][k] W[n][k] of rows ldx apart: the short-K kernel, or the
+// MFMA GEMM for a stored (not added) product when K is a multiple of 128. Few tiles:
+// split K with atomic adds into a zeroed output.
 int linear(vx_ctx *ctx, const float *x, uint32_t ldx, const __half *w, const __half *b16, const float *b32,
-           float *y, uint32_t ldy, uint32_t T, uint32_t N, uint32_t K, bool residual) {
+           float *y, uint32_t T, uint32_t N, uint32_t K, bool residual) {
     hipStream_t s = ctx->stream;
-    if (K % 128u || (uintptr_t)w & 15u) {
+    if (residual || K % 128u || (uintptr_t)w & 15u) {
         VaeLinearArgs a;
         a.x = x;
         a.ldx = ldx;
@@ -224,7 +224,7 @@ int linear(vx_ctx *ctx, const float *x, uint32_t ldx, const __half *w, const __h
         a.bias = b16;
         a.bias_f32 = b32;
         a.y = y;
-        a.ldy = ldy;
+        a.ldy = N;
         a.T = T;
         a.N = N;
         a.K = K;
@@ -233,12 +233,12 @@ int linear(vx_ctx *ctx, const float *x, uint32_t ldx, const __half *w, const __h
     }
     GemmArgs g;
     g.wk = WT_F16;
-    g.epi = residual ? GEPI_RESIDUAL : GEPI_STORE;
+    g.epi = GEPI_STORE;
     g.xf32 = 1;
     g.seg[0].w = w;
     g.seg[0].rows = N;
     g.seg[0].out = y;
-    g.seg[0].ldo = ldy;
+    g.seg[0].ldo = N;
     g.seg[0].bias = b32 ? static_cast<const void *>(b32) : static_cast<const void *>(b16);
     g.seg[0].bias_dtype = b32 ? 0u : 1u;
     g.K = K;
@@ -251,10 +251,7 @@ int linear(vx_ctx *ctx, const float *x, uint32_t ldx, const __half *w, const __h
     uint32_t ks = (cus + tiles - 1u) / tiles;
     ks = std::min<uint32_t>(std::min<uint32_t>(ks, 8u), std::max<uint32_t>(1u, K / 256u));
     g.ksplit = std::max<uint32_t>(ks, 1u);
-    if (g.ksplit > 1 && !residual) {
-        if (ldy != N) g.ksplit = 1;   // the zero fill covers dense rows only
-        else VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(y), 0u, (uint64_t)T * N));
-    }
+    if (g.ksplit > 1) VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(y), 0u, (uint64_t)T * N));
     return launch_gemm(s, g);
 }
 
@@ -302,7 +299,7 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
         d.dilation = 1;
         d.left_pad = 6;
         VX_CHECK(launch_vae_dwconv_fm(s, d));
-        VX_CHECK(linear(ctx, tmp, ch, e->m1_w, e->m1_b, nullptr, cur, c.decoder_dim, len, c.decoder_dim, ch, false));
+        VX_CHECK(linear(ctx, tmp, ch, e->m1_w, e->m1_b, nullptr, cur, len, c.decoder_dim, ch, false));
         ch = c.decoder_dim;
     }
     for (uint32_t i = 0; i < kStages; ++i) {
@@ -317,8 +314,8 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
             } else {
                 VX_CHECK(launch_fill_u32(s, reinterpret_cast<uint32_t *>(P - ch), 0u, ch));   // row -1
                 VX_CHECK(launch_vae_pre_fm(s, cur, P, S.pre, ch, len));
-                VX_CHECK(linear(ctx, P - ch, ch, S.ct_w, nullptr, S.ct_b, tmp, S.stride * S.cout, len,
-                                S.stride * S.cout, 2u * ch, false));
+                VX_CHECK(linear(ctx, P - ch, ch, S.ct_w, nullptr, S.ct_b, tmp, len, S.stride * S.cout, 2u * ch,
+                                false));
             }
         }
         std::swap(cur, tmp);
@@ -370,7 +367,7 @@ int enqueue_decode(vx_audiovae *e, const float *in, uint32_t frames, float *wave
                                       have_pre ? e->st[i + 1].pre : nullptr,
                                       have_pre ? planes_of(e->st[i + 1], len) : VaePlanes()));
             } else {
-                VX_CHECK(linear(ctx, tmp, ch, R.pw_w, R.pw_b, nullptr, cur, ch, len, ch, ch, true));
+                VX_CHECK(linear(ctx, tmp, ch, R.pw_w, R.pw_b, nullptr, cur, len, ch, ch, true));
             }
         }
     }

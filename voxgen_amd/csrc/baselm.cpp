@@ -481,17 +481,9 @@ int run_step(vx_baselm *e, bool with_embedding, uint32_t token, bool logits) {
 
 // ------------------------------------------------------------------ prefill
 // Token-batched prefill (the seq_* op family of local.rs:482-527 applied to the
-// BaseLM stack, with Q8_0 projections, a causal mask and a position base):
-//   embedding rows -> per layer:
-//     rmsnorm(h)*attn_norm -> f16 hi/lo planes        (k_seq_rmsnorm)
-//     q|k|v = planes . Wq|Wk|Wv                       (k_gemm, split-K)
-//     RoPE at pos0+t, K/V rows -> f16 cache, q planes  (k_seq_rope_store)
-//     causal attention over cache keys 0..pos0+t       (k_prefill_attn)
-//     h += scale * Wo . attn                           (k_gemm residual)
-//     rmsnorm(h)*ffn_norm -> planes                    (k_seq_rmsnorm)
-//     act = silu(Wg . n) * (Wu . n) -> planes          (k_gemm swiglu)
-//     h += scale * Wdown . act                         (k_gemm residual)
-//   then the last token's rmsnorm(h)*output_norm into the engine's norm buffer.
+// BaseLM stack, with a causal mask and a position base): embedding rows, the layers
+// over them with RoPE (prefill_stack.cpp), then the last token's rmsnorm(h)*output_norm
+// into the engine's norm buffer.
 // This computes what prefill_tokens (baselm.rs:823-839) computes one token at a
 // time: the same KV-cache rows and the same final state, to rounding.
 int ensure_prefill_work(vx_baselm *e) {

@@ -538,16 +538,15 @@ __global__ __launch_bounds__(256) void k_seq_rmsnorm4(SeqNormArgs a) {
             for (uint32_t i = tid; i < a.zero_n[z]; i += 256u) a.zero[z][(size_t)t * a.zero_n[z] + i] = 0.f;
 }
 
-// Per-token RoPE at position base + t (rope.comp:22-51 / seq_rope.comp:8 with a
-// position base), then the f16 KV store of token t at that position
-// (store_kv.comp:16-24), and q as hi/lo planes for the attention kernel.
-// The angle is computed exactly as the decode step's per-step table.
-__global__ __launch_bounds__(256) void k_seq_rope_store(SeqRopeArgs a) {
+// Per-token RoPE of q and k in place at position base + t (rope.comp:22-51 /
+// seq_rope.comp:8 with a position base). The angle is computed exactly as the decode
+// step's per-step table.
+__global__ __launch_bounds__(256) void k_seq_rope(SeqRopeArgs a) {
     __shared__ float2 cs[64];
     const uint32_t t = blockIdx.x;
     const uint32_t pos = a.pos_base + (a.pos_period ? t % a.pos_period : t);
     const uint32_t half_dim = a.head_dim / 2u;
-    if (threadIdx.x < half_dim && !a.no_rope) {
+    if (threadIdx.x < half_dim) {
         const uint32_t i = threadIdx.x;
         const float exponent = (float)(i * 2u) / (float)a.head_dim;
         const float inv_freq = 1.0f / powf(a.theta, exponent);
@@ -555,76 +554,20 @@ __global__ __launch_bounds__(256) void k_seq_rope_store(SeqRopeArgs a) {
         cs[i] = make_float2(cosf(angle) * a.scaling, sinf(angle) * a.scaling);
     }
     __syncthreads();
-    float *q = a.q + (size_t)t * a.ldq;
-    float *k = a.k + (size_t)t * a.ldk;
     const uint32_t q_pairs = a.q_heads * half_dim, k_pairs = a.kv_heads * half_dim;
-    const uint32_t ns = a.nsplit ? a.nsplit : 1u;
     for (uint32_t p = threadIdx.x; p < q_pairs + k_pairs; p += 256u) {
         const bool isq = p < q_pairs;
-        const uint32_t pp = isq ? p : p - q_pairs;
-        const uint32_t head = pp / half_dim, i = pp - head * half_dim;
-        float *buf = isq ? q : k;
-        const uint32_t base = head * a.head_dim;
-        // split-K partials (at most kSeqRopeMaxSplit), all loads issued together,
-        // summed in split order
-        float p0[kSeqRopeMaxSplit], p1[kSeqRopeMaxSplit];
-#pragma unroll
-        for (uint32_t sp = 0; sp < kSeqRopeMaxSplit; ++sp) {
-            const size_t o = (size_t)(sp < ns ? sp : 0u) * a.split_stride + base + i;
-            p0[sp] = buf[o];
-            p1[sp] = buf[o + half_dim];
-        }
-        float x0 = p0[0], x1 = p1[0];
-#pragma unroll
-        for (uint32_t sp = 1; sp < kSeqRopeMaxSplit; ++sp) {
-            x0 += sp < ns ? p0[sp] : 0.f;
-            x1 += sp < ns ? p1[sp] : 0.f;
-        }
-        float y0 = x0, y1 = x1;
-        if (!a.no_rope) {
-            const float c = cs[i].x, s = cs[i].y;
-            y0 = x0 * c - x1 * s;
-            y1 = x1 * c + x0 * s;
-        }
-        if (isq) {
-            if (a.q_inplace) {
-                buf[base + i] = y0;
-                buf[base + i + half_dim] = y1;
-            }
-            if (a.qh) {
-                const size_t o = (size_t)t * a.ldqp + base + i;
-                const _Float16 h0 = (_Float16)y0, h1 = (_Float16)y1;
-                a.qh[o] = __builtin_bit_cast(__half, h0);
-                a.ql[o] = __builtin_bit_cast(__half, (_Float16)(y0 - (float)h0));
-                a.qh[o + half_dim] = __builtin_bit_cast(__half, h1);
-                a.ql[o + half_dim] = __builtin_bit_cast(__half, (_Float16)(y1 - (float)h1));
-            }
-        } else {
-            buf[base + i] = y0;
-            buf[base + i + half_dim] = y1;
-        }
-    }
-    if (!a.kc) return;
-    __syncthreads();  // roped k visible to the store below
-    if (pos >= a.context) return;
-    const float *v = a.v + (size_t)t * a.ldk;
-    const uint32_t kv_dim = a.kv_heads * a.head_dim;
-    const size_t dst = ((size_t)a.layer * a.context + pos) * kv_dim;
-    for (uint32_t i = threadIdx.x; i < kv_dim; i += 256u) {
-        float pv[kSeqRopeMaxSplit];
-#pragma unroll
-        for (uint32_t sp = 0; sp < kSeqRopeMaxSplit; ++sp) pv[sp] = v[(size_t)(sp < ns ? sp : 0u) * a.split_stride + i];
-        float vv = pv[0];
-#pragma unroll
-        for (uint32_t sp = 1; sp < kSeqRopeMaxSplit; ++sp) vv += sp < ns ? pv[sp] : 0.f;
-        a.kc[dst + i] = __float2half_rn(k[i]);
-        a.vc[dst + i] = __float2half_rn(vv);
+        const uint32_t pp = isq ? p : p - q_pairs, head = pp / half_dim, i = pp - head * half_dim;
+        float *const x = (isq ? a.q + (size_t)t * a.ldq : a.k + (size_t)t * a.ldk) + head * a.head_dim + i;
+        const float x0 = x[0], x1 = x[half_dim], c = cs[i].x, s = cs[i].y;
+        x[0] = x0 * c - x1 * s;
+        x[half_dim] = x1 * c + x0 * s;
     }
 }
 
-// The prefill stack's RoPE and KV store. Per row it read the trigonometric functions
-// anew in every layer and walked q, k and v in five dependent steps (7.5 us at 512 rows,
-// 14.4 at 1900); here the angles come from a table made once a chunk, with the same
+// The prefill stack's RoPE and KV store. A workgroup a row that evaluated the
+// trigonometric functions in every layer and walked q, k and v in five dependent steps
+// took 7.5 us at 512 rows and 14.4 at 1900; here the angles come from a table made once a chunk, with the same
 // expressions, and a thread takes four neighbouring pairs of q or k, or four values of v,
 // all loads issued together.
 __global__ __launch_bounds__(256) void k_prefill_rope_table(SeqRopeArgs a, uint32_t n, float2 *tab) {
@@ -1550,7 +1493,7 @@ int launch_gemm(hipStream_t s, const GemmArgs &in) {
         return fail(VX_ERR_UNSUPPORTED, "gemm: fragment-layout operands need the short-batch kernel (F16, T <= 128, "
                                         "16-byte aligned, K %% 32 == 0; got T=%u K=%u)", a.T, a.K);
     if (a.split_store && a.ksplit > 1)
-        return fail(VX_ERR_INVALID_ARG, "gemm: split partial stores need the prefill-layout Q8_0 or the short-batch F16 kernel");
+        return fail(VX_ERR_INVALID_ARG, "gemm: split partial stores need the prefill-layout or the short-batch F16 kernel");
     const uint32_t stages = a.K / GK;
     if (a.ksplit == 0) a.ksplit = 1;
     if (a.ksplit > stages) a.ksplit = stages;
@@ -1576,7 +1519,6 @@ int launch_gemm(hipStream_t s, const GemmArgs &in) {
     VX_GEMM_CASE(WT_F16, false, GEPI_RESIDUAL)
     VX_GEMM_CASE(WT_F16, false, GEPI_SWIGLU)
     VX_GEMM_CASE(WT_F16, true, GEPI_STORE)
-    VX_GEMM_CASE(WT_F16, true, GEPI_RESIDUAL)
     VX_GEMM_CASE(WT_F16, true, GEPI_SWIGLU)
 #undef VX_GEMM_CASE
     return fail(VX_ERR_UNSUPPORTED, "gemm: no kernel for weight type %u, f32 input %d, epilogue %u", a.wk,
@@ -1611,15 +1553,12 @@ int launch_seq_rmsnorm(hipStream_t s, const SeqNormArgs &a, uint32_t tokens) {
     return VX_OK;
 }
 
-int launch_seq_rope_store(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens) {
+int launch_seq_rope(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens) {
     if (tokens == 0) return VX_OK;
-    if (a.nsplit > kSeqRopeMaxSplit)
-        return fail(VX_ERR_INVALID_ARG, "seq rope: at most %u split partials", kSeqRopeMaxSplit);
     if (a.head_dim == 0 || a.head_dim > 128u || (a.head_dim & 1u))
         return fail(VX_ERR_UNSUPPORTED, "seq rope: head_dim must be even and <= 128");
-    if (a.kc && (!a.vc || !a.v)) return fail(VX_ERR_INVALID_ARG, "seq rope: KV store needs v and both caches");
-    k_seq_rope_store<<<tokens, 256, 0, s>>>(a);
-    VX_LAUNCHED("k_seq_rope_store");
+    k_seq_rope<<<tokens, 256, 0, s>>>(a);
+    VX_LAUNCHED("k_seq_rope");
     return VX_OK;
 }
 
@@ -1714,7 +1653,7 @@ __global__ __launch_bounds__(256) void k_rope_pos_table(float2 *tab, const float
     const uint32_t j = blockIdx.x * 256u + threadIdx.x;
     if (j >= n) return;
     const uint32_t pos = j / half, i = j - pos * half;
-    const float exponent = (float)(i * 2u) / (float)head_dim;   // as k_seq_rope_store
+    const float exponent = (float)(i * 2u) / (float)head_dim;   // as k_seq_rope
     const float inv_freq = 1.0f / powf(theta, exponent);
     const float angle = (float)pos * inv_freq / factors[i];
     tab[j] = make_float2(cosf(angle) * scaling, sinf(angle) * scaling);

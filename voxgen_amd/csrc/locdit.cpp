@@ -292,7 +292,7 @@ int enqueue_layers_general(vx_locdit *e, uint32_t batch) {
             r.pos_period = S;   // seq_rope.comp:8: position = token index within the sequence
             r.theta = c.rope_theta;
             r.scaling = c.rope_scaling;
-            VX_CHECK(launch_seq_rope_store(s, r, M));
+            VX_CHECK(launch_seq_rope(s, r, M));
         }
         {
             ProfSpan sp(ctx, "local.attention");

@@ -4,13 +4,15 @@
 // (without RoPE):
 //   per layer over the rows of the residual stream h:
 //     rmsnorm(h)*attn_norm -> f16 hi/lo planes        (k_seq_rmsnorm)
-//     q|k|v = planes . Wq|Wk|Wv                       (k_gemm, split-K)
+//     q|k|v = planes . Wq|Wk|Wv                       (GEMM, split-K)
 //     RoPE at pos0+t (or none), K/V rows -> f16 cache, q planes  (k_prefill_rope)
 //     causal attention over cache keys 0..pos0+t       (k_prefill_attn)
-//     h += scale * Wo . attn                           (k_gemm residual)
+//     h += scale * Wo . attn                           (GEMM, residual)
 //     rmsnorm(h)*ffn_norm -> planes                    (k_seq_rmsnorm)
-//     act = silu(Wg . n) * (Wu . n) -> planes          (k_gemm swiglu)
-//     h += scale * Wdown . act                         (k_gemm residual)
+//     act = silu(Wg . n) * (Wu . n) -> planes          (GEMM, SwiGLU)
+//     h += scale * Wdown . act                         (GEMM, residual)
+// The GEMM is k_gemm_pf over weights in the prefill layout (k_gemm_ps below 128 rows),
+// k_gemm where the engine has none.
 // Row t computes what the decode step computes at position pos0 + t: the same
 // KV-cache rows and the same residual stream, to rounding.
 #include <algorithm>
@@ -21,7 +23,6 @@
 namespace vx {
 
 namespace {
-
 
 // Split-K factor for a projection of n_tiles 128-row tiles and tt-token tiles:
 // as many workgroups as fit one per CU (rounded down: a second workgroup on a CU
@@ -304,13 +305,11 @@ int enqueue_prefill_stack(const PrefillStack &p, uint32_t pos0, uint32_t T) {
             r.head_dim = p.head_dim;
             r.theta = p.theta;
             r.scaling = p.rope_scaling;
-            r.q_inplace = 0;
             r.qh = w.qh;
             r.ql = w.ql;
             r.ldqp = nH;
             r.kc = p.kc;
             r.vc = p.vc;
-            r.no_rope = p.rope ? 0u : 1u;
             r.layer = l;
             r.context = p.context;
             if (l == 0 && rope) VX_CHECK(launch_prefill_rope_table(s, r, T, rope));

@@ -357,7 +357,7 @@ int vx_seq_rope_at(vx_ctx *ctx, const vx_model *model, vx_buf *q, vx_buf *k, uin
     a.head_dim = pc->head_dim;
     a.theta = pc->rope_theta;
     a.scaling = pc->scaling_factor;
-    return launch_seq_rope_store(ctx->stream, a, pc->tokens);
+    return launch_seq_rope(ctx->stream, a, pc->tokens);
 }
 
 int vx_seq_rope(vx_ctx *ctx, const vx_model *model, vx_buf *q, vx_buf *k, const vx_seq_rope_push *pc) {

@@ -552,30 +552,31 @@ int launch_seq_rmsnorm(hipStream_t s, const SeqNormArgs &a, uint32_t tokens);
 
 struct SeqRopeArgs {
     float *q = nullptr, *k = nullptr;   // [T][ldq], [T][ldk]
-    const float *v = nullptr;           // [T][ldk] (KV store)
     uint32_t ldq = 0, ldk = 0;
     const float *factors = nullptr;
     uint32_t pos_base = 0, q_heads = 0, kv_heads = 0, head_dim = 0;
-    uint32_t pos_period = 0;            // nonzero: row t is at position pos_base + t % pos_period
     float theta = 10000.f, scaling = 1.f;
-    int q_inplace = 1;                  // write roped q back to q
-    __half *qh = nullptr, *ql = nullptr;   // nullable roped q planes [T][ldqp]
+    // launch_seq_rope only. Nonzero: row t is at position pos_base + t % pos_period.
+    uint32_t pos_period = 0;
+    // launch_prefill_rope only.
+    const float *v = nullptr;           // [T][ldk]
+    __half *qh = nullptr, *ql = nullptr;   // q planes [T][ldqp]
     uint32_t ldqp = 0;
-    __half *kc = nullptr, *vc = nullptr;   // nullable: store K/V rows [layer][context][kv_dim]
+    __half *kc = nullptr, *vc = nullptr;   // K/V rows [layer][context][kv_dim]
     uint32_t layer = 0, context = 0;
-    // q, k and v hold nsplit partial products split_stride floats apart (split-K
-    // GEMM output); the kernel reads their sums and writes roped k to split 0.
+    // q, k and v hold nsplit partial products split_stride floats apart (split-K GEMM
+    // output), whose sums are taken in split order.
     uint32_t nsplit = 1;
     uint64_t split_stride = 0;
-    uint32_t no_rope = 0;               // 1: q/k pass through unrotated (factors unused)
 };
-constexpr uint32_t kSeqRopeMaxSplit = 8;
-// The prefill stack's form of the step below: cos and sin (times scaling) of every row's
-// position in a table [T][head_dim / 2], made once a chunk, and one pass from the sums of
-// the QKV products to q planes and cache rows (head_dim % 8 == 0, 16-byte aligned rows).
+// q and k rotated in place.
+int launch_seq_rope(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens);
+// The prefill stack's form: cos and sin (times scaling) of every row's position in a
+// table [T][head_dim / 2], made once a chunk, and one pass from the sums of the QKV
+// products to q planes and cache rows (head_dim % 8 == 0, 16-byte aligned rows); no
+// table: q and k pass through unrotated.
 int launch_prefill_rope_table(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens, float2 *tab);
 int launch_prefill_rope(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens, const float2 *tab);
-int launch_seq_rope_store(hipStream_t s, const SeqRopeArgs &a, uint32_t tokens);
 
 // ------------------------------------------- token-batched decoder stack (prefill)
 struct StackLayer {
@@ -810,7 +811,7 @@ struct DenseAttnArgs {
 };
 int launch_dense_attn(hipStream_t s, const DenseAttnArgs &a, int which);
 // table[p][i] = (cos, sin)(p * theta^(-2i/head_dim) / factors[i]) * scaling for
-// positions p < tokens (the angle of k_seq_rope_store).
+// positions p < tokens (the angle of k_seq_rope).
 int launch_rope_pos_table(hipStream_t s, float2 *table, const float *factors, uint32_t tokens, uint32_t head_dim,
                           float theta, float scaling);
 // The three phases in one kernel (one workgroup per head, sequence and eight query
