@@ -54,13 +54,12 @@
 // against 4.0 ms, the A fragments then being read from LDS by four waves each.
 #include <type_traits>
 
-#include "vx_internal.h"
+#include "quant_dev.h"
 
 namespace vx {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float acc16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 128;                       // tokens per workgroup tile
@@ -75,23 +74,6 @@ struct Slot {                                  // one stage in the ring
     static constexpr int kXOff = 0, kWOff = 2 * kXBytes, kDOff = kWOff + kWBytes;
     static constexpr int kBytes = kDOff + kDBytes;                      // 20992 or 24576: two workgroups per CU
 };
-
-// Chunk permutations of the stored layouts: X rows of 64 bytes in 16-byte
-// chunks (tiled_plane_index), quant rows of 32 bytes in 8-byte chunks
-// (PrefillMatrix); both conflict-free for 32 and for 64 LDS banks.
-__device__ __forceinline__ uint32_t xperm(uint32_t t) { return ((t >> 1) ^ (t >> 3)) & 3u; }
-__device__ __forceinline__ uint32_t wperm(uint32_t n) { return ((n >> 2) ^ (n >> 4)) & 3u; }
-
-// Four stored quants u = q + 128 (one dword) -> four exact f16 values q: the f16
-// with bits 0x6400 | u is 1024 + u, minus 1152 = q.
-__device__ __forceinline__ uint2 q8x4_to_f16(uint32_t u) {
-    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
-    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-    const h2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    const h2v a = __builtin_bit_cast(h2v, lo) - bias;
-    const h2v b = __builtin_bit_cast(h2v, hi) - bias;
-    return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
-}
 
 __device__ __forceinline__ acc16 mfma(h8 a, h8 b, acc16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -478,8 +460,7 @@ __device__ __forceinline__ void swiglu_planes(const GemmArgs &a, uint32_t tn, ui
             const float g = acc[mt][0][r], u = acc[mt][1][r];
             const float v = m0 + ti < a.T ? g / (1.0f + expf(-g)) * u : 0.f;   // matvec_swiglu.comp:67
             const _Float16 hv = (_Float16)v;
-            const uint32_t o =
-                (wn * 128u + ti) * 32u + 8u * ((l32 >> 3) ^ (((ti >> 1) ^ (ti >> 3)) & 3u)) + (l32 & 7u);
+            const uint32_t o = (wn * 128u + ti) * 32u + 8u * ((l32 >> 3) ^ xperm(ti)) + (l32 & 7u);
             st[o] = hv;
             st[2u * 128u * 32u + o] = (_Float16)(v - (float)hv);
         }

@@ -23,13 +23,13 @@
 // workgroup reads all of X), 26 with 128 (too few workgroups); eight waves: 18. The
 // split projections are the other way round (their K ranges are short): 9 us with 32
 // rows, 11 with 64; one workgroup per CU beat two (X again) by 10%.
+#include "quant_dev.h"
 #include "vae_dev.h"
 
 namespace vx {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
@@ -37,21 +37,9 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 constexpr int NW = 4;             // waves per workgroup
 constexpr uint32_t kPiece = 128;  // weight rows and tokens of a stored tile
 
-__device__ __forceinline__ uint32_t xperm(uint32_t t) { return ((t >> 1) ^ (t >> 3)) & 3u; }
-__device__ __forceinline__ uint32_t wperm(uint32_t n) { return ((n >> 2) ^ (n >> 4)) & 3u; }
-
-// Eight stored quants u = q + 128 -> exact f16 q: 0x6400 | u is 1024 + u.
 __device__ __forceinline__ h8 widen(u2v u) {
-    const h2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    u4v r;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u[i], 0x04010400u);
-        const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u[i], 0x04030402u);
-        r[2 * i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, lo) - bias);
-        r[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, hi) - bias);
-    }
-    return __builtin_bit_cast(h8, r);
+    const uint2 lo = q8x4_to_f16(u[0]), hi = q8x4_to_f16(u[1]);
+    return __builtin_bit_cast(h8, u4v{lo.x, lo.y, hi.x, hi.y});
 }
 
 __device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) {

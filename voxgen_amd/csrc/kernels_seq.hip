@@ -27,14 +27,13 @@
 //     projections, so that a T = 384 prefill still fills 256 CUs.
 #include <cfloat>
 
-#include "vx_internal.h"
+#include "quant_dev.h"
 
 namespace vx {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float acc16 __attribute__((ext_vector_type(16)));
 
 constexpr int GM = 64;      // tokens per workgroup tile
@@ -48,18 +47,6 @@ __device__ __forceinline__ acc16 mfma(h8 a, h8 b, acc16 c) {
 
 __device__ __forceinline__ float h2f(unsigned short bits) {
     return (float)__builtin_bit_cast(_Float16, bits);
-}
-
-// Four signed int8 quants (one dword) -> four exact f16 values: (q ^ 0x80) is
-// q + 128 in 0..255; the f16 with bits 0x6400 | u is 1024 + u, minus 1152 = q.
-__device__ __forceinline__ uint2 q8x4_to_f16(uint32_t w) {
-    const uint32_t u = w ^ 0x80808080u;
-    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
-    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-    const h2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    const h2v a = __builtin_bit_cast(h2v, lo) - bias;
-    const h2v b = __builtin_bit_cast(h2v, hi) - bias;
-    return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
 }
 
 // hi/lo f16 split of four floats.
@@ -197,7 +184,7 @@ __device__ __forceinline__ void store_stage(const StageRegs<WK, XF32> &r, _Float
             _Float16 *dst = Wl + rho * LROW + 4u * p;
             const uint32_t words[4] = {r.w[i].x, r.w[i].y, r.w[i].z, r.w[i].w};
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) *reinterpret_cast<uint2 *>(dst + 32 * kk) = q8x4_to_f16(words[kk]);
+            for (int kk = 0; kk < 4; ++kk) *reinterpret_cast<uint2 *>(dst + 32 * kk) = q8x4s_to_f16(words[kk]);
         }
         if (tid < (uint32_t)GN) {
             Ds[0 * GN + tid] = h2f((unsigned short)(r.d.x & 0xffffu));

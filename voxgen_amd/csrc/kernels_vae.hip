@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void k_vae_pre_planes(const float *x, VaePlane
         }
     }
     __half *const yh = y.h + (size_t)blockIdx.y * (y.block / 2u), *const yl = y.l + (size_t)blockIdx.y * (y.block / 2u);
-    const size_t o = (size_t)t * 32u + 8u * ((i & 3u) ^ (((t >> 1) ^ (t >> 3)) & 3u));
+    const size_t o = (size_t)t * 32u + 8u * ((i & 3u) ^ xperm(t));
     if (t == 0u) {
         *reinterpret_cast<h8v *>(yh + 8u * (i & 3u) - 32) = h8v{};
         *reinterpret_cast<h8v *>(yl + 8u * (i & 3u) - 32) = h8v{};

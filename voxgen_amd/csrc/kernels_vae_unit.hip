@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_vae_unit(VaeUnitArgs a) {
     const VaePlanes &P = a.planes;
     auto po = [&](int n, uint32_t t) {   // halves from the tile's row 0 of block 0, this lane's channel
         return (size_t)(wn * NTL + n) * (P.block / 2u) + t * 32u +
-               8u * ((l32 >> 3) ^ (((t >> 1) ^ (t >> 3)) & 3u)) + (l32 & 7u);
+               8u * ((l32 >> 3) ^ xperm(t)) + (l32 & 7u);
     };
     __half *const yh = P.h + (size_t)t0 * 32u, *const yl = P.l + (size_t)t0 * 32u;
     float ps[NTL], pt[NTL], pa[NTL], pi[NTL], big = 0.f;

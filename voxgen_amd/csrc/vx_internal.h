@@ -473,15 +473,19 @@ __host__ __device__ __forceinline__ size_t frag32_index(uint32_t r, uint32_t c, 
 // Rewrites an F16 [rows][K] row-major matrix in the fragment layout (rows padded
 // to a multiple of 16 with zeros): dst holds ceil(rows/16)*16*K halves.
 int launch_repack_frag16(hipStream_t s, const __half *src, __half *dst, uint32_t rows, uint32_t K);
+// Chunk permutations of the prefill GEMM's stored layouts, by row: the 16-byte chunks
+// of a row of 32 halves (chunk c stored at c ^ xperm(t)) and the 8-byte chunks of a row
+// of 32 quants (c ^ wperm(n)). They make the GEMM's fragment reads conflict-free, for 32
+// and for 64 LDS banks, once a piece is copied to LDS.
+__host__ __device__ __forceinline__ uint32_t xperm(uint32_t t) { return ((t >> 1) ^ (t >> 3)) & 3u; }
+__host__ __device__ __forceinline__ uint32_t wperm(uint32_t n) { return ((n >> 2) ^ (n >> 4)) & 3u; }
 // Tiled hi/lo plane layout read by the prefill GEMM (kernels_gemm.hip):
 // f16 [T/128][K/32][128][32], i.e. one contiguous 8 KB piece per (128-token
-// tile, 32-column block); the four 8-column chunks of a token's 32 values are
-// permuted by the token's index in the tile (chunk c stored at c ^ f(t),
-// f(t) = ((t >> 1) ^ (t >> 3)) & 3), which makes the GEMM's fragment reads
-// conflict-free once the piece is copied to LDS. T is padded to a multiple of 128.
+// tile, 32-column block), the 16-byte chunks of a token's 32 values permuted by
+// xperm. T is padded to a multiple of 128.
 __host__ __device__ __forceinline__ size_t tiled_plane_index(uint32_t t, uint32_t c, uint32_t K) {
-    const uint32_t ti = t & 127u, f = ((ti >> 1) ^ (ti >> 3)) & 3u;
-    return ((((size_t)(t >> 7) * (K >> 5) + (c >> 5)) << 7) + ti) * 32u + 8u * (((c >> 3) & 3u) ^ f) + (c & 7u);
+    const uint32_t ti = t & 127u;
+    return ((((size_t)(t >> 7) * (K >> 5) + (c >> 5)) << 7) + ti) * 32u + 8u * (((c >> 3) & 3u) ^ xperm(ti)) + (c & 7u);
 }
 // Q8_0 matrix in the prefill-GEMM layout: quants stored as q + 128 (uint8, the
 // sign bit flipped) [rows_pad/128][K/32][128][32]
