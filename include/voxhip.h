@@ -895,7 +895,7 @@ int vx_residual_prefill_text_from_gpu_rows(vx_residual *eng, const vx_buf *rows,
 /* The text runs of prefill_conditioning_plan (runtime.rs:483-566): for each token,
  * a BaseLM decode then a ResidualLM text-prefix step from its output, computed as
  * a batched BaseLM prefill (every position's output row kept) followed by the
- * batched ResidualLM text prefix, in chunks of up to 512 positions. Both engines
+ * batched ResidualLM text prefix, in chunks of up to 2048 positions. Both engines
  * advance by n and end in the state of the last position. Enqueue only. */
 int vx_prefill_text_cross_engine(vx_baselm *base, vx_residual *eng, const uint32_t *tokens, uint32_t n);
 

@@ -3,7 +3,7 @@
 //
 // The engine keeps activations frame-major, [length][channels], so that the
 // matrix-shaped parts run as GEMMs on MFMA:
-//   model.0   depthwise k=7 causal conv                  k_vae_dwconv_fm
+//   model.0   depthwise k=7 causal conv                  k_vae_dw7_fm / k_vae_dwconv_*
 //   model.1   1x1 conv latent -> decoder_dim             k_vae_linear_fm (K = latent)
 //   6 stages  scale/bias + snake + ConvTranspose1d(k=2s, stride s):
 //               P = pre(x) behind a zero row,           k_vae_pre_planes, or the epilogue of
@@ -14,9 +14,9 @@
 //               32 to 512 channels: one pass             k_vae_unit
 //               else snake -> depthwise k=7 -> snake     k_vae_dw7_fm / k_vae_dwconv_*
 //               and x += 1x1 conv + bias                 k_gemm_pf / k_gemm_ps
-//             (Cin no multiple of 64, or a 1x1 conv over channels that are none of 128:
-//             f32 products instead of planes, k_vae_linear_fm)
-//   head      snake -> conv k=7 to one channel -> tanh   k_vae_head_fm
+//             (other widths, Cin no multiple of 64 or a 1x1 conv over channels that
+//             are none of 128: f32 products instead of planes, k_vae_linear_fm)
+//   head      snake -> conv k=7 to one channel -> tanh   k_vae_head*_fm
 // Row j of the transposed convolution's output phases r = 0..s-1 is output time
 // s j + r, so the GEMM's [L][s Cout] output is the frame-major [s L][Cout] output.
 #include <algorithm>

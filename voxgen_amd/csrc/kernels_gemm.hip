@@ -6,7 +6,8 @@
 // and the products accumulate in place, with no widening and no scale step. Against
 // k_gemm's 64-token tiles (operands through registers, two barriers a stage, 4-byte
 // atomic epilogues), four F16 layers of the VoxCPM2 geometry took on MI355X at
-// T = 130 / 256 / 384 / 512: 475 / 546 / 773 / 840 -> 441 / 501 / 613 / 691 us. A lone
+// T = 130 / 256 / 384 / 512: 475 / 546 / 773 / 840 -> 441 / 501 / 613 / 691 us (423 / 486 /
+// 596 / 675 with the RoPE and norm kernels of today). A lone
 // workgroup's block costs 436 ns: the DMA of its 24 KB alone 347 (29 bytes a cycle
 // whatever the ring depth, 3 to 6 slots, and whether the source is one cached block),
 // its products and LDS reads alone 310; the rest of a launch is about 10 us of

@@ -43,8 +43,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float *x, float *y, const
 }
 
 // The same for n = 1024 NV, 16-byte aligned rows: x and w in registers from one round of
-// loads (the loop above waits for each of its 2 n / 256 reads: 4.6 to 6.3 us at n = 2048
-// on MI355X). `copy` (nullable) receives x.
+// loads, where the loop above waits for each of its 2 n / 256 reads (5.5 -> 4.5 us at
+// n = 2048 in a kernel trace on MI355X; one such launch in a decode step of 0.66 ms does
+// not show). `copy` (nullable) receives x.
 template <int NV>
 __global__ __launch_bounds__(256) void k_rmsnorm4(const float *x, float *y, const float *w, float eps,
                                                   uint32_t *advance, float *copy) {

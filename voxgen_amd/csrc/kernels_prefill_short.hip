@@ -19,10 +19,11 @@
 // Against k_gemm (64-token tiles, at most four splits, atomic sums) four Q8_0 layers
 // took on MI355X at 2 / 16 / 37 / 64 / 127 rows 381 / 409 / 431 / 435 / 448 ->
 // 193 / 207 / 268 / 308 / 429 us, F16 381 / 406 / 431 / 434 / 448 -> 206 / 221 / 281 /
-// 318 / 427. Gate/up at 37 rows: 17 us with 64 rows a workgroup, 22 with 32 (every
-// workgroup reads all of X), 26 with 128 (too few workgroups); eight waves: 18. The
-// split projections are the other way round (their K ranges are short): 9 us with 32
-// rows, 11 with 64; one workgroup per CU beat two (X again) by 10%.
+// 318 / 427; with the RoPE and norm kernels of today 180 / 197 / 258 / 298 / 412 and
+// 195 / 212 / 273 / 311 / 416. Gate/up at 37 rows: 17 us with 64 rows a workgroup, 22
+// with 32 (every workgroup reads all of X), 26 with 128 (too few workgroups); eight
+// waves: 18. The split projections are the other way round (their K ranges are short):
+// 9 us with 32 rows, 11 with 64; one workgroup per CU beat two (X again) by 10%.
 #include "quant_dev.h"
 #include "vae_dev.h"
 

@@ -29,8 +29,8 @@
 // channels 91 -> 44, 32 channels 62 -> 35. Larger tiles of 256 and 128 channels at one
 // workgroup of eight waves per CU were slower (79 and 60 us), and so was holding them
 // to 128 vector registers for two (140 and 100 us: spills). The unit that ends a stage
-// writes the next stage's planes: 15 us more at 256 channels (20 with an address a store), where a pass of its own
-// over f32 would read and write 120 MB.
+// writes the next stage's planes: 12 us more at 256 channels (20 with an address a
+// store), where a pass of its own over f32 would read and write 120 MB.
 #include "vae_dev.h"
 
 namespace vx {
