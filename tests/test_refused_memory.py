@@ -129,6 +129,44 @@ assert eng.position == 5
 """)
 
 
+def test_prefill_in_smaller_chunks_where_the_large_workspace_does_not_fit(fake):
+    """Where the workspace of a whole chunk is refused, one of 512 rows is taken: 600
+    positions are two chunks (two sets of layer launches), 600 with room are one."""
+    child(fake, """
+cfg = synth.baselm_config(layers=1, hidden=256, ffn=512, vocab=64, q_heads=2, kv_heads=1, context_length=4096,
+                          active_context=4096)
+m = synth.build_baselm(cfg, seed=1, weight_type="f16")
+model = Model(ctx, m.data, m.tensors)
+acfg = synth.acoustic_config(layers=1, hidden=256, ffn=512, q_heads=2, kv_heads=1, latent=64, active_context=4096)
+am = synth.build_acoustic(acfg, seed=2)
+amodel = Model(ctx, am.data, am.tensors)
+rows = ctx.zeros(600 * 256 * 4)
+def chunks(run):
+    n = launches("k_prefill_attn")
+    run()
+    return launches("k_prefill_attn") - n
+def base():
+    eng = BaseLmEngine(ctx, model, cfg, strict_geometry=False)
+    n = chunks(lambda: eng.prefill_tokens_batched_gpu_only([1] * 600))
+    assert eng.position == 600
+    return n
+def residual():
+    eng = ResidualFsqEngine(ctx, amodel, acfg, strict_geometry=False)
+    n = chunks(lambda: eng.prefill_text_from_gpu_rows(rows, 600))
+    assert eng.position == 600
+    return n
+fake.fake_largest()
+assert base() == 1
+whole = fake.fake_largest()   # the workspace
+refuse(whole, 1 << 40)
+assert base() == 2 and residual() == 2
+refuse(2048 * 512 * 4, 2048 * 512 * 4)   # the fusion input of a whole chunk
+assert residual() == 2
+refuse(0, 0)
+assert residual() == 1
+""")
+
+
 @pytest.mark.gpu
 def test_refused_device_allocation_leaves_no_error_behind(ctx):
     """The same on the device: 2^50 bytes are more than any card has."""

@@ -488,8 +488,13 @@ int run_step(vx_baselm *e, bool with_embedding, uint32_t token, bool logits) {
 // time: the same KV-cache rows and the same final state, to rounding.
 int ensure_prefill_work(vx_baselm *e) {
     const vx_baselm_config &c = e->cfg;
-    const uint32_t cap = std::min<uint32_t>(kPrefillChunk, c.active_context_length);
-    VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
+    int st = VX_OK;
+    for (uint32_t chunk : {kPrefillChunk, kPrefillChunkSmall}) {
+        const uint32_t cap = std::min<uint32_t>(chunk, c.active_context_length);
+        st = prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf);
+        if (st != VX_ERR_OOM) break;
+    }
+    VX_CHECK(st);
     return e->pf_tok ? VX_OK : alloc(e->ctx, (uint64_t)c.active_context_length * 4u, &e->pf_tok);
 }
 

@@ -158,19 +158,22 @@ int validate(const vx_acoustic_config &c, bool strict) {
     return VX_OK;
 }
 
+void free_prefill_work(vx_residual *e) {
+    prefill_stack_free(e->ctx, &e->pf);
+    for (vx_buf **b : {&e->fuse_x, &e->rows}) {
+        vx_free(e->ctx, *b);
+        *b = nullptr;
+    }
+}
+
 void free_all(vx_residual *e) {
     for (CachedGraph &g : e->graphs)
         if (g.g) vx_graph_free(e->ctx, g.g);
     e->graphs.clear();
-    prefill_stack_free(e->ctx, &e->pf);
+    free_prefill_work(e);
     e->pw.clear();
     if (e->pw_arena) vx_free(e->ctx, e->pw_arena);
     e->pw_arena = nullptr;
-    for (vx_buf **b : {&e->fuse_x, &e->rows})
-        if (*b) {
-            vx_free(e->ctx, *b);
-            *b = nullptr;
-        }
     vx_buf **bufs[] = {&e->base_input, &e->current_embed, &e->zero_embed, &e->fsq_latent, &e->fsq_output,
                        &e->current_lm, &e->hidden,        &e->fusion_snapshot, &e->norm,  &e->q,
                        &e->k,          &e->v,             &e->attention, &e->gate,        &e->branch,
@@ -582,10 +585,21 @@ int predict_stop(vx_residual *e, const float *x, vx_stop_prediction *out) {
 int ensure_prefill_work(vx_residual *e) {
     if (e->pf_ready) return VX_OK;
     const vx_acoustic_config &c = e->cfg;
-    const uint32_t cap = std::min<uint32_t>(kPrefillChunk, c.active_context_length);
-    VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
-    if (!e->fuse_x) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.fusion_input_dim * 4u, &e->fuse_x));
-    if (!e->rows) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.embedding_length * 4u, &e->rows));
+    auto alloc = [&](uint32_t cap) {
+        VX_CHECK(prefill_stack_alloc(e->ctx, cap, c.embedding_length, c.feed_forward_length, c.kv_dim, &e->pf));
+        if (!e->fuse_x) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.fusion_input_dim * 4u, &e->fuse_x));
+        if (!e->rows) VX_CHECK(vx_alloc(e->ctx, (uint64_t)cap * c.embedding_length * 4u, &e->rows));
+        return (int)VX_OK;
+    };
+    int st = alloc(std::min<uint32_t>(kPrefillChunk, c.active_context_length));
+    if (st == VX_ERR_OOM && c.active_context_length > kPrefillChunkSmall) {
+        free_prefill_work(e);
+        st = alloc(kPrefillChunkSmall);
+    }
+    if (st != VX_OK) {
+        free_prefill_work(e);
+        return st;
+    }
     VX_HIP(hipMemsetAsync(e->fuse_x->ptr, 0, e->fuse_x->bytes, e->ctx->stream));
     VX_CHECK(prefill_stack_weights(e->ctx, e->layers.data(), c.residual_block_count, c.embedding_length,
                                    c.feed_forward_length, c.kv_dim, &e->pw, &e->pw_arena));

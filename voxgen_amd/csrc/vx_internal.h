@@ -605,8 +605,9 @@ struct StackWork {                  // activations of one chunk of rows (cap row
 // 1934 / 2872 us) 1024 gave 811 / 1747 / 2518 and 2048 814 / 1568 / 2190: fewer tiles run
 // beside an idle slot, the attention's workgroups overlap, and no split's slabs are
 // written and read. 2048 rows of work are 0.3 GB at the VoxCPM2 geometry. Cancellation
-// is seen between chunks.
+// is seen between chunks. Engines whose device has no room for that take 512.
 constexpr uint32_t kPrefillChunk = 2048;
+constexpr uint32_t kPrefillChunkSmall = 512;
 constexpr uint32_t kPrefillMaxSplit = 8;    // split-K factor bound
 constexpr uint32_t kSkTileFloats = 128u * 128u;   // accumulators of one 128 x 128 prefill GEMM tile
 struct PrefillStack {
