@@ -147,7 +147,7 @@ int grow(vx_ctx *ctx, vx_buf **b, uint64_t *cap, uint64_t floats) {
 inline bool wide_run(uint32_t channels, uint32_t len) { return channels > 256u && (channels != 512u || len < 2048u); }
 
 // Whether a 1x1 or transposed convolution over `channels` (K of a product's columns)
-// takes its input as f16 hi and lo planes: 22 bits of a value, and 65504 is the largest.
+// takes its input as f16 hi and lo planes: 22 bits of |x| < 65504 (2^-25 below 2^-3).
 // The f32 kernel keeps every bit and the whole range; it takes the sums that are short
 // or odd (K no multiple of 128) up to its longest one.
 inline bool plane_products(uint32_t channels, uint32_t K) {

@@ -13,13 +13,14 @@
 // The planes are kept [row][KB] with the 16-byte chunks of a row permuted by the row
 // index, so that the A reads of 8 consecutive rows cover all banks.
 //
-// A pair of planes holds 22 bits of |h| < 65504, and from 2^-14 down fewer. Units of 32
-// and 64 channels, where f32 products are a choice, scale each row by a power of two
-// into the planes and back after the products, so that neither the range nor small rows
-// lose: 3 us a unit at 252 frames (64 channels 41.0 -> 44.2, 32 channels 32.8 -> 35.5).
-// Error of a decode against 64 bits, f32 products -> this: 1.7e-6 -> 1.5e-6, with h
-// around 1e5 in these units 4.1e-6 -> 3.5e-6, around 1e-5 2.8e-6 -> 2.5e-6 (unscaled:
-// not finite, 9e-3). Wider units keep the plain range of the GEMMs around them.
+// A pair of planes holds 22 bits of |h| < 65504 down to 2^-3, and 2^-25 absolutely below.
+// Units of 32 and 64 channels, where f32 products are a choice, scale each row by a power
+// of two into the planes and back after the products, so that neither the range nor
+// small rows lose (22 bits of what is within 2^-18 of its row's largest). Cost: 3 us a
+// unit at 252 frames (64 channels 41.0 -> 44.2, 32 channels 32.8 -> 35.5). Error of a
+// decode against 64 bits, f32 products -> this: 1.7e-6 -> 1.5e-6, with h around 1e5 in
+// these units 4.1e-6 -> 3.5e-6, around 1e-5 2.8e-6 -> 2.5e-6 (unscaled: not finite,
+// 9e-3). Wider units keep the plain range of the GEMMs around them.
 //
 // Bound: x in and y out (8 bytes an element, 24 us a unit at 252 frames) against the
 // two snakes' vector work (about 60 instructions an element with the history rows, as
